@@ -33,6 +33,12 @@ struct LoopState {
     // fused steps (k <= 64): bit j set when a block of iteration i's fused
     // kernel labelled a row j: present[i & 1]
     unsigned long long present[2];
+    // the screened E-step: rows the last one left to the six products (added
+    // by k_assign3_list, taken and cleared by k_finalize_loop), the count
+    // above which the screen does not pay, and 1 once a step went past it
+    int unsure;
+    int unsure_limit;
+    int screen_off;
 };
 
 enum StepFlags : int {
@@ -82,6 +88,33 @@ int assign3_ready(int d, int k);
 // Bytes of k_assign3's centre image (written by launch_assign3 before the E-step).
 size_t assign3_image_bytes(int k, int ld);
 hipError_t launch_assign3(const AssignArgs& a, int num_cu, hipStream_t s);
+// The centre images of launch_screen (simg, [screen_image_bytes(k, ld)]) and
+// launch_assign3_list (a.img), before both.
+hipError_t launch_centre_images(const AssignArgs& a, char* simg, hipStream_t s);
+// k_assign3 for the rows that k_screen left (screen_kernels.hip): bit r of
+// masks[i] set, row 64 i + r.  With a.state's screen_off set every row is
+// taken.  The rows taken are added to state->unsure.
+hipError_t launch_assign3_list(const AssignArgs& a, const unsigned long long* masks, int num_cu, hipStream_t s);
+
+// The certified screen in front of the E-step (screen_kernels.hip): labels
+// the rows whose nearest centre one bf16 product settles and leaves the
+// others' bits in masks, for launch_assign3_list.
+constexpr int kScreenSC = 128;  // centres per LDS stage
+struct ScreenArgs {
+    const float* X; long n; int ld;
+    int k;
+    int* labels;
+    LoopState* state;             // nullable: no early exit
+    int* changed;                 // nullable, as AssignArgs
+    const char* img;              // launch_centre_images's simg
+    float* emin;                  // nullable: the labelled rows' minima, within 2^-8 (||x||^2 + max ||c||^2)
+    unsigned long long* masks;    // [ceil(n / 64)]
+};
+size_t screen_image_bytes(int k, int ld);
+inline bool screen_ready(int ld) { return ld <= 128; }
+inline bool screen_pays(long n, int ld, int k) { return k > 128 && (double)n * ld * k >= 1.2e10; }
+hipError_t launch_screen(const ScreenArgs& a, int num_cu, hipStream_t s);
+
 // The three-part bf16 split is exact for finite values of magnitude >= 2^-103,
 // and the E-step's smallest kept part products stay normal fp32 numbers when
 // the data's largest magnitude is 0 or at least 2^-50.
@@ -260,6 +293,9 @@ struct InRelocArgs {
     // 128 floats)
     const float* xnorm = nullptr;
     const float* emin = nullptr;
+    // xnorm + emin lies within margin (max ||x||^2 + max ||c||^2) of the
+    // distance (2^-10 for the six products, 2^-7 for the screen's minima)
+    float margin = 0x1p-10f;
 };
 constexpr int kRelocInlineBlocks = 256;  // grid of k_reloc / k_finalize_reloc (one block per CU: their LDS)
 constexpr int kRelocLdsRows = 4096;      // a block's row distances kept in LDS (more rows: InRelocArgs::dist)

@@ -1136,6 +1136,10 @@ __global__ __launch_bounds__(256) void k_finalize_loop(FinalizeArgs a, int nch)
             done = 2;
         if (done != 0) st->halt_iter = a.iter;
         st->done = done;
+        // a step that left more rows than the screen is worth is the last
+        // screened one of the run
+        if (st->unsure > st->unsure_limit) st->screen_off = 1;
+        st->unsure = 0;
     }
 }
 
@@ -1863,7 +1867,10 @@ __device__ __forceinline__ void reloc_body(const InRelocArgs& a, int E)
     // (A') With the E-step's row minima: the approximate distance xnorm[r]
     // + emin[r] (= ||x||^2 + ||c||^2 - 2 x.c, c the row's centre) of every
     // row, the block's E-th largest of them, T, and as candidates the rows
-    // within 2M of T, M = 2^-10 (max ||x||^2 + max ||c||^2): for rows of
+    // within 2M of T, M = margin (max ||x||^2 + max ||c||^2).  The rows
+    // wanted are all among them when the approximation and the direct form
+    // together err by at most M.  Screened steps: 1.1 2^-8 and 2^-13 of that
+    // sum, margin 2^-7.  Six-product steps (margin 2^-10): for rows of
     // at most 128 floats the approximation and the direct form each lie
     // within 2^-13 of that sum of the true distance (fp32 norms, the split's
     // dropped terms, the fp32 accumulation of at most 768 part products, and
@@ -1927,7 +1934,7 @@ __device__ __forceinline__ void reloc_body(const InRelocArgs& a, int E)
                 cm = fmaxf(cm, s2);
             }
             __syncthreads();  // sdist from every thread
-            const float M = 0x1p-10f * (block_max(xm, sd) + block_max(cm, sd));
+            const float M = a.margin * (block_max(xm, sd) + block_max(cm, sd));
             float dl = INFINITY;
             long il = -1;
             for (int e = 0; e < E; ++e) {

@@ -1,0 +1,362 @@
+// screen_kernels.hip -- a certified screen in front of the split E-step
+// (gfx950).
+//
+// k_assign3 takes six bf16 part products for every x.c and is bound by them.
+// For most rows one of the six settles the label: the product of the high
+// parts, hh, differs from the six-product value by less than
+//   e = 1.05 (2^-8 + ..) ||x|| max ||c||   (screen_slack below),
+// so when a row's largest hh.. value leads its second largest by more than
+// 2 e, the six products have their first minimum at the same centre, and no
+// other centre can tie with it.  k_screen labels those rows and leaves the
+// others' bits in `masks`; k_assign3_list (split_kernels.hip) then runs the
+// six products for these rows alone.  Labels are those of k_assign3, bit for
+// bit, whatever the data.
+#include "split_common.h"
+
+namespace skm {
+
+// A bound on how far a screen value lies from x.c - ||c||^2 / 2 as the six
+// products give it, for a row with ||x||^2 = xx (fp32 sum) and C2 = the
+// largest ||c||^2, ldp features with the padding:
+//   rounding x and c to bf16 and the index in the low six bits: 2^-8 +
+//   2^-18 + 2^-17 of ||x|| ||c||; the screen's fp32 accumulation, ldp + 1
+//   terms, and the six products', 6 ldp terms, at most 2^-23 of the terms'
+//   magnitudes each (the terms of one row and centre total at most ||x||
+//   ||c|| by Cauchy-Schwarz); the products left out, 2^-22; the same for
+//   ||c||^2 / 2; and what a flush of subnormal parts and products can take.
+// The factors 1.05 and 1.01 cover the norms' own rounding.
+__device__ __forceinline__ float screen_slack(float xx, float C2, int ldp)
+{
+    const float xn = sqrtf(xx), cn = sqrtf(C2);
+    const float a = 0x1p-8f + 0x1p-16f + 8.f * (float)ldp * 0x1p-23f;
+    const float b = 0x1p-16f + (float)(ldp + 2) * 0x1p-23f;
+    return 1.05f * (a * xn * cn + b * 0.5f * C2) + 0x1p-100f * (xn + cn) + 0x1p-100f;
+}
+
+// The largest of three: fmaxf would quiet each operand with an instruction of
+// its own first.  (Its operands are VALU results, never an MFMA's.)
+__device__ __forceinline__ float max3(float a, float b, float c)
+{
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// D += A B on bf16, 32x32x16: lane l holds A[m = l%32][kk = 8(l/32) + j] and
+// B[kk = 8(l/32) + j][n = l%32], j < 8, and receives D[m = 8(i/4) + 4(l/32) +
+// i%4][n = l%32], i < 16.
+typedef float v16f __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ v16f mfma32_bf16(v8bf a, v8bf b, v16f c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// A block of 8 waves owns 512 rows, 64 per wave in two 32-row groups whose
+// high parts stay in registers (rows of at most 128 floats) while the
+// centres pass by in LDS stages of kScreenSC (the next stage copied in with
+// direct-to-LDS loads while the current one is used).  Per 32 centres a wave
+// reads 2 NK 1 KB operands for 4 NK MFMAs; the accumulators start from
+// -||c||^2 / 2, so that they end as the value to maximise.  Lane l keeps the
+// two largest over its centres of row l%32 of each group, the centre's place
+// in the stage in the low six bits of the value: nine VALU instructions for
+// four values.  MFMAs and VALU instructions hardly overlap here, whether of
+// one wave or of several: 8 16x16x32 MFMAs and 36 v_max3 take 57 and 65 ns a
+// wave and SIMD alone, 106 together; the same work in 32x32x16 MFMAs 81.
+// So the rows' K steps take features 32 s + 16 (l/32) + 8 t + j: each lane's
+// 64 bytes of a row in a row.
+template <int NK>
+__global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
+{
+    using G = ScreenGeom<NK>;
+    constexpr bool PIPE = true;
+    const LoopState* st = a.state;
+    if (st != nullptr && (st->done != 0 || st->screen_off != 0)) return;
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    __shared__ int sChg;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, r32 = lane & 31;
+    const int ld = a.ld;
+    const long n = a.n;
+    if (tid == 0) sChg = 0;
+    int nchg = 0;
+    const int nst = (a.k + kScreenSC - 1) / kScreenSC;
+    const int stage_bytes = G::STAGE;
+    const __amdgpu_buffer_rsrc_t irs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.img), (short)0, nst * stage_bytes, 0x00020000);
+    auto copy_stage = [&](int stg, int b) {
+        char* dst = smem + b * stage_bytes;
+        for (int i = wave; i < stage_bytes / 1024; i += 8) {
+            const int soff = stg * stage_bytes + i * 1024;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16,
+                                                     lane * 16, soff, 0, 0);
+        }
+    };
+    if (resident)
+        for (int stg = 0; stg < nst; ++stg) copy_stage(stg, stg);
+    else
+        copy_stage(0, 0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    int cur = 0;
+    // (resident: a wave stops at its own last rows; else all waves take part
+    // in the stages of the block's)
+    const long wstep = (long)gridDim.x * 512;
+    auto rows_at = [&](long base) { return resident ? base : base + (long)gridDim.x * 64 * wave; };
+    auto rows_rsrc = [&](long wrow) {
+        const long nrow = n - wrow < 64 ? (n - wrow > 0 ? n - wrow : 0) : 64;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.X + (nrow > 0 ? wrow * ld : 0)), (short)0,
+                                                 (int)(nrow * ld * 4), 0x00020000);
+    };
+    // group g's rows (a lane past the rows' end loads 0, one past a row's end
+    // the next row's values: these meet zero centre parts and are kept out of
+    // the norm).  PG of the next 64 rows' groups are in flight while the
+    // current ones meet the centres: registers for no more.
+    constexpr int PG = NK <= 2 ? 2 : 1;
+    f4v raw[PG][NK][4];
+    auto load = [&](f4v(&q)[NK][4], __amdgpu_buffer_rsrc_t rs, int g) {
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(
+                    rs, ((32 * g + r32) * ld + 32 * s + 16 * h + 4 * t) * 4, 0, 0);
+                q[s][t] = __builtin_bit_cast(f4v, v);
+            }
+        }
+    };
+    const long first = (long)blockIdx.x * 64 + (resident ? (long)gridDim.x * 64 * wave : 0);
+    {
+        const __amdgpu_buffer_rsrc_t rs = rows_rsrc(rows_at(first));
+#pragma unroll
+        for (int g = 0; g < PG; ++g) load(raw[g], rs, g);
+    }
+    for (long base = first; base < n; base += wstep) {
+        const long wrow = rows_at(base);
+        const long nrow = n - wrow < 64 ? (n - wrow > 0 ? n - wrow : 0) : 64;
+        // the rows' high parts and ||x||^2
+        v8bf xh[2][2 * NK];
+        float xx[2];
+        auto parts = [&](const f4v(&q)[NK][4], int g) {
+            xx[g] = 0.f;
+#pragma unroll
+            for (int s = 0; s < NK; ++s) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const float in = 32 * s + 16 * h + 4 * t < ld ? 1.f : 0.f;
+                    const f4v v = q[s][t];
+                    xx[g] = fmaf(fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w))), in, xx[g]);
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const f4v u = q[s][2 * t], v = q[s][2 * t + 1];
+                    xh[g][2 * s + t] = __builtin_bit_cast(v8bf, v4u{pack_bf16(u.x, u.y), pack_bf16(u.z, u.w),
+                                                                    pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)});
+                }
+            }
+            // the norm is taken here (sunk to its use it keeps the fp32 row
+            // alive)
+            asm volatile("" : "+v"(xx[g]));
+        };
+        parts(raw[0], 0);
+        if constexpr (PG == 2) {
+            parts(raw[1], 1);
+        } else {
+            load(raw[0], rows_rsrc(wrow), 1);
+            parts(raw[0], 1);
+        }
+        if (base + wstep < n) {
+            const __amdgpu_buffer_rsrc_t rs = rows_rsrc(rows_at(base + wstep));
+#pragma unroll
+            for (int g = 0; g < PG; ++g) load(raw[g], rs, g);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float m1[2], m2[2];
+        int ms[2];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            m1[g] = m2[g] = -INFINITY;
+            ms[g] = 0;
+        }
+        unsigned cmax = 0u;
+        // the 32 rows of group g against one block's centres: the two largest
+        auto take = [&](int g, const v16f& acc, int cb) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float u[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    u[i] = __uint_as_float((__float_as_uint(acc[4 * q + i]) & ~63u) | (unsigned)(16 * cb + 4 * q + i));
+                // with m1 >= m2 the second largest of m1, m2 and two more is
+                // the larger of m2 and the middle one of the rest
+                const float a1 = __builtin_amdgcn_fmed3f(m1[g], u[0], u[1]);
+                m1[g] = max3(m1[g], u[0], u[1]);
+                const float a2 = __builtin_amdgcn_fmed3f(m1[g], u[2], u[3]);
+                m1[g] = max3(m1[g], u[2], u[3]);
+                m2[g] = max3(m2[g], a1, a2);
+            }
+            // the values are used up here: sunk to the end of the stage they
+            // spill
+            asm volatile("" : "+v"(m1[g]), "+v"(m2[g]));
+        };
+        v16f late;  // group 1 of the block before
+        if constexpr (PIPE) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) late[i] = -3e38f;
+        }
+        float was[2] = {m1[0], m1[1]};
+        for (int stg = 0; stg < nst; ++stg) {
+            if (!resident) copy_stage(stg + 1 < nst ? stg + 1 : 0, cur ^ 1);
+            const char* const sb = smem + (resident ? stg : cur) * stage_bytes;
+            const __bf16* const cb0 = reinterpret_cast<const __bf16*>(sb) + r32 * G::CSTR + 16 * h;
+            const float* const sn = reinterpret_cast<const float*>(sb + G::PBYTES);
+            cmax = max(cmax, reinterpret_cast<const unsigned*>(sn)[kScreenSC]);
+            constexpr int NB = kScreenSC / 32;
+#pragma unroll
+            for (int cb = 0; cb < NB; ++cb) {
+                v16f init;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const v4f c4 = *reinterpret_cast<const v4f*>(sn + 32 * cb + 8 * q + 4 * h);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) init[4 * q + i] = c4[i];
+                }
+                auto centres = [&](int s) {
+                    return *reinterpret_cast<const v8bf*>(cb0 + 32 * cb * G::CSTR + 32 * (s >> 1) + 8 * (s & 1));
+                };
+                if constexpr (PIPE) {
+                    v8bf ca[2 * NK];
+#pragma unroll
+                    for (int s = 0; s < 2 * NK; ++s) ca[s] = centres(s);
+                    v16f acc = init;
+#pragma unroll
+                    for (int s = 0; s < 2 * NK; ++s) acc = mfma32_bf16(ca[s], xh[0][s], acc);
+                    take(1, late, cb == 0 ? NB - 1 : cb - 1);
+                    if (cb == 0) {  // the stage before is through
+#pragma unroll
+                        for (int g = 0; g < 2; ++g) {
+                            ms[g] = m1[g] != was[g] ? stg - 1 : ms[g];
+                            was[g] = m1[g];
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    late = init;
+#pragma unroll
+                    for (int s = 0; s < 2 * NK; ++s) late = mfma32_bf16(ca[s], xh[1][s], late);
+                    take(0, acc, cb);
+                    __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    v16f acc[2] = {init, init};
+#pragma unroll
+                    for (int s = 0; s < 2 * NK; ++s) {
+                        const v8bf ca = centres(s);
+#pragma unroll
+                        for (int g = 0; g < 2; ++g) acc[g] = mfma32_bf16(ca, xh[g][s], acc[g]);
+                    }
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) take(g, acc[g], cb);
+                }
+            }
+            if constexpr (!PIPE) {
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    ms[g] = m1[g] != was[g] ? stg : ms[g];
+                    was[g] = m1[g];
+                }
+            }
+            if (!resident) {
+                // the next stage is in (every wave's copies) and this one is
+                // read: swap
+                __builtin_amdgcn_s_waitcnt(0);
+                __syncthreads();
+                cur ^= 1;
+            }
+        }
+        if constexpr (PIPE) {
+            take(1, late, kScreenSC / 32 - 1);
+#pragma unroll
+            for (int g = 0; g < 2; ++g) ms[g] = m1[g] != was[g] ? nst - 1 : ms[g];
+        }
+        // the two lanes of a row; lane l keeps row l of the wave's 64
+        float b1 = 0.f, b2 = 0.f, bx = 0.f;
+        int bi = 0;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            // place p of the stage: reg i = p % 16 of block p / 16
+            const int p = (int)(__float_as_uint(m1[g]) & 63u);
+            int i1 = ms[g] * kScreenSC + 32 * (p >> 4) + 8 * ((p & 15) >> 2) + 4 * h + (p & 3);
+            const float o1 = __shfl_xor(m1[g], 32), o2 = __shfl_xor(m2[g], 32);
+            const int oi = __shfl_xor(i1, 32);
+            const float x2 = xx[g] + __shfl_xor(xx[g], 32);
+            const float d2 = fmaxf(fminf(m1[g], o1), fmaxf(m2[g], o2));
+            i1 = o1 > m1[g] ? oi : i1;
+            if (h == g) {
+                b1 = fmaxf(m1[g], o1);
+                b2 = d2;
+                bi = i1;
+                bx = x2;
+            }
+        }
+        const float C2 = __uint_as_float(cmax);
+        const float slack = screen_slack(bx, C2, 32 * NK);
+        // (the magnitudes' bound keeps every sum finite; a NaN in the norms
+        // fails it)
+        const bool sure = (b1 - b2 > 2.f * slack) & (sqrtf(bx) * sqrtf(C2) + C2 < 1e37f);
+        const bool valid = lane < nrow;
+        const long row = wrow + lane;
+        int moved = 0;
+        if (valid && sure) {
+            if (a.changed != nullptr) moved = a.labels[row] != bi;
+            a.labels[row] = bi;
+            if (a.emin != nullptr) a.emin[row] = -2.f * b1;
+        }
+        if (a.changed != nullptr) nchg += (int)__popcll(__ballot(moved));
+        const unsigned long long left = __ballot(valid && !sure);
+        if (lane == 0 && nrow > 0) a.masks[wrow >> 6] = left;
+    }
+    if (a.changed != nullptr) {
+        if (lane == 0 && nchg != 0) atomicAdd(&sChg, nchg);
+        __syncthreads();
+        if (tid == 0 && sChg != 0) atomicAdd(a.changed, sChg);
+    }
+}
+
+template <int NK>
+static hipError_t launch_screen_nk(const ScreenArgs& a, int num_cu, hipStream_t s)
+{
+    using G = ScreenGeom<NK>;
+    static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_screen<NK>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, G::RES * G::STAGE);
+    if (e != hipSuccess) return e;
+    const int nst = (a.k + kScreenSC - 1) / kScreenSC;
+    const int resident = nst <= G::RES;
+    const long blocks = (a.n + 511) / 512;
+    hipLaunchKernelGGL(k_screen<NK>, dim3((unsigned)(blocks < num_cu ? blocks : num_cu)), dim3(512),
+                       (size_t)(resident ? nst : 2) * G::STAGE, s, a, resident);
+    return hipGetLastError();
+}
+
+size_t screen_image_bytes(int k, int ld)
+{
+    const size_t nst = size_t(k + kScreenSC - 1) / kScreenSC;
+    switch ((ld + 31) / 32) {
+    case 1: return nst * ScreenGeom<1>::STAGE;
+    case 2: return nst * ScreenGeom<2>::STAGE;
+    case 3: return nst * ScreenGeom<3>::STAGE;
+    default: return nst * ScreenGeom<4>::STAGE;
+    }
+}
+
+hipError_t launch_screen(const ScreenArgs& a, int num_cu, hipStream_t s)
+{
+    if (a.n <= 0) return hipSuccess;
+    switch ((a.ld + 31) / 32) {
+    case 1: return launch_screen_nk<1>(a, num_cu, s);
+    case 2: return launch_screen_nk<2>(a, num_cu, s);
+    case 3: return launch_screen_nk<3>(a, num_cu, s);
+    case 4: return launch_screen_nk<4>(a, num_cu, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace skm

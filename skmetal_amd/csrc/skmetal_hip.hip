@@ -683,6 +683,17 @@ struct Lloyd {
     }
 
     char* a3img = nullptr;  // k_assign3's centre image
+    char* simg = nullptr;   // k_screen's
+    unsigned long long* smask = nullptr;  // [ceil(n / 64)] the rows it leaves
+    // the E-step behind k_screen.  SKMETAL_HIP_SCREEN=0 keeps every row on
+    // the six products, 1 screens every shape that the screen takes (tests)
+    bool screened() const
+    {
+        if (!split_on || !a3cap || !screen_ready(ld)) return false;
+        const char* e = getenv("SKMETAL_HIP_SCREEN");
+        if (e != nullptr && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
+        return screen_pays(n, ld, k);
+    }
 
     int assign(const float* cents, LoopState* state, int* changed, bool minima = false)
     {
@@ -691,6 +702,17 @@ struct Lloyd {
             if (a3img == nullptr) TRY(grab((void**)&a3img, assign3_image_bytes(k, ld)));
             a.img = a3img;
             if (minima) a.emin = emin;
+            if (screened()) {
+                if (simg == nullptr) {
+                    TRY(grab((void**)&simg, screen_image_bytes(k, ld)));
+                    TRY(grab((void**)&smask, size_t((n + 63) / 64) * sizeof(unsigned long long)));
+                }
+                const ScreenArgs sa{X, n, ld, k, labels, state, changed, simg, a.emin, smask};
+                HIP_TRY(launch_centre_images(a, simg, s), "centre image launch");
+                HIP_TRY(launch_screen(sa, C->num_cu, s), "screen launch");
+                HIP_TRY(launch_assign3_list(a, smask, C->num_cu, s), "assign launch");
+                return 0;
+            }
             HIP_TRY(launch_assign3(a, C->num_cu, s), "assign launch");
         } else
             HIP_TRY(launch_assign(a, C->num_cu, s), "assign launch");
@@ -704,7 +726,7 @@ struct Lloyd {
     int assign_inertia(const float* cents, double* out)
     {
         const long blocks = std::min<long>(C->num_cu, (n + 255) / 256);
-        if (split_on && a3cap && blocks <= rowdist_grid(n)) {
+        if (split_on && a3cap && blocks <= rowdist_grid(n) && !screened()) {
             if (a3img == nullptr) TRY(grab((void**)&a3img, assign3_image_bytes(k, ld)));
             AssignArgs a{X, n, ld, cents, cnorm, k, labels, nullptr, nullptr, a3img};
             int nb = 0;
@@ -784,6 +806,7 @@ struct Lloyd {
             // this step's E-step was k_fused3 or k_assign3, which wrote its row minima
             r.xnorm = xnorm;
             r.emin = emin;
+            if (fblocks == 0 && screened()) r.margin = 0x1p-7f;
         }
         if (reloc_inline && fblocks > 0 && k <= 64 && 8 * ((k * r.nch + 7) / 8) <= kRelocInlineBlocks) {
             // the fused kernel's presence bits name the empty clusters: one launch
@@ -947,6 +970,7 @@ struct Lloyd {
         }
         LoopState hs{};
         hs.reloc_iter = -1;
+        hs.unsure_limit = (int)std::min<long>(n / 2, 1L << 30);
         // the reset is a kernel on the stream: nothing waits for the host
         HIP_TRY(launch_state_reset(st, hs, s), "state reset launch");
         HIP_TRY(hipMemsetAsync(labels, 0xff, size_t(n) * sizeof(int), s), "hipMemsetAsync(labels)");

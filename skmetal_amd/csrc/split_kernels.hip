@@ -15,100 +15,9 @@
 
 #include <type_traits>
 
-#include "fused_common.h"
+#include "split_common.h"
 
 namespace skm {
-
-// ---------------------------------------------------------------------------
-// Three-part bf16 split.  bf16 keeps fp32's exponent range with 8 significant
-// bits, so every finite fp32 v with |v| >= 2^-103 is the exact sum of three
-// bf16 values, each rounded to nearest:
-//   hi = bf16(v),  mid = bf16(v - hi),  lo = (v - hi) - mid.
-// v - hi is a multiple of v's fp32 ulp no larger than 2^16 of them, so the fp32
-// subtraction is exact; likewise (v - hi) - mid, which is at most 2^8 ulps and
-// therefore exactly a bf16.  |mid| <= 2^-8 |v|, |lo| <= 2^-16 |v|.
-// A product of two bf16 values is exact in fp32, and the MFMAs accumulate in
-// fp32, so
-//  - the per-cluster sums (one-hot x hi, x mid, x lo) add every x exactly as
-//    given, in fp32 (the one-hot operand is exact);
-//  - the E-step takes 6 of the 9 part products of x.c (hh, hm, mh, hl, lh, mm):
-//    the three left out (ml, lm, ll) total at most (2^-23 + 2^-32) |x_i c_i|
-//    per feature, two units of fp32 roundoff, against the one unit by which an
-//    fp32 product of x_i and c_i is itself rounded.
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-
-// (a, b) rounded to nearest even bf16, a in the low half: v_cvt_pk_bf16_f32
-__device__ __forceinline__ unsigned pack_bf16(float a, float b)
-{
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a, b}, v2bf));
-}
-
-__device__ __forceinline__ float bf16_lo(unsigned p) { return __uint_as_float(p << 16); }
-__device__ __forceinline__ float bf16_hi(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
-
-// The parts of a and b, as bf16 pairs (a's part in the low half).
-__device__ __forceinline__ void split3(float a, float b, unsigned& hi, unsigned& mid, unsigned& lo)
-{
-    hi = pack_bf16(a, b);
-    const float ra = a - bf16_lo(hi), rb = b - bf16_hi(hi);  // exact
-    mid = pack_bf16(ra, rb);
-    lo = pack_bf16(ra - bf16_lo(mid), rb - bf16_hi(mid));   // exact, and exactly bf16
-}
-
-struct Parts8 {
-    v8bf h, m, l;
-};
-struct Parts4 {
-    v4s h, m, l;  // 16x16x16 bf16 operands are passed as shorts
-};
-
-__device__ __forceinline__ Parts8 split8(float4 u, float4 v)
-{
-    unsigned h0, h1, h2, h3, m0, m1, m2, m3, l0, l1, l2, l3;
-    split3(u.x, u.y, h0, m0, l0);
-    split3(u.z, u.w, h1, m1, l1);
-    split3(v.x, v.y, h2, m2, l2);
-    split3(v.z, v.w, h3, m3, l3);
-    return Parts8{__builtin_bit_cast(v8bf, v4u{h0, h1, h2, h3}), __builtin_bit_cast(v8bf, v4u{m0, m1, m2, m3}),
-                  __builtin_bit_cast(v8bf, v4u{l0, l1, l2, l3})};
-}
-
-__device__ __forceinline__ Parts4 split4(float4 u)
-{
-    unsigned h0, h1, m0, m1, l0, l1;
-    split3(u.x, u.y, h0, m0, l0);
-    split3(u.z, u.w, h1, m1, l1);
-    return Parts4{__builtin_bit_cast(v4s, v2u{h0, h1}), __builtin_bit_cast(v4s, v2u{m0, m1}),
-                  __builtin_bit_cast(v4s, v2u{l0, l1})};
-}
-
-// D += A B on bf16: 16x16x32 (8 values per lane) and 16x16x16 (4)
-__device__ __forceinline__ v4f mfma_bf16(v8bf a, v8bf b, v4f c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ v4f mfma_bf16(v4s a, v4s b, v4f c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-}
-
-// acc += the six kept part products of a.b (smaller terms first)
-template <typename P>
-__device__ __forceinline__ v4f dot6(const P& a, const P& b, v4f acc)
-{
-    acc = mfma_bf16(a.m, b.m, acc);
-    acc = mfma_bf16(a.l, b.h, acc);
-    acc = mfma_bf16(a.h, b.l, acc);
-    acc = mfma_bf16(a.m, b.h, acc);
-    acc = mfma_bf16(a.h, b.m, acc);
-    return mfma_bf16(a.h, b.h, acc);
-}
 
 // ---------------------------------------------------------------------------
 // k_fused3: the fused step with the E-step and the per-cluster sums on bf16
@@ -852,8 +761,8 @@ struct Assign3Geom {
 };
 
 template <int CB>
-__global__ __launch_bounds__(256) void k_centre_image(const float* __restrict__ C, const float* __restrict__ cnorm,
-                                                      int k, int ld, int nseg, char* __restrict__ img)
+__device__ __forceinline__ void centre_image(const float* __restrict__ C, const float* __restrict__ cnorm, int k,
+                                             int ld, int nseg, char* __restrict__ img)
 {
     using G = Assign3Geom<CB>;
     const int stg = blockIdx.x, p = stg / nseg, sg = stg - p * nseg;
@@ -883,6 +792,158 @@ __global__ __launch_bounds__(256) void k_centre_image(const float* __restrict__ 
 }
 
 template <int CB>
+__global__ __launch_bounds__(256) void k_centre_image(const float* __restrict__ C, const float* __restrict__ cnorm,
+                                                      int k, int ld, int nseg, char* __restrict__ img)
+{
+    centre_image<CB>(C, cnorm, k, ld, nseg, img);
+}
+
+// The images of k_assign3_list (its nst stages) and of k_screen (the blocks
+// past them) in one launch.
+template <int CB, int NK>
+__global__ __launch_bounds__(256) void k_centre_images(const float* __restrict__ C, const float* __restrict__ cnorm,
+                                                       int k, int ld, int nseg, int nst, char* __restrict__ img,
+                                                       char* __restrict__ simg, const LoopState* st)
+{
+    if (st != nullptr && st->done != 0) return;
+    if ((int)blockIdx.x < nst)
+        centre_image<CB>(C, cnorm, k, ld, nseg, img);
+    else
+        screen_image<NK>(C, cnorm, k, ld, simg, (int)blockIdx.x - nst);
+}
+
+// One 32-row block of a wave against every centre: lane l < 32 ends with row
+// l's label and minimum ||c||^2 - 2 x.c.  xr holds the rows' first K step
+// (rows 16g + l%16, features 8h..) and `cur` the LDS stage with stage 0 of
+// the image; xload(f) loads the rows' K step at feature f into xr, next()
+// the next block's first.
+template <int CB, typename Copy, typename XLoad, typename Next>
+__device__ __forceinline__ void assign3_rows(char* smem, int ld, int npass, int nseg, int h, int r16, int& cur,
+                                             float4 (&xr)[2][2], Copy copy_stage, XLoad xload, Next next, int& mylab,
+                                             float& mymin)
+{
+    using G = Assign3Geom<CB>;
+    constexpr int CPC = G::CPC, SEG = G::SEG, NKS = G::NKS, CSTR = G::CSTR, CPART = G::CPART;
+    const int nst = npass * nseg;
+    float bd[2] = {INFINITY, INFINITY};
+    int bi[2] = {0, 0};
+    for (int p = 0; p < npass; ++p) {
+        v4f acc[2][CB];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) acc[g][cb] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
+        for (int sg = 0; sg < nseg; ++sg) {
+            const int stg = p * nseg + sg;
+            const int f0 = sg * SEG;
+            const __bf16* const cbase = reinterpret_cast<const __bf16*>(smem + cur * G::STAGE) + r16 * CSTR + 8 * h;
+            const int nks = min(NKS, (ld - f0 + 31) / 32);
+            for (int ks = 0; ks < nks; ++ks) {
+                Parts8 xp[2];
+#pragma unroll
+                for (int g = 0; g < 2; ++g) xp[g] = split8(xr[g][0], xr[g][1]);
+                // the next K step's rows: this stage's next, the next
+                // segment's or pass's first (same rows), or the next row
+                // block's first
+                if (ks + 1 < nks) {
+                    xload(f0 + 32 * (ks + 1));
+                } else if (sg + 1 < nseg) {
+                    xload(f0 + SEG);
+                } else if (p + 1 < npass) {
+                    xload(0);
+                } else {
+                    next();
+                }
+                // the next stage's copy goes out behind the X loads that
+                // this stage still waits on (loads complete in order)
+                if (ks == nks - 1 && nst > 1) copy_stage(stg + 1 < nst ? stg + 1 : 0, cur ^ 1);
+                // four centre blocks at a time, product-major over their
+                // eight accumulators: consecutive MFMAs write different
+                // accumulators (a block's six products back to back wait
+                // on each other).  Each accumulator takes dot6's products
+                // in dot6's order.
+                constexpr int CG = 4;
+#pragma unroll
+                for (int cb0 = 0; cb0 < CB; cb0 += CG) {
+                    Parts8 cpt[CG];
+#pragma unroll
+                    for (int c = 0; c < CG; ++c) {
+                        const __bf16* cp = cbase + 16 * (cb0 + c) * CSTR + 32 * ks;
+                        cpt[c] = Parts8{*reinterpret_cast<const v8bf*>(cp),
+                                        *reinterpret_cast<const v8bf*>(cp + CPART),
+                                        *reinterpret_cast<const v8bf*>(cp + 2 * CPART)};
+                    }
+#pragma unroll
+                    for (int pr = 0; pr < 6; ++pr) {
+#pragma unroll
+                        for (int c = 0; c < CG; ++c) {
+                            const Parts8& cc = cpt[c];
+                            const v8bf ca = pr == 0 ? cc.m : pr == 1 ? cc.l : pr == 2 ? cc.h : pr == 3 ? cc.m : cc.h;
+#pragma unroll
+                            for (int g = 0; g < 2; ++g) {
+                                const Parts8& x = xp[g];
+                                const v8bf xb = pr == 0 ? x.m : pr == 1 ? x.h : pr == 2 ? x.l : pr == 3 ? x.h
+                                                                                           : pr == 4 ? x.m : x.h;
+                                acc[g][cb0 + c] = mfma_bf16(ca, xb, acc[g][cb0 + c]);
+                            }
+                        }
+                    }
+                }
+            }
+            if (nst > 1) {
+                // the next stage is in (every wave's copies) and this one
+                // is read: swap
+                __builtin_amdgcn_s_waitcnt(0);
+                __syncthreads();
+                cur ^= 1;
+            }
+        }
+        // ||c||^2 - 2 x.c, first minimum wins (_k_means_lloyd.pyx:196-212);
+        // the lane's centres come in ascending order, passes too.  With
+        // one stage, the pass's ||c||^2 are in it; else they are read as
+        // the previous pass's norms of the stage now current, which the
+        // stage copies rewrite only after the next barrier (a wave past
+        // that barrier has every wave's reads of this behind it).
+        const float* sN = reinterpret_cast<const float*>(smem + cur * G::STAGE + G::PBYTES) + (nst > 1 ? CPC : 0);
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            const float4 c4 = *reinterpret_cast<const float4*>(&sN[16 * cb + 4 * h]);
+            const float cn[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float dd = fmaf(-2.0f, acc[g][cb][i], cn[i]);  // NaN compares false
+                    const bool take = dd < bd[g];
+                    bd[g] = take ? dd : bd[g];
+                    bi[g] = take ? p * CPC + 16 * cb + 4 * h + i : bi[g];
+                }
+            }
+        }
+    }
+    mylab = 0;
+    mymin = 0.f;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        float d0 = bd[g];
+        int i0 = bi[g];
+#pragma unroll
+        for (int m = 16; m <= 32; m *= 2) {
+            const float od = __shfl_xor(d0, m);
+            const int oi = __shfl_xor(i0, m);
+            const bool take = (od < d0) | ((od == d0) & (oi < i0));
+            d0 = take ? od : d0;
+            i0 = take ? oi : i0;
+        }
+        if (h == g) {  // lanes 0..31: row = lane
+            mylab = i0;
+            mymin = d0;
+        }
+    }
+}
+
+template <int CB>
 __global__ __launch_bounds__(512, 1) void k_assign3(const float* __restrict__ X, long n, int ld,
                                                    const char* __restrict__ img, int k, int* __restrict__ labels,
                                                    LoopState* st, int* changed, const float* __restrict__ C, int d,
@@ -890,7 +951,7 @@ __global__ __launch_bounds__(512, 1) void k_assign3(const float* __restrict__ X,
 {
     if (st != nullptr && st->done != 0) return;
     using G = Assign3Geom<CB>;
-    constexpr int CPC = G::CPC, SEG = G::SEG, NKS = G::NKS, CSTR = G::CSTR, CPART = G::CPART;
+    constexpr int CPC = G::CPC, SEG = G::SEG;
     extern __shared__ __attribute__((aligned(1024))) char smem[];  // two stages
     __shared__ int sChg;  // labels the block changed
     const int tid = threadIdx.x;
@@ -948,122 +1009,14 @@ __global__ __launch_bounds__(512, 1) void k_assign3(const float* __restrict__ X,
         const long wrow = base + 32 * wave;  // this wave's first row
         const long nrow = n - wrow < 32 ? (n - wrow > 0 ? n - wrow : 0) : 32;
         const __amdgpu_buffer_rsrc_t rs = rows_rsrc(base);
-        float bd[2] = {INFINITY, INFINITY};
-        int bi[2] = {0, 0};
-        for (int p = 0; p < npass; ++p) {
-            v4f acc[2][CB];
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-#pragma unroll
-                for (int cb = 0; cb < CB; ++cb) acc[g][cb] = v4f{0.f, 0.f, 0.f, 0.f};
-            }
-            for (int sg = 0; sg < nseg; ++sg) {
-                const int stg = p * nseg + sg;
-                const int f0 = sg * SEG;
-                const __bf16* const cbase = reinterpret_cast<const __bf16*>(smem + cur * G::STAGE) + r16 * CSTR + 8 * h;
-                const int nks = min(NKS, (ld - f0 + 31) / 32);
-                for (int ks = 0; ks < nks; ++ks) {
-                    Parts8 xp[2];
-#pragma unroll
-                    for (int g = 0; g < 2; ++g) xp[g] = split8(xr[g][0], xr[g][1]);
-                    // the next K step's rows: this stage's next, the next
-                    // segment's or pass's first (same rows), or the next row
-                    // block's first
-                    if (ks + 1 < nks) {
-                        xload(rs, f0 + 32 * (ks + 1));
-                    } else if (sg + 1 < nseg) {
-                        xload(rs, f0 + SEG);
-                    } else if (p + 1 < npass) {
-                        xload(rs, 0);
-                    } else if (base + (long)gridDim.x * 256 < n) {
-                        xload(rows_rsrc(base + (long)gridDim.x * 256), 0);
-                    }
-                    // the next stage's copy goes out behind the X loads that
-                    // this stage still waits on (loads complete in order)
-                    if (ks == nks - 1 && nst > 1) copy_stage(stg + 1 < nst ? stg + 1 : 0, cur ^ 1);
-                    // four centre blocks at a time, product-major over their
-                    // eight accumulators: consecutive MFMAs write different
-                    // accumulators (a block's six products back to back wait
-                    // on each other).  Each accumulator takes dot6's products
-                    // in dot6's order.
-                    constexpr int CG = 4;
-#pragma unroll
-                    for (int cb0 = 0; cb0 < CB; cb0 += CG) {
-                        Parts8 cpt[CG];
-#pragma unroll
-                        for (int c = 0; c < CG; ++c) {
-                            const __bf16* cp = cbase + 16 * (cb0 + c) * CSTR + 32 * ks;
-                            cpt[c] = Parts8{*reinterpret_cast<const v8bf*>(cp),
-                                            *reinterpret_cast<const v8bf*>(cp + CPART),
-                                            *reinterpret_cast<const v8bf*>(cp + 2 * CPART)};
-                        }
-#pragma unroll
-                        for (int pr = 0; pr < 6; ++pr) {
-#pragma unroll
-                            for (int c = 0; c < CG; ++c) {
-                                const Parts8& cc = cpt[c];
-                                const v8bf ca = pr == 0 ? cc.m : pr == 1 ? cc.l : pr == 2 ? cc.h : pr == 3 ? cc.m : cc.h;
-#pragma unroll
-                                for (int g = 0; g < 2; ++g) {
-                                    const Parts8& x = xp[g];
-                                    const v8bf xb = pr == 0 ? x.m : pr == 1 ? x.h : pr == 2 ? x.l : pr == 3 ? x.h
-                                                                                               : pr == 4 ? x.m : x.h;
-                                    acc[g][cb0 + c] = mfma_bf16(ca, xb, acc[g][cb0 + c]);
-                                }
-                            }
-                        }
-                    }
-                }
-                if (nst > 1) {
-                    // the next stage is in (every wave's copies) and this one
-                    // is read: swap
-                    __builtin_amdgcn_s_waitcnt(0);
-                    __syncthreads();
-                    cur ^= 1;
-                }
-            }
-            // ||c||^2 - 2 x.c, first minimum wins (_k_means_lloyd.pyx:196-212);
-            // the lane's centres come in ascending order, passes too.  With
-            // one stage, the pass's ||c||^2 are in it; else they are read as
-            // the previous pass's norms of the stage now current, which the
-            // stage copies rewrite only after the next barrier (a wave past
-            // that barrier has every wave's reads of this behind it).
-            const float* sN = reinterpret_cast<const float*>(smem + cur * G::STAGE + G::PBYTES) + (nst > 1 ? CPC : 0);
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
-                const float4 c4 = *reinterpret_cast<const float4*>(&sN[16 * cb + 4 * h]);
-                const float cn[4] = {c4.x, c4.y, c4.z, c4.w};
-#pragma unroll
-                for (int g = 0; g < 2; ++g) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float dd = fmaf(-2.0f, acc[g][cb][i], cn[i]);  // NaN compares false
-                        const bool take = dd < bd[g];
-                        bd[g] = take ? dd : bd[g];
-                        bi[g] = take ? p * CPC + 16 * cb + 4 * h + i : bi[g];
-                    }
-                }
-            }
-        }
-        int mylab = 0;
-        float mymin = 0.f;
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            float d0 = bd[g];
-            int i0 = bi[g];
-#pragma unroll
-            for (int m = 16; m <= 32; m *= 2) {
-                const float od = __shfl_xor(d0, m);
-                const int oi = __shfl_xor(i0, m);
-                const bool take = (od < d0) | ((od == d0) & (oi < i0));
-                d0 = take ? od : d0;
-                i0 = take ? oi : i0;
-            }
-            if (h == g) {  // lanes 0..31: row = lane
-                mylab = i0;
-                mymin = d0;
-            }
-        }
+        int mylab;
+        float mymin;
+        assign3_rows<CB>(
+            smem, ld, npass, nseg, h, r16, cur, xr, copy_stage, [&](int f) { xload(rs, f); },
+            [&]() {
+                if (base + (long)gridDim.x * 256 < n) xload(rows_rsrc(base + (long)gridDim.x * 256), 0);
+            },
+            mylab, mymin);
         const bool valid = lane < nrow;
         const long row = wrow + lane;
         int moved = 0;
@@ -1132,6 +1085,155 @@ __global__ __launch_bounds__(512, 1) void k_assign3(const float* __restrict__ X,
     }
 }
 
+// k_assign3 for the rows that k_screen left.  Block b takes a contiguous
+// share of the rows: it turns their mask bits into a list in LDS, 2,048 rows'
+// bits at a time until 256 rows are on it, and runs the six products for 256
+// rows of the list (32 per wave) at a time.  Once the screen is off every
+// row is taken.  The list keeps the blocks' work even while rows are left
+// all over X; a share with few rows costs a block one pass over the centres.
+template <int CB>
+__global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict__ X, long n, int ld,
+                                                         const char* __restrict__ img, int k,
+                                                         int* __restrict__ labels, LoopState* st, int* changed,
+                                                         float* __restrict__ emin,
+                                                         const unsigned long long* __restrict__ masks)
+{
+    if (st != nullptr && st->done != 0) return;
+    const bool all = st != nullptr && st->screen_off != 0;
+    using G = Assign3Geom<CB>;
+    constexpr int CPC = G::CPC, SEG = G::SEG;
+    constexpr int CH = 2048;  // rows whose bits are listed at a time, 256 per wave
+    extern __shared__ __attribute__((aligned(1024))) char smem[];  // two stages
+    __shared__ unsigned sList[CH + 256];                           // rows, from the share's first
+    __shared__ int sCnt[8];
+    __shared__ int sChg;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 4, r16 = lane & 15;
+    if (tid == 0) sChg = 0;
+    int nchg = 0;
+    const int npass = (k + CPC - 1) / CPC;
+    const int nseg = (ld + SEG - 1) / SEG;
+    const int nst = npass * nseg;
+    const __amdgpu_buffer_rsrc_t irs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(img), (short)0,
+                                                                         nst * G::STAGE, 0x00020000);
+    const int stage_bytes = G::STAGE;
+    auto copy_stage = [&](int stg, int b) {
+        char* dst = smem + b * stage_bytes;
+        for (int i = wave; i < stage_bytes / 1024; i += 8) {
+            const int soff = stg * stage_bytes + i * 1024;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16,
+                                                     lane * 16, soff, 0, 0);
+        }
+    };
+    const long share = ((n + gridDim.x - 1) / gridDim.x + 63) / 64 * 64;
+    const long r0 = min(n, (long)blockIdx.x * share), r1 = min(n, r0 + share);
+    // (the share's bytes fit 31 bits: at most 1/256 of X, or 256 rows)
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(X + r0 * ld), (short)0,
+                                                                        (int)((r1 - r0) * ld * 4), 0x00020000);
+    float4 xr[2][2];
+    int xo[2];  // byte offsets of this lane's rows
+    // rows i.. of the list (a place past its end repeats the last row)
+    auto rows_at = [&](int i, int cnt) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+            xo[g] = ((int)sList[min(i + 32 * wave + 16 * g + r16, cnt - 1)] * ld + 8 * h) * 4;
+    };
+    // past the row's end the next row's values (or 0) meet zero centre parts
+    auto xload = [&](int f) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            xr[g][0] = load_quad(rs, xo[g] + 4 * f);
+            xr[g][1] = load_quad(rs, xo[g] + 4 * f + 16);
+        }
+    };
+    long c = r0;         // first row whose bits are not listed yet
+    int cnt = 0;         // rows on the list
+    int taken = 0;       // rows listed so far
+    bool staged = false; // stage 0 is in LDS
+    int cur = 0;
+    while (true) {
+        while (cnt < 256 && c < r1) {
+            unsigned long long m[4];
+            int mine = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const long q = c + 256 * wave + 64 * j;
+                const long left = r1 - q;
+                m[j] = left <= 0 ? 0ull : all ? (left >= 64 ? ~0ull : (1ull << left) - 1ull) : masks[q >> 6];
+                mine += (int)__popcll(m[j]);
+            }
+            if (lane == 0) sCnt[wave] = mine;
+            __syncthreads();
+            int at = cnt, tot = 0;
+            for (int w = 0; w < 8; ++w) {
+                at += w < wave ? sCnt[w] : 0;
+                tot += sCnt[w];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if ((m[j] >> lane) & 1ull)
+                    sList[at + (int)__popcll(m[j] & ((1ull << lane) - 1ull))] =
+                        (unsigned)(c - r0) + 256u * wave + 64u * j + lane;
+                at += (int)__popcll(m[j]);
+            }
+            __syncthreads();  // (also: sCnt is read)
+            cnt += tot;
+            taken += tot;
+            c += CH;
+        }
+        if (cnt == 0) break;
+        if (!staged) {
+            copy_stage(0, 0);
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            staged = true;
+        }
+        int pos = 0;
+        rows_at(0, cnt);
+        xload(0);
+        while (cnt - pos >= 256 || (c >= r1 && cnt > pos)) {
+            int mylab;
+            float mymin;
+            assign3_rows<CB>(
+                smem, ld, npass, nseg, h, r16, cur, xr, copy_stage, xload,
+                [&]() {
+                    if (pos + 256 < cnt) {
+                        rows_at(pos + 256, cnt);
+                        xload(0);
+                    }
+                },
+                mylab, mymin);
+            const int i = pos + 32 * wave + lane;
+            const bool valid = lane < 32 && i < cnt;
+            int moved = 0;
+            if (valid) {
+                const long row = r0 + sList[i];
+                if (changed != nullptr) moved = labels[row] != mylab;
+                labels[row] = mylab;
+                if (emin != nullptr) emin[row] = mymin;
+            }
+            if (changed != nullptr) nchg += (int)__popcll(__ballot(moved));
+            pos += 256;
+        }
+        // what is left of the list to its front (less than 256 rows)
+        const int rest = max(0, cnt - pos);
+        const unsigned keep = tid < rest ? sList[pos + tid] : 0u;
+        __syncthreads();
+        if (tid < rest) sList[tid] = keep;
+        cnt = rest;
+        if (cnt == 0 && c >= r1) break;
+        __syncthreads();
+    }
+    if (changed != nullptr) {
+        if (lane == 0 && nchg != 0) atomicAdd(&sChg, nchg);
+        __syncthreads();
+        if (tid == 0 && sChg != 0) atomicAdd(changed, sChg);
+    }
+    if (st != nullptr && !all && tid == 0 && taken != 0) atomicAdd(&st->unsure, taken);
+}
+
 typedef void (*assign3_fn)(const float*, long, int, const char*, int, int*, LoopState*, int*, const float*, int,
                            double*, float*);
 typedef void (*image_fn)(const float*, const float*, int, int, int, char*);
@@ -1176,15 +1278,25 @@ static bool split_disabled()
     return env != nullptr && env[0] == '0';
 }
 
+typedef void (*assign3_list_fn)(const float*, long, int, const char*, int, int*, LoopState*, int*, float*,
+                                const unsigned long long*);
+static assign3_list_fn assign3_list_kernel(int k)
+{
+    const int cb = assign3_cb(k);
+    return cb == 4 ? &k_assign3_list<4> : cb == 8 ? &k_assign3_list<8> : &k_assign3_list<16>;
+}
+
 int assign3_ready(int d, int k)
 {
     if (split_disabled() || d < 17 || k < 1) return 0;
     for (const int kk : {64, 128, 129}) {
-        assign3_fn f = assign3_kernel(kk);
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)assign3_lds(kk)) != hipSuccess) {
-            (void)hipGetLastError();
-            return 0;
+        for (const void* f : {reinterpret_cast<const void*>(assign3_kernel(kk)),
+                              reinterpret_cast<const void*>(assign3_list_kernel(kk))}) {
+            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)assign3_lds(kk)) !=
+                hipSuccess) {
+                (void)hipGetLastError();
+                return 0;
+            }
         }
     }
     return 1;
@@ -1205,6 +1317,42 @@ hipError_t launch_assign3(const AssignArgs& a, int num_cu, hipStream_t s)
     hipLaunchKernelGGL(assign3_kernel(a.k), dim3((unsigned)blocks), dim3(512), assign3_lds(a.k), s, a.X, a.n, a.ld,
                        a.img, a.k, a.labels, a.state, a.changed, a.C, a.d, a.inert, a.emin);
     if (a.inert_blocks != nullptr) *a.inert_blocks = (int)blocks;
+    return hipGetLastError();
+}
+typedef void (*images_fn)(const float*, const float*, int, int, int, int, char*, char*, const LoopState*);
+template <int CB>
+static images_fn images_kernel(int ld)
+{
+    switch ((ld + 31) / 32) {
+    case 1: return &k_centre_images<CB, 1>;
+    case 2: return &k_centre_images<CB, 2>;
+    case 3: return &k_centre_images<CB, 3>;
+    default: return &k_centre_images<CB, 4>;
+    }
+}
+
+hipError_t launch_centre_images(const AssignArgs& a, char* simg, hipStream_t s)
+{
+    if (a.img == nullptr || simg == nullptr) return hipErrorInvalidValue;
+    int nst = 0, nseg = 0;
+    size_t stage = 0;
+    assign3_stages(a.k, a.ld, &nst, &nseg, &stage);
+    const int cb = assign3_cb(a.k);
+    const images_fn f = cb == 4 ? images_kernel<4>(a.ld) : cb == 8 ? images_kernel<8>(a.ld) : images_kernel<16>(a.ld);
+    const int snst = (a.k + kScreenSC - 1) / kScreenSC;
+    hipLaunchKernelGGL(f, dim3((unsigned)(nst + snst)), dim3(256), 0, s, a.C, a.cnorm, a.k, a.ld, nseg, nst, a.img, simg,
+                       a.state);
+    return hipGetLastError();
+}
+
+hipError_t launch_assign3_list(const AssignArgs& a, const unsigned long long* masks, int num_cu, hipStream_t s)
+{
+    if (a.n <= 0) return hipSuccess;
+    if (a.img == nullptr || masks == nullptr) return hipErrorInvalidValue;
+    long blocks = (a.n + 255) / 256;
+    if (blocks > num_cu) blocks = num_cu;
+    hipLaunchKernelGGL(assign3_list_kernel(a.k), dim3((unsigned)blocks), dim3(512), assign3_lds(a.k), s, a.X, a.n,
+                       a.ld, a.img, a.k, a.labels, a.state, a.changed, a.emin, masks);
     return hipGetLastError();
 }
 typedef void (*fused_fn)(FusedArgs);

@@ -1,0 +1,95 @@
+"""The screened E-step (k_screen + k_assign3_list) against the same E-step
+without the screen: the labels, and with them centres and inertia, are the
+same bit for bit whatever share of the rows the screen settles."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _blobs(n, d, k, spread, seed):
+    rng = np.random.default_rng(seed)
+    cen = rng.standard_normal((k, d)) * spread
+    X = (cen[rng.integers(0, k, n)] + rng.standard_normal((n, d))).astype(np.float32)
+    return X, np.ascontiguousarray(X[:k])
+
+
+def _both(monkeypatch, X, C, steps=5):
+    from skmetal_amd import _bridge
+
+    n, d = X.shape
+    k = C.shape[0]
+    got = []
+    for mode in "01":
+        monkeypatch.setenv("SKMETAL_HIP_SCREEN", mode)
+        lab = np.empty(n, np.int32)
+        _bridge.kmeans_assign(X, C, lab, n, d, k)
+        with _bridge.LloydHandle(n, d, k) as h:
+            h.load(X)
+            h.set_centers(C)
+            run = h.run(steps, 0.0, strict=False)
+            got.append((lab, run, h.centers(), h.labels()))
+            assert h.info()["asplit"] and not h.info()["fused"]
+    (l0, r0, c0, f0), (l1, r1, c1, f1) = got
+    np.testing.assert_array_equal(l0, l1)
+    np.testing.assert_array_equal(f0, f1)
+    np.testing.assert_array_equal(c0, c1)
+    assert r0[0] == r1[0] and r0[1] == pytest.approx(r1[1], rel=1e-12)
+    return f1
+
+
+# every K-step count, row ends off the 32-feature and 64-row grid, one stage
+# of centres, several, and more than LDS keeps (k = 2000 at 4 K steps)
+@pytest.mark.parametrize("n,d,k,spread", [
+    (300, 17, 300, 1.0), (777, 37, 101, 0.6), (4099, 66, 129, 0.5), (513, 128, 200, 0.2), (20011, 96, 128, 0.4),
+    (33333, 125, 257, 0.1), (70001, 64, 300, 0.9), (5000, 104, 2000, 0.5), (66, 32, 65, 1.0),
+])
+def test_screen_labels_match_six_products(monkeypatch, n, d, k, spread):
+    _both(monkeypatch, *_blobs(n, d, k, spread, n + d))
+
+
+@pytest.mark.parametrize("kind", ["duplicates", "lattice", "large", "small", "mixed", "zeros"])
+def test_screen_hard_data(monkeypatch, kind):
+    X, C = _blobs(6000, 24, 100, 0.5, 3)
+    if kind == "duplicates":
+        C[50], C[99] = C[3], C[0]  # ties: the lowest index wins
+    elif kind == "lattice":  # exact ties everywhere: the screen settles few rows and is turned off
+        rng = np.random.default_rng(4)
+        X = rng.integers(0, 3, X.shape).astype(np.float32)
+        C = rng.integers(0, 3, C.shape).astype(np.float32)
+    elif kind == "large":
+        X, C = X * np.float32(1e15), C * np.float32(1e15)
+    elif kind == "small":
+        X, C = X * np.float32(1e-14), C * np.float32(1e-14)
+    elif kind == "mixed":
+        X[:, 3] *= 1e6
+        C = np.ascontiguousarray(X[:100])
+    else:
+        X[-50:] = 0.0
+        C[7] = 0.0
+    _both(monkeypatch, X, C)
+
+
+def test_screen_non_finite_centres(monkeypatch):
+    from skmetal_amd import _bridge
+
+    X, C = _blobs(3000, 40, 90, 0.5, 6)
+    C[7], C[9] = np.nan, np.inf
+    lab = [np.empty(3000, np.int32) for _ in range(2)]
+    for mode in (0, 1):
+        monkeypatch.setenv("SKMETAL_HIP_SCREEN", str(mode))
+        _bridge.kmeans_assign(X, C, lab[mode], 3000, 40, 90)
+    np.testing.assert_array_equal(lab[0], lab[1])
+
+
+@pytest.mark.parametrize("n,d,k", [(9000, 50, 80), (30000, 128, 140)])
+def test_screen_relocation(monkeypatch, n, d, k):
+    """Empty clusters: the farthest rows come from the screen's row minima and
+    are those of the six products' minima."""
+    X, C = _blobs(n, d, k, 0.5, 8)
+    C[[4, 20, k - 1]] += 300.0
+    lab = _both(monkeypatch, X, C)
+    assert len(np.unique(lab)) == k
