@@ -96,6 +96,14 @@ hipError_t launch_centre_images(const AssignArgs& a, char* simg, hipStream_t s);
 // taken.  The rows taken are added to state->unsure.
 hipError_t launch_assign3_list(const AssignArgs& a, const unsigned long long* masks, int num_cu, hipStream_t s);
 
+// The same for rows of more than 128 floats: the images of launch_screen_wide
+// (wimg, [wide_image_bytes(k, ld)]) and launch_assign3_units (a.img, k_assign3's
+// for more than 128 centres) with the list emptied; then the six products of
+// the listed rows, unit by unit, and their labels.
+hipError_t launch_wide_images(const AssignArgs& a, char* wimg, int* nlist, hipStream_t s);
+hipError_t launch_assign3_units(const AssignArgs& a, const unsigned* list, const int* nlist, unsigned long long* keys,
+                                int num_cu, hipStream_t s);
+
 // The certified screen in front of the E-step (screen_kernels.hip): labels
 // the rows whose nearest centre one bf16 product settles and leaves the
 // others' bits in masks, for launch_assign3_list.
@@ -111,9 +119,45 @@ struct ScreenArgs {
     unsigned long long* masks;    // [ceil(n / 64)]
 };
 size_t screen_image_bytes(int k, int ld);
-inline bool screen_ready(int ld) { return ld <= 128; }
-inline bool screen_pays(long n, int ld, int k) { return k > 128 && (double)n * ld * k >= 1.2e10; }
 hipError_t launch_screen(const ScreenArgs& a, int num_cu, hipStream_t s);
+// Rows of more than 128 floats: k_screen_wide takes 256 rows x 256 centres a
+// block and leaves each row's two largest values of every 128 centres in
+// `part`; k_screen_merge labels the rows they settle and lists the others.
+struct WideArgs {
+    const float* X; long n; int ld;
+    const float* cnorm; int k;
+    int* labels;
+    LoopState* state;             // nullable: no early exit
+    int* changed;                 // nullable, as AssignArgs
+    const char* img;              // launch_wide_images's wimg
+    float* part;                  // [2 ceil(k / 256)][n][2]
+    float* xx;                    // [n] ||x||^2
+    unsigned* list; int* nlist;   // [n], [1]: the rows left
+    unsigned long long* keys;     // [n], of the rows left
+};
+size_t wide_image_bytes(int k, int ld);
+inline size_t wide_part_floats(long n, int k) { return size_t(n) * size_t(k + 255) / 256 * 4; }
+hipError_t launch_screen_wide(const WideArgs& a, hipStream_t s);
+
+// Where the screen pays.  k_assign3 alone takes its 256-row blocks in rounds
+// of 256 (one a CU), each round proportional to the padded centres times
+// features (0.64 us per 1,000).  Rows of at most 128 floats: what is left
+// costs about one round again (nearly every block has a row) and the second
+// launch and its image 20 us, so it is the rounds after the first that are
+// saved.  Timed, a step without / with the screen: 64 floats, k = 1,024:
+// 60,000 rows 95 / 121 us, 120,000 139 / 129, 1,000,000 767 / 318; 128
+// floats, k = 256: 120,000 97 / 101, 250,000 152 / 127, 1,000,000 493 / 308.
+// Longer rows: the rest goes by units of 256 rows x 256 centres and costs
+// little, but there are two more launches.  768 floats: k = 200 (one unit
+// wide) 64,000 rows 173 / 212 us, 130,000 335 / 306; k = 1,500: 8,000 rows
+// 638 / 156; 300 floats, k = 600: 8,000 rows 168 / 122.
+inline bool screen_pays(long n, int ld, int k)
+{
+    if (n >= (1L << 31) || k <= 128) return false;
+    const double round = (double)((k + 255) / 256 * 256) * ((ld + 31) / 32 * 32);
+    const double rounds = (double)((n + 65535) / 65536);
+    return ld <= 128 ? (rounds - 1) * round >= 60e3 : rounds * round >= 230e3;
+}
 
 // The three-part bf16 split is exact for finite values of magnitude >= 2^-103,
 // and the E-step's smallest kept part products stay normal fp32 numbers when

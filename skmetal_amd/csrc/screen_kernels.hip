@@ -18,8 +18,8 @@ namespace skm {
 // A bound on how far a screen value lies from x.c - ||c||^2 / 2 as the six
 // products give it, for a row with ||x||^2 = xx (fp32 sum) and C2 = the
 // largest ||c||^2, ldp features with the padding:
-//   rounding x and c to bf16 and the index in the low six bits: 2^-8 +
-//   2^-18 + 2^-17 of ||x|| ||c||; the screen's fp32 accumulation, ldp + 1
+//   rounding x and c to bf16 and the index in the low six or seven bits:
+//   2^-8 + 2^-18 + 2^-16 of ||x|| ||c||; the screen's fp32 accumulation, ldp + 1
 //   terms, and the six products', 6 ldp terms, at most 2^-23 of the terms'
 //   magnitudes each (the terms of one row and centre total at most ||x||
 //   ||c|| by Cauchy-Schwarz); the products left out, 2^-22; the same for
@@ -28,8 +28,8 @@ namespace skm {
 __device__ __forceinline__ float screen_slack(float xx, float C2, int ldp)
 {
     const float xn = sqrtf(xx), cn = sqrtf(C2);
-    const float a = 0x1p-8f + 0x1p-16f + 8.f * (float)ldp * 0x1p-23f;
-    const float b = 0x1p-16f + (float)(ldp + 2) * 0x1p-23f;
+    const float a = 0x1p-8f + 0x1p-15f + 8.f * (float)ldp * 0x1p-23f;
+    const float b = 0x1p-15f + (float)(ldp + 2) * 0x1p-23f;
     return 1.05f * (a * xn * cn + b * 0.5f * C2) + 0x1p-100f * (xn + cn) + 0x1p-100f;
 }
 
@@ -49,6 +49,34 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ v16f mfma32_bf16(v8bf a, v8bf b, v16f c)
 {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// A lane's 16 values of a block into its two largest, places p0.. of the
+// stage in their low six bits.
+__device__ __forceinline__ void two_largest(float& m1, float& m2, const v16f& acc, int p0)
+{
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        float u[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            u[i] = __uint_as_float((__float_as_uint(acc[4 * q + i]) & ~63u) | (unsigned)(p0 + 4 * q + i));
+        // with m1 >= m2 the second largest of m1, m2 and two more is the
+        // larger of m2 and the middle one of the rest
+        const float a1 = __builtin_amdgcn_fmed3f(m1, u[0], u[1]);
+        m1 = max3(m1, u[0], u[1]);
+        const float a2 = __builtin_amdgcn_fmed3f(m1, u[2], u[3]);
+        m1 = max3(m1, u[2], u[3]);
+        m2 = max3(m2, a1, a2);
+    }
+    // the values are used up here: sunk to the end of the stage they spill
+    asm volatile("" : "+v"(m1), "+v"(m2));
+}
+
+// The centre of place p of a 128-centre stage, for a lane with h = lane / 32.
+__device__ __forceinline__ int place_centre(int p, int h)
+{
+    return 32 * (p >> 4) + 8 * ((p & 15) >> 2) + 4 * h + (p & 3);
 }
 
 // A block of 8 waves owns 512 rows, 64 per wave in two 32-row groups whose
@@ -179,26 +207,7 @@ __global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
             ms[g] = 0;
         }
         unsigned cmax = 0u;
-        // the 32 rows of group g against one block's centres: the two largest
-        auto take = [&](int g, const v16f& acc, int cb) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float u[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    u[i] = __uint_as_float((__float_as_uint(acc[4 * q + i]) & ~63u) | (unsigned)(16 * cb + 4 * q + i));
-                // with m1 >= m2 the second largest of m1, m2 and two more is
-                // the larger of m2 and the middle one of the rest
-                const float a1 = __builtin_amdgcn_fmed3f(m1[g], u[0], u[1]);
-                m1[g] = max3(m1[g], u[0], u[1]);
-                const float a2 = __builtin_amdgcn_fmed3f(m1[g], u[2], u[3]);
-                m1[g] = max3(m1[g], u[2], u[3]);
-                m2[g] = max3(m2[g], a1, a2);
-            }
-            // the values are used up here: sunk to the end of the stage they
-            // spill
-            asm volatile("" : "+v"(m1[g]), "+v"(m2[g]));
-        };
+        auto take = [&](int g, const v16f& acc, int cb) { two_largest(m1[g], m2[g], acc, 16 * cb); };
         v16f late;  // group 1 of the block before
         if constexpr (PIPE) {
 #pragma unroll
@@ -282,9 +291,7 @@ __global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
         int bi = 0;
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-            // place p of the stage: reg i = p % 16 of block p / 16
-            const int p = (int)(__float_as_uint(m1[g]) & 63u);
-            int i1 = ms[g] * kScreenSC + 32 * (p >> 4) + 8 * ((p & 15) >> 2) + 4 * h + (p & 3);
+            int i1 = ms[g] * kScreenSC + place_centre((int)(__float_as_uint(m1[g]) & 63u), h);
             const float o1 = __shfl_xor(m1[g], 32), o2 = __shfl_xor(m2[g], 32);
             const int oi = __shfl_xor(i1, 32);
             const float x2 = xx[g] + __shfl_xor(xx[g], 32);
@@ -333,6 +340,233 @@ static hipError_t launch_screen_nk(const ScreenArgs& a, int num_cu, hipStream_t 
     const long blocks = (a.n + 511) / 512;
     hipLaunchKernelGGL(k_screen<NK>, dim3((unsigned)(blocks < num_cu ? blocks : num_cu)), dim3(512),
                        (size_t)(resident ? nst : 2) * G::STAGE, s, a, resident);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// rows of more than 128 floats
+// ---------------------------------------------------------------------------
+//
+// A block: 256 rows x 256 centres, wave w the 64 rows 64 (w % 4).. against the
+// 128 centres 128 (w / 4)..: eight 32 x 32 accumulators, six 1 KB operands for
+// eight MFMAs a K16 step (LDS at 96 of its 128 bytes a cycle).  K goes by in
+// stages of 64 features, two in LDS: while one is used, the next one's
+// centres come in with direct-to-LDS loads, and its rows as fp32 into
+// registers, rounded to bf16 on the way to LDS.  Blocks of one row block
+// follow each other on one XCD (block b runs on XCD b % 8), so that X and the
+// image come from its L2.
+__global__ __launch_bounds__(512, 2) void k_screen_wide(WideArgs a)
+{
+    const LoopState* st = a.state;
+    if (st != nullptr && (st->done != 0 || st->screen_off != 0)) return;
+    const int ncg = (a.k + 255) / 256, nks = (a.ld + 63) / 64;
+    const long nrb = (a.n + 255) / 256;
+    const long i = blockIdx.x >> 3;
+    const long rb = (blockIdx.x & 7) + 8 * (i / ncg);
+    const int cg = (int)(i % ncg);
+    if (rb >= nrb) return;
+    extern __shared__ __attribute__((aligned(1024))) char smem[];  // [2] rows, [2] centres
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, r32 = lane & 31;
+    const int ld = a.ld;
+    const long r0 = rb * 256;
+    const int nrow = (int)(a.n - r0 < 256 ? a.n - r0 : 256);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.X + r0 * ld), (short)0,
+                                                                        nrow * ld * 4, 0x00020000);
+    const int stage_bytes = kWideStage;
+    const __amdgpu_buffer_rsrc_t irs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(a.img + (size_t)cg * nks * stage_bytes), (short)0, nks * stage_bytes, 0x00020000);
+    auto copy_centres = [&](int ks, int b) {
+        char* dst = smem + (2 + b) * stage_bytes;
+        for (int q = wave; q < stage_bytes / 1024; q += 8) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (__attribute__((address_space(3))) void*)(dst + q * 1024), 16,
+                                                     lane * 16, ks * stage_bytes + q * 1024, 0, 0);
+        }
+    };
+    // the stage's rows: lane l of wave w loads float4 l % 16 of rows 32 w + 4 u
+    // + l / 16 (past the rows' end 0, past a row's end the next row's values,
+    // which meet zero centre parts)
+    const int q16 = lane & 15, lr = 32 * wave + (lane >> 4);
+    f4v raw[8];
+    float xx[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) xx[u] = 0.f;
+    auto load_rows = [&](int ks) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            raw[u] = __builtin_bit_cast(
+                f4v, __builtin_amdgcn_raw_buffer_load_b128(rs, ((lr + 4 * u) * ld + 64 * ks + 4 * q16) * 4, 0, 0));
+    };
+    auto put_rows = [&](int ks, int b) {
+        __bf16* dst = reinterpret_cast<__bf16*>(smem + b * stage_bytes);
+        const float in = 64 * ks + 4 * q16 < ld ? 1.f : 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const f4v v = raw[u];
+            *reinterpret_cast<v2u*>(dst + (lr + 4 * u) * kWideStr + 4 * q16) =
+                v2u{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
+            if (cg == 0) xx[u] = fmaf(fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w))), in, xx[u]);
+        }
+    };
+    load_rows(0);
+    copy_centres(0, 0);
+    const int wr = wave & 3, wc = wave >> 2;
+    // the accumulators start from -||c||^2 / 2
+    const float* const ini =
+        reinterpret_cast<const float*>(a.img + (size_t)ncg * nks * stage_bytes) + 256 * cg + 128 * wc + 4 * h;
+    v16f acc[4][2];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f4v v = *reinterpret_cast<const f4v*>(ini + 32 * c + 8 * q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[c][0][4 * q + e] = v[e];
+        }
+        acc[c][1] = acc[c][0];
+    }
+    put_rows(0, 0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    for (int ks = 0; ks < nks; ++ks) {
+        const int cur = ks & 1;
+        if (ks + 1 < nks) {
+            copy_centres(ks + 1, cur ^ 1);
+            load_rows(ks + 1);
+        }
+        const __bf16* const xb =
+            reinterpret_cast<const __bf16*>(smem + cur * stage_bytes) + (64 * wr + r32) * kWideStr + 8 * h;
+        const __bf16* const cb =
+            reinterpret_cast<const __bf16*>(smem + (2 + cur) * stage_bytes) + (128 * wc + r32) * kWideStr + 8 * h;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            v8bf x[2], c[4];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) x[g] = *reinterpret_cast<const v8bf*>(xb + 32 * g * kWideStr + 16 * s);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c[e] = *reinterpret_cast<const v8bf*>(cb + 32 * e * kWideStr + 16 * s);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int g = 0; g < 2; ++g) acc[e][g] = mfma32_bf16(c[e], x[g], acc[e][g]);
+            }
+        }
+        if (ks + 1 < nks) {
+            put_rows(ks + 1, cur ^ 1);
+            // the next stage is in and this one is read: swap
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        float m1 = -INFINITY, m2 = -INFINITY;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) two_largest(m1, m2, acc[c][g], 16 * c);
+        // the two lanes of a row: the larger value carries the centre's place
+        // among the 128 in its low seven bits
+        const int id = place_centre((int)(__float_as_uint(m1) & 63u), h);
+        m1 = __uint_as_float((__float_as_uint(m1) & ~127u) | (unsigned)id);
+        const float o1 = __shfl_xor(m1, 32), o2 = __shfl_xor(m2, 32);
+        m2 = fmaxf(fminf(m1, o1), fmaxf(m2, o2));
+        m1 = fmaxf(m1, o1);
+        const int r = 64 * wr + 32 * g + r32;
+        if (h == 0 && r < nrow)
+            reinterpret_cast<float2*>(a.part)[(long)(2 * cg + wc) * a.n + r0 + r] = make_float2(m1, m2);
+    }
+    if (cg == 0) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            float t = xx[u];
+            t += __shfl_xor(t, 1);
+            t += __shfl_xor(t, 2);
+            t += __shfl_xor(t, 4);
+            t += __shfl_xor(t, 8);
+            const int r = lr + 4 * u;
+            if (q16 == 0 && r < nrow) a.xx[r0 + r] = t;
+        }
+    }
+}
+
+// A thread per row: the two largest over the parts, then the row's label or
+// its place on the list.
+__global__ __launch_bounds__(256) void k_screen_merge(WideArgs a)
+{
+    const LoopState* st = a.state;
+    if (st != nullptr && st->done != 0) return;
+    const bool all = st != nullptr && st->screen_off != 0;
+    constexpr unsigned long long kNone = 0xff800000ull << 32;  // +inf in order_bits's form, centre 0
+    const long row = (long)blockIdx.x * 256 + threadIdx.x;
+    if (all) {
+        if (row < a.n) a.keys[row] = kNone;
+        return;
+    }
+    __shared__ unsigned sMax;
+    __shared__ int sChg, sLeft, sAt;
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        sMax = 0u;
+        sChg = 0;
+        sLeft = 0;
+    }
+    __syncthreads();
+    unsigned cm = 0u;  // the largest ||c||^2 as bits: NaN counts above every number
+    for (int j = tid; j < a.k; j += 256) cm = max(cm, __float_as_uint(a.cnorm[j]) & 0x7fffffffu);
+    atomicMax(&sMax, cm);
+    const int np = 2 * ((a.k + 255) / 256);
+    float m1 = -INFINITY, m2 = -INFINITY;
+    int mp = 0;
+    const bool valid = row < a.n;
+    if (valid) {
+        for (int p = 0; p < np; ++p) {
+            const float2 v = reinterpret_cast<const float2*>(a.part)[(long)p * a.n + row];
+            m2 = fmaxf(fminf(m1, v.x), fmaxf(m2, v.y));
+            if (v.x > m1) {
+                m1 = v.x;
+                mp = p;
+            }
+        }
+    }
+    __syncthreads();
+    const float C2 = __uint_as_float(sMax), xx = valid ? a.xx[row] : 0.f;
+    const float slack = screen_slack(xx, C2, 64 * ((a.ld + 63) / 64));
+    const bool sure = (m1 - m2 > 2.f * slack) & (sqrtf(xx) * sqrtf(C2) + C2 < 1e37f);
+    int at = 0;
+    if (valid && sure) {
+        const int lab = 128 * mp + (int)(__float_as_uint(m1) & 127u);
+        if (a.changed != nullptr && a.labels[row] != lab) atomicAdd(&sChg, 1);
+        a.labels[row] = lab;
+    } else if (valid) {
+        at = atomicAdd(&sLeft, 1);
+        a.keys[row] = kNone;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        if (a.changed != nullptr && sChg != 0) atomicAdd(a.changed, sChg);
+        sAt = sLeft != 0 ? atomicAdd(a.nlist, sLeft) : 0;
+    }
+    __syncthreads();
+    if (valid && !sure) a.list[sAt + at] = (unsigned)row;
+}
+
+size_t wide_image_bytes(int k, int ld)
+{
+    const size_t ncg = size_t(k + 255) / 256, nks = size_t(ld + 63) / 64;
+    return ncg * nks * kWideStage + ncg * 256 * sizeof(float);
+}
+
+hipError_t launch_screen_wide(const WideArgs& a, hipStream_t s)
+{
+    if (a.n <= 0) return hipSuccess;
+    static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_screen_wide),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, 4 * kWideStage);
+    if (e != hipSuccess) return e;
+    const long nrb = (a.n + 255) / 256, ncg = (a.k + 255) / 256;
+    const long grid = 8 * ((nrb + 7) / 8) * ncg;
+    if (grid >= (1L << 31)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_screen_wide, dim3((unsigned)grid), dim3(512), 4 * kWideStage, s, a);
+    hipLaunchKernelGGL(k_screen_merge, dim3((unsigned)nrb), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -684,12 +684,16 @@ struct Lloyd {
 
     char* a3img = nullptr;  // k_assign3's centre image
     char* simg = nullptr;   // k_screen's
-    unsigned long long* smask = nullptr;  // [ceil(n / 64)] the rows it leaves
+    unsigned long long* smask = nullptr;  // [ceil(n / 64)] the rows it leaves; long rows: their keys [n]
+    float* spart = nullptr;  // long rows: WideArgs::part, xx, list and nlist
+    float* sxx = nullptr;
+    unsigned* slist = nullptr;
+    int* snlist = nullptr;
     // the E-step behind k_screen.  SKMETAL_HIP_SCREEN=0 keeps every row on
     // the six products, 1 screens every shape that the screen takes (tests)
     bool screened() const
     {
-        if (!split_on || !a3cap || !screen_ready(ld)) return false;
+        if (!split_on || !a3cap || n >= (1L << 31) || (ld > 128 && k <= 128)) return false;
         const char* e = getenv("SKMETAL_HIP_SCREEN");
         if (e != nullptr && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
         return screen_pays(n, ld, k);
@@ -702,6 +706,21 @@ struct Lloyd {
             if (a3img == nullptr) TRY(grab((void**)&a3img, assign3_image_bytes(k, ld)));
             a.img = a3img;
             if (minima) a.emin = emin;
+            if (screened() && ld > 128) {
+                if (simg == nullptr) {
+                    TRY(grab((void**)&spart, wide_part_floats(n, k) * sizeof(float)));
+                    TRY(grab((void**)&sxx, size_t(n) * sizeof(float)));
+                    TRY(grab((void**)&slist, size_t(n) * sizeof(unsigned)));
+                    TRY(grab((void**)&snlist, sizeof(int)));
+                    TRY(grab((void**)&smask, size_t(n) * sizeof(unsigned long long)));
+                    TRY(grab((void**)&simg, wide_image_bytes(k, ld)));
+                }
+                const WideArgs wa{X, n, ld, cnorm, k, labels, state, changed, simg, spart, sxx, slist, snlist, smask};
+                HIP_TRY(launch_wide_images(a, simg, snlist, s), "centre image launch");
+                HIP_TRY(launch_screen_wide(wa, s), "screen launch");
+                HIP_TRY(launch_assign3_units(a, slist, snlist, smask, C->num_cu, s), "assign launch");
+                return 0;
+            }
             if (screened()) {
                 if (simg == nullptr) {
                     TRY(grab((void**)&simg, screen_image_bytes(k, ld)));

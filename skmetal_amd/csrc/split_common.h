@@ -139,4 +139,28 @@ __device__ __forceinline__ void screen_image(const float* __restrict__ C, const 
     if (tid == 0) reinterpret_cast<unsigned*>(sn)[kScreenSC] = sMax;
 }
 
+// Stage b = cg nks + ks of k_screen_wide's image, by a block of 256 threads:
+// features 64 ks.. of centres 256 cg.. as rows of 64 bf16 (the high parts),
+// padded to 72; after the last stage, -||c||^2 / 2 of every centre (-3e38
+// past k).
+constexpr int kWideStr = 72;                       // bf16 per LDS row: an odd number of 16-byte units
+constexpr int kWideStage = 256 * kWideStr * 2;     // bytes
+__device__ __forceinline__ void wide_image(const float* __restrict__ C, const float* __restrict__ cnorm, int k, int ld,
+                                           char* __restrict__ img, int b)
+{
+    const int nks = (ld + 63) / 64, cg = b / nks, ks = b - cg * nks, ncg = (k + 255) / 256;
+    __bf16* const out = reinterpret_cast<__bf16*>(img + (size_t)b * kWideStage);
+    for (int e = threadIdx.x; e < 256 * 16; e += 256) {
+        const int c = e >> 4, q = e & 15, j = 256 * cg + c, f = 64 * ks + 4 * q;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (j < k && f < ld) v = *reinterpret_cast<const float4*>(C + (long)j * ld + f);
+        *reinterpret_cast<v2u*>(out + c * kWideStr + 4 * q) = v2u{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
+    }
+    if (ks == 0) {
+        const int j = 256 * cg + threadIdx.x;
+        float* const ini = reinterpret_cast<float*>(img + (size_t)ncg * nks * kWideStage);
+        ini[j] = j < k ? -0.5f * cnorm[j] : -3e38f;
+    }
+}
+
 }  // namespace skm

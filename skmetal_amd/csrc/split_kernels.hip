@@ -812,6 +812,47 @@ __global__ __launch_bounds__(256) void k_centre_images(const float* __restrict__
         screen_image<NK>(C, cnorm, k, ld, simg, (int)blockIdx.x - nst);
 }
 
+// acc += one K step (32 features) of the wave's 32 rows (xp, two 16-row
+// groups) against 16 CB centres: cbase is the K step of this lane's centre
+// row in the stage's high parts.
+template <int CB>
+__device__ __forceinline__ void six_products(v4f (&acc)[2][CB], const Parts8 (&xp)[2], const __bf16* cbase)
+{
+    using G = Assign3Geom<CB>;
+    // four centre blocks at a time, product-major over their
+    // eight accumulators: consecutive MFMAs write different
+    // accumulators (a block's six products back to back wait
+    // on each other).  Each accumulator takes dot6's products
+    // in dot6's order.
+    constexpr int CG = 4;
+#pragma unroll
+    for (int cb0 = 0; cb0 < CB; cb0 += CG) {
+        Parts8 cpt[CG];
+#pragma unroll
+        for (int c = 0; c < CG; ++c) {
+            const __bf16* cp = cbase + 16 * (cb0 + c) * G::CSTR;
+            cpt[c] = Parts8{*reinterpret_cast<const v8bf*>(cp),
+                            *reinterpret_cast<const v8bf*>(cp + G::CPART),
+                            *reinterpret_cast<const v8bf*>(cp + 2 * G::CPART)};
+        }
+#pragma unroll
+        for (int pr = 0; pr < 6; ++pr) {
+#pragma unroll
+            for (int c = 0; c < CG; ++c) {
+                const Parts8& cc = cpt[c];
+                const v8bf ca = pr == 0 ? cc.m : pr == 1 ? cc.l : pr == 2 ? cc.h : pr == 3 ? cc.m : cc.h;
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const Parts8& x = xp[g];
+                    const v8bf xb = pr == 0 ? x.m : pr == 1 ? x.h : pr == 2 ? x.l : pr == 3 ? x.h
+                                                                               : pr == 4 ? x.m : x.h;
+                    acc[g][cb0 + c] = mfma_bf16(ca, xb, acc[g][cb0 + c]);
+                }
+            }
+        }
+    }
+}
+
 // One 32-row block of a wave against every centre: lane l < 32 ends with row
 // l's label and minimum ||c||^2 - 2 x.c.  xr holds the rows' first K step
 // (rows 16g + l%16, features 8h..) and `cur` the LDS stage with stage 0 of
@@ -858,38 +899,7 @@ __device__ __forceinline__ void assign3_rows(char* smem, int ld, int npass, int 
                 // the next stage's copy goes out behind the X loads that
                 // this stage still waits on (loads complete in order)
                 if (ks == nks - 1 && nst > 1) copy_stage(stg + 1 < nst ? stg + 1 : 0, cur ^ 1);
-                // four centre blocks at a time, product-major over their
-                // eight accumulators: consecutive MFMAs write different
-                // accumulators (a block's six products back to back wait
-                // on each other).  Each accumulator takes dot6's products
-                // in dot6's order.
-                constexpr int CG = 4;
-#pragma unroll
-                for (int cb0 = 0; cb0 < CB; cb0 += CG) {
-                    Parts8 cpt[CG];
-#pragma unroll
-                    for (int c = 0; c < CG; ++c) {
-                        const __bf16* cp = cbase + 16 * (cb0 + c) * CSTR + 32 * ks;
-                        cpt[c] = Parts8{*reinterpret_cast<const v8bf*>(cp),
-                                        *reinterpret_cast<const v8bf*>(cp + CPART),
-                                        *reinterpret_cast<const v8bf*>(cp + 2 * CPART)};
-                    }
-#pragma unroll
-                    for (int pr = 0; pr < 6; ++pr) {
-#pragma unroll
-                        for (int c = 0; c < CG; ++c) {
-                            const Parts8& cc = cpt[c];
-                            const v8bf ca = pr == 0 ? cc.m : pr == 1 ? cc.l : pr == 2 ? cc.h : pr == 3 ? cc.m : cc.h;
-#pragma unroll
-                            for (int g = 0; g < 2; ++g) {
-                                const Parts8& x = xp[g];
-                                const v8bf xb = pr == 0 ? x.m : pr == 1 ? x.h : pr == 2 ? x.l : pr == 3 ? x.h
-                                                                                           : pr == 4 ? x.m : x.h;
-                                acc[g][cb0 + c] = mfma_bf16(ca, xb, acc[g][cb0 + c]);
-                            }
-                        }
-                    }
-                }
+                six_products<CB>(acc, xp, cbase + 32 * ks);
             }
             if (nst > 1) {
                 // the next stage is in (every wave's copies) and this one
@@ -1234,6 +1244,187 @@ __global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict
     if (st != nullptr && !all && tid == 0 && taken != 0) atomicAdd(&st->unsure, taken);
 }
 
+// k_assign3 split over the centres as well, for long rows: a unit is 256 rows
+// (of the list that k_screen_merge left, or, once the screen is off, of X)
+// against one pass of 256 centres, and its row minima meet in `keys` by a
+// 64-bit minimum of (distance, centre) -- the first minimum over all centres,
+// in any order of the units.  With 768 floats a row 256 rows against 2,048
+// centres keep a CU busy for 0.8 ms, so a few hundred rows left all over X
+// would cost as much as all of them, and 391 row blocks 2 full rounds of 256
+// CUs.  Units of one row block follow each other on one XCD (block b runs on
+// XCD b % 8): X comes from its L2.
+__device__ __forceinline__ unsigned order_bits(float v)
+{
+    const unsigned b = __float_as_uint(v + 0.f);  // -0 counts as 0
+    return b ^ ((b >> 31) != 0u ? 0xffffffffu : 0x80000000u);
+}
+
+__global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restrict__ X, long n, int ld,
+                                                          const char* __restrict__ img,
+                                                          const float* __restrict__ cnorm, int k,
+                                                          const unsigned* __restrict__ list, const int* nlist,
+                                                          LoopState* st, unsigned long long* __restrict__ keys)
+{
+    if (st != nullptr && st->done != 0) return;
+    constexpr int CB = 16;
+    using G = Assign3Geom<CB>;
+    constexpr int CPC = G::CPC;
+    static_assert(G::NKS == 1, "one K step a stage");
+    const bool all = st != nullptr && st->screen_off != 0;
+    const long cnt = all ? n : (long)*nlist;
+    if (st != nullptr && !all && blockIdx.x == 0 && threadIdx.x == 0) st->unsure = (int)min(cnt, 0x7fffffffL);
+    const int npass = (k + CPC - 1) / CPC;
+    const int nseg = (ld + 31) / 32;
+    const long nb = (cnt + 255) / 256;
+    // XCD x takes the row blocks x, x + 8, ..: its unit i is pass i % npass
+    // of row block x + 8 (i / npass)
+    const int xcd = blockIdx.x & 7, slots = (int)(gridDim.x >> 3);
+    long i = blockIdx.x >> 3;
+    auto block_of = [&](long j) { return xcd + 8 * (j / npass); };
+    if (block_of(i) >= nb) return;
+    extern __shared__ __attribute__((aligned(1024))) char smem[];  // two stages
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 4, r16 = lane & 15;
+    const __amdgpu_buffer_rsrc_t irs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(img), (short)0,
+                                                                         npass * nseg * G::STAGE, 0x00020000);
+    const int stage_bytes = G::STAGE;
+    auto copy_stage = [&](int stg, int b) {
+        char* dst = smem + b * stage_bytes;
+        for (int q = wave; q < stage_bytes / 1024; q += 8) {
+            const int soff = stg * stage_bytes + q * 1024;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (__attribute__((address_space(3))) void*)(dst + q * 1024), 16,
+                                                     lane * 16, soff, 0, 0);
+        }
+    };
+    float4 xr[2][2];
+    const float* xp[2];
+    // (a place past the list's end repeats its last row)
+    auto rows_at = [&](long j) {
+        const long b0 = block_of(j) * 256 + 32 * wave + r16;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const long q = min(b0 + 16 * g, cnt - 1);
+            xp[g] = X + (all ? q : (long)list[q]) * ld;
+        }
+    };
+    // past the row's end its first values meet zero centre parts
+    auto xload = [&](int f) {
+        const int o0 = f + 8 * h < ld ? f + 8 * h : 0, o1 = f + 8 * h + 4 < ld ? f + 8 * h + 4 : 0;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            xr[g][0] = *reinterpret_cast<const float4*>(xp[g] + o0);
+            xr[g][1] = *reinterpret_cast<const float4*>(xp[g] + o1);
+        }
+    };
+    rows_at(i);
+    xload(0);
+    copy_stage((int)(i % npass) * nseg, 0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    int cur = 0;
+    while (true) {
+        const int p = (int)(i % npass);
+        const long row0 = block_of(i) * 256 + 32 * wave;
+        const long nx = i + slots;
+        const bool more = block_of(nx) < nb;
+        v4f acc[2][CB];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) acc[g][cb] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
+        for (int sg = 0; sg < nseg; ++sg) {
+            const __bf16* const cbase = reinterpret_cast<const __bf16*>(smem + cur * G::STAGE) + r16 * G::CSTR + 8 * h;
+            Parts8 part[2];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) part[g] = split8(xr[g][0], xr[g][1]);
+            if (sg + 1 < nseg) {
+                xload(32 * (sg + 1));
+                copy_stage(p * nseg + sg + 1, cur ^ 1);
+            } else if (more) {
+                rows_at(nx);
+                xload(0);
+                copy_stage((int)(nx % npass) * nseg, cur ^ 1);
+            }
+            six_products<CB>(acc, part, cbase);
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            cur ^= 1;
+        }
+        // ||c||^2 - 2 x.c, first minimum wins
+        float bd[2] = {INFINITY, INFINITY};
+        int bi[2] = {0, 0};
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int j = p * CPC + 16 * cb + 4 * h + q;
+                const float cn = j < k ? cnorm[j] : INFINITY;
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const float dd = fmaf(-2.0f, acc[g][cb][q], cn);  // NaN compares false
+                    const bool take = dd < bd[g];
+                    bd[g] = take ? dd : bd[g];
+                    bi[g] = take ? j : bi[g];
+                }
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            unsigned long long key = ((unsigned long long)order_bits(bd[g]) << 32) | (unsigned)bi[g];
+#pragma unroll
+            for (int m = 16; m <= 32; m *= 2) {
+                const unsigned long long o = __shfl_xor(key, m);
+                key = o < key ? o : key;
+            }
+            const long q = row0 + 16 * g + r16;
+            if (h == g && q < cnt && (key >> 32) < order_bits(INFINITY)) {
+                const long row = all ? q : (long)list[q];
+                atomicMin(&keys[row], key);
+            }
+        }
+        if (!more) break;
+        i = nx;
+    }
+}
+
+// The labels of the units' rows from their keys.
+__global__ __launch_bounds__(256) void k_units_finish(long n, const unsigned* __restrict__ list, const int* nlist,
+                                                      const unsigned long long* __restrict__ keys,
+                                                      int* __restrict__ labels, LoopState* st, int* changed)
+{
+    if (st != nullptr && st->done != 0) return;
+    const bool all = st != nullptr && st->screen_off != 0;
+    const long cnt = all ? n : (long)*nlist;
+    __shared__ int sChg;
+    if (threadIdx.x == 0) sChg = 0;
+    __syncthreads();
+    for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < cnt; q += (long)gridDim.x * 256) {
+        const long row = all ? q : (long)list[q];
+        const int lab = (int)(unsigned)keys[row];
+        if (changed != nullptr && labels[row] != lab) atomicAdd(&sChg, 1);
+        labels[row] = lab;
+    }
+    __syncthreads();
+    if (changed != nullptr && threadIdx.x == 0 && sChg != 0) atomicAdd(changed, sChg);
+}
+
+// The centre images of k_assign3_units (nst stages) and of k_screen_wide (the
+// blocks past them); block 0 empties the list.
+__global__ __launch_bounds__(256) void k_wide_images(const float* __restrict__ C, const float* __restrict__ cnorm, int k,
+                                                     int ld, int nst, char* __restrict__ img, char* __restrict__ wimg,
+                                                     int* nlist, const LoopState* st)
+{
+    if (st != nullptr && st->done != 0) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *nlist = 0;
+    if ((int)blockIdx.x < nst)
+        centre_image<16>(C, cnorm, k, ld, (ld + 31) / 32, img);
+    else
+        wide_image(C, cnorm, k, ld, wimg, (int)blockIdx.x - nst);
+}
+
 typedef void (*assign3_fn)(const float*, long, int, const char*, int, int*, LoopState*, int*, const float*, int,
                            double*, float*);
 typedef void (*image_fn)(const float*, const float*, int, int, int, char*);
@@ -1353,6 +1544,35 @@ hipError_t launch_assign3_list(const AssignArgs& a, const unsigned long long* ma
     if (blocks > num_cu) blocks = num_cu;
     hipLaunchKernelGGL(assign3_list_kernel(a.k), dim3((unsigned)blocks), dim3(512), assign3_lds(a.k), s, a.X, a.n,
                        a.ld, a.img, a.k, a.labels, a.state, a.changed, a.emin, masks);
+    return hipGetLastError();
+}
+hipError_t launch_wide_images(const AssignArgs& a, char* wimg, int* nlist, hipStream_t s)
+{
+    if (a.img == nullptr || wimg == nullptr) return hipErrorInvalidValue;
+    const int nst = (a.k + 255) / 256 * ((a.ld + 31) / 32);
+    const int wst = (a.k + 255) / 256 * ((a.ld + 63) / 64);
+    hipLaunchKernelGGL(k_wide_images, dim3((unsigned)(nst + wst)), dim3(256), 0, s, a.C, a.cnorm, a.k, a.ld, nst, a.img,
+                       wimg, nlist, a.state);
+    return hipGetLastError();
+}
+
+hipError_t launch_assign3_units(const AssignArgs& a, const unsigned* list, const int* nlist, unsigned long long* keys,
+                                int num_cu, hipStream_t s)
+{
+    if (a.n <= 0) return hipSuccess;
+    static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_assign3_units),
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    (int)Assign3Geom<16>::LDS);
+    if (e != hipSuccess) return e;
+    // whole rounds of the eight XCDs, one block per CU
+    const long units = (a.n + 255) / 256 * ((a.k + 255) / 256);
+    long blocks = num_cu < units ? num_cu : units;
+    blocks = (blocks + 7) / 8 * 8;
+    hipLaunchKernelGGL(k_assign3_units, dim3((unsigned)blocks), dim3(512), Assign3Geom<16>::LDS, s, a.X, a.n, a.ld,
+                       a.img, a.cnorm, a.k, list, nlist, a.state, keys);
+    const long fb = (a.n + 255) / 256;
+    hipLaunchKernelGGL(k_units_finish, dim3((unsigned)(fb < num_cu ? fb : num_cu)), dim3(256), 0, s, a.n, list, nlist,
+                       keys, a.labels, a.state, a.changed);
     return hipGetLastError();
 }
 typedef void (*fused_fn)(FusedArgs);

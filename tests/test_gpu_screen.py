@@ -46,14 +46,18 @@ def _both(monkeypatch, X, C, steps=5):
 @pytest.mark.parametrize("n,d,k,spread", [
     (300, 17, 300, 1.0), (777, 37, 101, 0.6), (4099, 66, 129, 0.5), (513, 128, 200, 0.2), (20011, 96, 128, 0.4),
     (33333, 125, 257, 0.1), (70001, 64, 300, 0.9), (5000, 104, 2000, 0.5), (66, 32, 65, 1.0),
+    # rows of more than 128 floats: 256 x 256 units, ends off both, one
+    # 64-feature stage more than whole ones
+    (3000, 129, 200, 0.5), (777, 300, 257, 0.4), (20011, 768, 700, 0.3), (300, 1000, 300, 0.2), (256, 192, 256, 0.3),
 ])
 def test_screen_labels_match_six_products(monkeypatch, n, d, k, spread):
     _both(monkeypatch, *_blobs(n, d, k, spread, n + d))
 
 
+@pytest.mark.parametrize("d", [24, 150])
 @pytest.mark.parametrize("kind", ["duplicates", "lattice", "large", "small", "mixed", "zeros"])
-def test_screen_hard_data(monkeypatch, kind):
-    X, C = _blobs(6000, 24, 100, 0.5, 3)
+def test_screen_hard_data(monkeypatch, kind, d):
+    X, C = _blobs(6000, d, 140, 0.5, 3)
     if kind == "duplicates":
         C[50], C[99] = C[3], C[0]  # ties: the lowest index wins
     elif kind == "lattice":  # exact ties everywhere: the screen settles few rows and is turned off
@@ -66,26 +70,27 @@ def test_screen_hard_data(monkeypatch, kind):
         X, C = X * np.float32(1e-14), C * np.float32(1e-14)
     elif kind == "mixed":
         X[:, 3] *= 1e6
-        C = np.ascontiguousarray(X[:100])
+        C = np.ascontiguousarray(X[:140])
     else:
         X[-50:] = 0.0
         C[7] = 0.0
     _both(monkeypatch, X, C)
 
 
-def test_screen_non_finite_centres(monkeypatch):
+@pytest.mark.parametrize("d", [40, 130])
+def test_screen_non_finite_centres(monkeypatch, d):
     from skmetal_amd import _bridge
 
-    X, C = _blobs(3000, 40, 90, 0.5, 6)
+    X, C = _blobs(3000, d, 150, 0.5, 6)
     C[7], C[9] = np.nan, np.inf
     lab = [np.empty(3000, np.int32) for _ in range(2)]
     for mode in (0, 1):
         monkeypatch.setenv("SKMETAL_HIP_SCREEN", str(mode))
-        _bridge.kmeans_assign(X, C, lab[mode], 3000, 40, 90)
+        _bridge.kmeans_assign(X, C, lab[mode], 3000, d, 150)
     np.testing.assert_array_equal(lab[0], lab[1])
 
 
-@pytest.mark.parametrize("n,d,k", [(9000, 50, 80), (30000, 128, 140)])
+@pytest.mark.parametrize("n,d,k", [(9000, 50, 80), (30000, 128, 140), (5000, 200, 150)])
 def test_screen_relocation(monkeypatch, n, d, k):
     """Empty clusters: the farthest rows come from the screen's row minima and
     are those of the six products' minima."""
