@@ -263,8 +263,9 @@ struct FinalizeArgs {
 };
 // Per-(cluster, column chunk) totals, then (with_loop) the loop decision.
 hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t s, bool with_loop);
-// The loop decision alone (after a fused step whose successor is not enqueued).
-// nch: the chunk count the partials were written with (0: that of a.R).
+// The loop decision alone (after a fused step whose successor is not enqueued,
+// or without the in-stream relocation).  nch: the chunk count the partials were
+// written with (0: that of a.R, or in record mode the folded values).
 hipError_t launch_finalize_loop(const FinalizeArgs& a, hipStream_t s, int nch = 0);
 // A finalize block is 256 threads = 8 float4 columns (32 columns) x 32
 // partial-sum lanes.
@@ -340,11 +341,16 @@ struct InRelocArgs {
     // xnorm + emin lies within margin (max ||x||^2 + max ||c||^2) of the
     // distance (2^-10 for the six products, 2^-7 for the screen's minima)
     float margin = 0x1p-10f;
+    // record mode (both or neither): the clusters' folded shift^2 and ||c||^2
+    float* fold_shift = nullptr;
+    float* fold_cnorm = nullptr;
 };
 constexpr int kRelocInlineBlocks = 256;  // grid of k_reloc / k_finalize_reloc (one block per CU: their LDS)
 constexpr int kRelocLdsRows = 4096;      // a block's row distances kept in LDS (more rows: InRelocArgs::dist)
 constexpr int kRelocCandBlocks = kRelocInlineBlocks > kRelocBlocks ? kRelocInlineBlocks : kRelocBlocks;  // candidate list rows
-hipError_t launch_reloc_inline(const InRelocArgs& a, hipStream_t s);
+// decide: the step's loop decision (f) is made here too, once the clusters are
+// relocated.
+hipError_t launch_reloc_inline(const InRelocArgs& a, const FinalizeArgs& f, int decide, hipStream_t s);
 // The fused step's k_finalize_cols and k_reloc in one launch (k <= 64, at
 // most kRelocInlineBlocks finalize chunks, no update records): the empty
 // clusters come from the fused kernel's presence bits.
@@ -441,11 +447,11 @@ hipError_t launch_transform(const TransformArgs& a, hipStream_t s);
 hipError_t launch_colsum(const float* X, long n, int ld, int d, double* part, int nblk, hipStream_t s);
 int colsum_grid(long n);
 hipError_t launch_colmean(const double* part, int nblk, long n, int d, float* mean, hipStream_t s);
-hipError_t launch_center(float* X, long n, int ld, int d, const float* mean, hipStream_t s);
-// max |x| over count floats (NaN as +inf) into *out as float bits
-hipError_t launch_absmax(const float* X, long count, unsigned* out, hipStream_t s);
-// out[r] = ||x_r||^2 (fp32) of the n rows of stride ld (d features)
-hipError_t launch_rownorm(const float* X, long n, int ld, int d, float* out, hipStream_t s);
-hipError_t launch_cnorm(const float* C, int k, int ld, float* cnorm, hipStream_t s);
+// One pass over X [n x ld]: mean (nullable, [ld], 0 in the pad columns) taken
+// off, max |x| (NaN as +inf) into *out as float bits, ||x||^2 of the rows
+// (fp32) into norm (nullable).  X is written only with a mean.
+hipError_t launch_load_pass(float* X, long n, int ld, const float* mean, unsigned* out, float* norm, hipStream_t s);
+// The centres' mean taken off (nullable; d columns) and their ||c||^2.
+hipError_t launch_cnorm(float* C, int k, int ld, int d, const float* mean, float* cnorm, hipStream_t s);
 
 }  // namespace skm

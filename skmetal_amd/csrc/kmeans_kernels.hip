@@ -1026,78 +1026,150 @@ __global__ __launch_bounds__(256) void k_finalize_cols(FinalizeArgs a)
     finalize_cols_block(a, blockIdx.x, blockIdx.y, gridDim.y);
 }
 
-// Record mode (the sorted update: a cluster has a few records, one per
-// chunk of sorted rows it touches): one wave per (cluster j, column chunk
-// cc), item 4 blockIdx.x + wave of k nch.  Lane (rs, q) = (lane / 8, lane %
-// 8) adds the float4 of columns 32 cc + 4q of records rs, rs + 8, .. in
-// fp64, and the eight rs lanes are combined by an xor butterfly.  A block
-// per item made 98,304 blocks at 4096 clusters of 768 floats, each waiting
-// on one round trip.
-__global__ __launch_bounds__(256) void k_finalize_recs(FinalizeArgs a, int nch)
+// One 32-column chunk of record mode's finalize from its fp64 column sums:
+// lane c < 32 holds column 32 cc + c's total.  Returns the chunk's shift^2
+// (lanes 0..31) and ||c||^2 (lanes 32..63).
+__device__ __forceinline__ void finalize_chunk(const FinalizeArgs& a, int j, int cc, int count, double tot,
+                                               float c_old, double* sq_out, double* nrm_out)
 {
-    const int lane = threadIdx.x & 63;
-    const long item = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (item >= (long)a.k * nch) return;
-    const int j = (int)(item / nch), cc = (int)(item - (long)j * nch);
-    const int done = a.state->done;
-    const int q = lane & 7, rs = lane >> 3;
-    const int c4 = cc * 32 + 4 * q;
-    const int ccol = cc * 32 + lane;  // lanes 0..31: one column each
-    const float c_old = lane < 32 && ccol < a.d ? a.C_old[(long)j * a.ld + ccol] : 0.f;
-    const int R = a.rec_cnt[j];
-    const int count = a.cnt_in[j];
-    const float* src = a.psum + (long)a.rec_off[j] * a.ld + c4;
-    if (done != 0) return;  // tested once the loads above are in flight
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    if (c4 < a.ld) {  // ld is a multiple of 4: the float4 is in or out
-        for (int r = rs; r < R; r += 8) {
-            const float4 v = *reinterpret_cast<const float4*>(src + (long)r * a.ld);
-            s0 += (double)v.x;
-            s1 += (double)v.y;
-            s2 += (double)v.z;
-            s3 += (double)v.w;
-        }
-    }
-    for (int off = 8; off < 64; off <<= 1) {
-        s0 += __shfl_xor(s0, off, 64);
-        s1 += __shfl_xor(s1, off, 64);
-        s2 += __shfl_xor(s2, off, 64);
-        s3 += __shfl_xor(s3, off, 64);
-    }
-    // lane c < 32 takes column 32 cc + c: component c % 4 of lane c / 4
-    const int e = lane & 3, src_lane = (lane >> 2) & 7;
-    const double t0 = __shfl(s0, src_lane, 64), t1 = __shfl(s1, src_lane, 64);
-    const double t2 = __shfl(s2, src_lane, 64), t3 = __shfl(s3, src_lane, 64);
-    const double tot = e == 0 ? t0 : e == 1 ? t1 : e == 2 ? t2 : t3;
+    const int lane = threadIdx.x & 63, col = cc * 32 + lane;
     double sq = 0.0, nrm = 0.0;
-    if (lane < 32 && ccol < a.d) {
-        a.sums[(long)j * a.ld + ccol] = tot;
+    if (lane < 32 && col < a.d) {
+        a.sums[(long)j * a.ld + col] = tot;
         if (count > 0) {
             const float cn = (float)(tot / (double)count);
-            a.C_new[(long)j * a.ld + ccol] = cn;
+            a.C_new[(long)j * a.ld + col] = cn;
             const double df = (double)cn - (double)c_old;
             sq = df * df;
             nrm = (double)cn * (double)cn;
         }
     }
-    sq = wave_sum(sq);
-    nrm = wave_sum(nrm);
-    if (lane == 0) {
-        a.part[((long)j * nch + cc) * 2 + 0] = sq;
-        a.part[((long)j * nch + cc) * 2 + 1] = nrm;
-        if (cc == 0) a.counts[j] = count;
-        if (cc == 0 && count == 0) atomicAdd(&a.state->empty_cnt[a.iter & 1], 1);  // for k_reloc
-        if (j == 0 && cc == 0) {
+    // one butterfly for both (they bound the kernel at 768 floats a row): the
+    // upper half of the wave, which has no columns, takes ||c||^2
+    const double up = __shfl_xor(nrm, 32, 64);
+    double v = lane < 32 ? sq : up;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) v += __shfl_xor(v, off, 64);
+    *sq_out = v;                       // lanes 0..31
+    *nrm_out = v;                      // lanes 32..63
+}
+
+// Record mode (the sorted update: a cluster has a record per chunk of sorted
+// rows it touches, usually one or two): a block per cluster, its 32-column
+// chunks dealt to the four waves.  Lane (rs, q) = (lane / 8, lane % 8) adds
+// the float4 of columns 32 cc + 4q of records rs, rs + 8, .. in fp64, and the
+// eight rs lanes are combined by an xor butterfly.  A cluster of more than 64
+// records (a hot one: 280,000 of 2M rows make 1,083) has all 32 groups of
+// eight lanes on one chunk, eight records a lane in flight.  The cluster's
+// shift^2 and ||c||^2 are folded here, in chunk order.  Bound by the records'
+// round trip and, for long rows, by the shuffles.  A wave per (cluster, chunk)
+// and the fold in one block's loop decision took 71 + 6 us a step at 2M x 64
+// with 1,024 Zipf-sized clusters and 33 + 36 us at 2,048 clusters of 768
+// floats; now 19 and 32, with 5 to 7 for the decision.
+__global__ __launch_bounds__(256) void k_finalize_recs(FinalizeArgs a, int nch)
+{
+    constexpr int kFold = 64;
+    __shared__ double red[4][8][4];
+    __shared__ double fold[2][kFold];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int j = blockIdx.x;
+    const int done = a.state->done;
+    const int q = lane & 7;
+    const int R = a.rec_cnt[j];
+    const int count = a.cnt_in[j];
+    const float* const src = a.psum + (long)a.rec_off[j] * a.ld;
+    if (done != 0) return;  // tested once the loads above are in flight
+    // lane c < 32 of a chunk takes column 32 cc + c: component c % 4 of lane c / 4
+    const int e = lane & 3, src_lane = (lane >> 2) & 7;
+    constexpr int NR = 8;  // records a lane in flight
+    double s[4];
+    auto sums = [&](int cc, int rs, int step) {
+        const int c4 = cc * 32 + 4 * q;  // ld is a multiple of 4: the float4 is in or out
+#pragma unroll
+        for (int x = 0; x < 4; ++x) s[x] = 0.0;
+        if (c4 < a.ld) {
+            for (int r0 = rs; r0 < R; r0 += step * NR) {
+                float4 v[NR];
+#pragma unroll
+                for (int x = 0; x < NR; ++x)
+                    if (r0 + step * x < R) v[x] = *reinterpret_cast<const float4*>(src + (long)(r0 + step * x) * a.ld + c4);
+#pragma unroll
+                for (int x = 0; x < NR; ++x) {
+                    if (r0 + step * x < R) {
+                        s[0] += (double)v[x].x;
+                        s[1] += (double)v[x].y;
+                        s[2] += (double)v[x].z;
+                        s[3] += (double)v[x].w;
+                    }
+                }
+            }
+        }
+        // (lanes past the records hold zeros)
+        for (int off = 8; off < 64 && off < 8 * R; off <<= 1) {
+#pragma unroll
+            for (int x = 0; x < 4; ++x) s[x] += __shfl_xor(s[x], off, 64);
+        }
+    };
+    auto put = [&](int cc, double sq, double nrm) {
+        const int x = lane >> 5;
+        if ((lane & 31) == 0)
+            *(nch <= kFold ? &fold[x][cc] : &a.part[((long)j * nch + cc) * 2 + x]) = x == 0 ? sq : nrm;
+    };
+    if (R <= 64) {
+        for (int cc = w; cc < nch; cc += 4) {
+            const int col = cc * 32 + lane;
+            const float c_old = lane < 32 && col < a.d ? a.C_old[(long)j * a.ld + col] : 0.f;
+            sums(cc, lane >> 3, 8);
+            const double t0 = __shfl(s[0], src_lane, 64), t1 = __shfl(s[1], src_lane, 64);
+            const double t2 = __shfl(s[2], src_lane, 64), t3 = __shfl(s[3], src_lane, 64);
+            double sq, nrm;
+            finalize_chunk(a, j, cc, count, e == 0 ? t0 : e == 1 ? t1 : e == 2 ? t2 : t3, c_old, &sq, &nrm);
+            put(cc, sq, nrm);
+        }
+    } else {
+        for (int cc = 0; cc < nch; ++cc) {
+            sums(cc, threadIdx.x >> 3, 32);
+            if (lane < 8) {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) red[w][lane][x] = s[x];
+            }
+            __syncthreads();
+            if (w == 0) {
+                const int col = cc * 32 + lane;
+                const float c_old = lane < 32 && col < a.d ? a.C_old[(long)j * a.ld + col] : 0.f;
+                const double tot = ((red[0][src_lane][e] + red[1][src_lane][e]) + red[2][src_lane][e]) + red[3][src_lane][e];
+                double sq, nrm;
+                finalize_chunk(a, j, cc, count, tot, c_old, &sq, &nrm);
+                put(cc, sq, nrm);
+            }
+            __syncthreads();
+        }
+    }
+    __threadfence_block();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double tsq = 0.0, tnr = 0.0;
+        for (int c = 0; c < nch; ++c) {
+            tsq += nch <= kFold ? fold[0][c] : a.part[((long)j * nch + c) * 2 + 0];
+            tnr += nch <= kFold ? fold[1][c] : a.part[((long)j * nch + c) * 2 + 1];
+        }
+        a.shift_sq[j] = (float)tsq;
+        if (count > 0) a.cnorm[j] = (float)tnr;
+        a.counts[j] = count;
+        if (count == 0) atomicAdd(&a.state->empty_cnt[a.iter & 1], 1);  // for k_reloc
+        if (j == 0) {
             if (a.chg_next != nullptr) *a.chg_next = 0;
             a.state->empty_cnt[(a.iter + 1) & 1] = 0;  // read by k_reloc of iteration iter - 1, which has run
         }
     }
 }
 
-__global__ __launch_bounds__(256) void k_finalize_loop(FinalizeArgs a, int nch)
+// The loop's stopping rules (_kmeans.py:717-732), by a block of 256 threads.
+// nch > 0: every cluster's shift^2 and ||c||^2 from its chunk partials, in
+// chunk order; 0: its shift^2 is in shift_sq already.
+__device__ __forceinline__ void loop_decision(const FinalizeArgs& a, int nch)
 {
     LoopState* st = a.state;
-    if (st->done != 0) return;
     const int tid = threadIdx.x;
     __shared__ double shd[4];
     __shared__ int shi[4];
@@ -1106,17 +1178,23 @@ __global__ __launch_bounds__(256) void k_finalize_loop(FinalizeArgs a, int nch)
     double tot = 0.0;
     float mx = 0.f;
     for (int j = tid; j < a.k; j += 256) {
-        double tsq = 0.0, tnr = 0.0;
-        for (int c = 0; c < nch; ++c) {
-            tsq += a.part[((long)j * nch + c) * 2 + 0];
-            tnr += a.part[((long)j * nch + c) * 2 + 1];
-        }
         const int count = a.counts[j];
-        a.shift_sq[j] = (float)tsq;
-        if (count > 0 || a.after_reloc) a.cnorm[j] = (float)tnr;
+        float shift;
+        if (nch > 0) {
+            double tsq = 0.0, tnr = 0.0;
+            for (int c = 0; c < nch; ++c) {
+                tsq += a.part[((long)j * nch + c) * 2 + 0];
+                tnr += a.part[((long)j * nch + c) * 2 + 1];
+            }
+            shift = (float)tsq;
+            a.shift_sq[j] = shift;
+            if (count > 0 || a.after_reloc) a.cnorm[j] = (float)tnr;
+        } else {
+            shift = a.shift_sq[j];
+        }
         n_empty += count == 0;
-        tot += (double)(float)tsq;
-        mx = fmaxf(mx, (float)tsq);
+        tot += (double)shift;
+        mx = fmaxf(mx, shift);
     }
     n_empty = block_sum(n_empty, shi);
     tot = block_sum(tot, shd);
@@ -1143,11 +1221,17 @@ __global__ __launch_bounds__(256) void k_finalize_loop(FinalizeArgs a, int nch)
     }
 }
 
+__global__ __launch_bounds__(256) void k_finalize_loop(FinalizeArgs a, int nch)
+{
+    if (a.state->done != 0) return;
+    loop_decision(a, nch);
+}
+
 hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t s, bool with_loop)
 {
     const int nch = finalize_col_chunks(a.d, a.R);
     if (a.rec_off != nullptr)
-        hipLaunchKernelGGL(k_finalize_recs, dim3((unsigned)(((long)a.k * nch + 3) / 4)), dim3(256), 0, s, a, nch);
+        hipLaunchKernelGGL(k_finalize_recs, dim3((unsigned)a.k), dim3(256), 0, s, a, nch);
     else
         hipLaunchKernelGGL(k_finalize_cols, dim3(a.k, nch), dim3(256), 0, s, a);
     const hipError_t e = hipGetLastError();
@@ -1157,7 +1241,9 @@ hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t s, bool with_loop)
 
 hipError_t launch_finalize_loop(const FinalizeArgs& a, hipStream_t s, int nch)
 {
-    hipLaunchKernelGGL(k_finalize_loop, dim3(1), dim3(256), 0, s, a, nch > 0 ? nch : finalize_col_chunks(a.d, a.R));
+    // (record mode: k_finalize_recs has folded the chunks)
+    if (nch == 0 && a.rec_off == nullptr) nch = finalize_col_chunks(a.d, a.R);
+    hipLaunchKernelGGL(k_finalize_loop, dim3(1), dim3(256), 0, s, a, nch);
     return hipGetLastError();
 }
 
@@ -1830,8 +1916,9 @@ constexpr int kRelocCand = 256;  // candidate rows per block, at most (one per t
 
 // The relocation of E (1..kMaxReloc) empty clusters by every block of the
 // grid (gridDim.x <= kRelocCandBlocks): phases A, B and C above.
+// Returns true in the last block, which has moved the rows.
 template <int LDM, bool CL>
-__device__ __forceinline__ void reloc_body(const InRelocArgs& a, int E)
+__device__ __forceinline__ bool reloc_body(const InRelocArgs& a, int E)
 {
     using RG = RelocGeom<LDM, CL>;
     __shared__ __attribute__((aligned(16))) float tiles[4 * RG::TF];
@@ -2010,7 +2097,7 @@ __device__ __forceinline__ void reloc_body(const InRelocArgs& a, int E)
         last_s = __hip_atomic_fetch_add(&st->reloc_ctr, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) ==
                  gridDim.x - 1;
     __syncthreads();
-    if (!last_s) return;
+    if (!last_s) return false;
     if (tid == 0) {
         st->reloc_ctr = 0u;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // every block's stores
@@ -2191,17 +2278,42 @@ __device__ __forceinline__ void reloc_body(const InRelocArgs& a, int E)
             a.part[((long)j * a.nch + cc) * 2 + 1] = nrm;
         }
     }
+    if (a.fold_shift != nullptr) {
+        // record mode: the clusters' shift^2 and ||c||^2 folded again
+        __threadfence_block();
+        __syncthreads();
+        for (int q = tid; q < nitems; q += 256) {
+            const int j = q < nm ? empt[q] : q < 2 * nm ? donor[q - nm] : still[q - 2 * nm];
+            double tsq = 0.0, tnr = 0.0;
+            for (int c = 0; c < a.nch; ++c) {
+                tsq += a.part[((long)j * a.nch + c) * 2 + 0];
+                tnr += a.part[((long)j * a.nch + c) * 2 + 1];
+            }
+            a.fold_shift[j] = (float)tsq;
+            if (a.counts[j] > 0) a.fold_cnorm[j] = (float)tnr;
+        }
+    }
     if (tid == 0) st->reloc_iter = a.iter;
+    return true;
 }
 
-// After k_finalize_cols: the clusters it counted empty.
+// After k_finalize_recs or k_finalize_cols: the clusters it counted empty are
+// relocated, and the last block to touch them (block 0 when there are none,
+// or more than k_reloc takes) makes the step's loop decision: one launch (a
+// launch that finds nothing to do costs 4 to 5 us).
 template <int LDM>
-__global__ __launch_bounds__(256) void k_reloc(InRelocArgs a)
+__global__ __launch_bounds__(256) void k_reloc(InRelocArgs a, FinalizeArgs f, int nch, int decide)
 {
     if (a.state->done != 0) return;
     const int E = a.state->empty_cnt[a.iter & 1];
-    if (E == 0 || E > kMaxReloc) return;
-    reloc_body<LDM, false>(a, E);
+    if (E == 0 || E > kMaxReloc) {
+        if (decide && blockIdx.x == 0) loop_decision(f, nch);
+        return;
+    }
+    if (!reloc_body<LDM, false>(a, E) || !decide) return;
+    __threadfence_block();
+    __syncthreads();
+    loop_decision(f, nch);
 }
 
 // The fused step's finalize and relocation in one launch.  The F = k nch
@@ -2246,15 +2358,16 @@ hipError_t launch_finalize_reloc(const FinalizeArgs& f, const InRelocArgs& a, hi
     return hipGetLastError();
 }
 
-hipError_t launch_reloc_inline(const InRelocArgs& a, hipStream_t s)
+hipError_t launch_reloc_inline(const InRelocArgs& a, const FinalizeArgs& f, int decide, hipStream_t s)
 {
     const dim3 g(kRelocInlineBlocks);
+    const int nch = f.rec_off != nullptr ? 0 : a.nch;
     switch (row_path(a.ld)) {
-    case 32: hipLaunchKernelGGL(k_reloc<32>, g, dim3(256), 0, s, a); break;
-    case 64: hipLaunchKernelGGL(k_reloc<64>, g, dim3(256), 0, s, a); break;
-    case 104: hipLaunchKernelGGL(k_reloc<104>, g, dim3(256), 0, s, a); break;
-    case 128: hipLaunchKernelGGL(k_reloc<128>, g, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL(k_reloc<0>, g, dim3(256), 0, s, a); break;
+    case 32: hipLaunchKernelGGL(k_reloc<32>, g, dim3(256), 0, s, a, f, nch, decide); break;
+    case 64: hipLaunchKernelGGL(k_reloc<64>, g, dim3(256), 0, s, a, f, nch, decide); break;
+    case 104: hipLaunchKernelGGL(k_reloc<104>, g, dim3(256), 0, s, a, f, nch, decide); break;
+    case 128: hipLaunchKernelGGL(k_reloc<128>, g, dim3(256), 0, s, a, f, nch, decide); break;
+    default: hipLaunchKernelGGL(k_reloc<0>, g, dim3(256), 0, s, a, f, nch, decide); break;
     }
     return hipGetLastError();
 }
@@ -2351,43 +2464,62 @@ hipError_t launch_colmean(const double* part, int nblk, long n, int d, float* me
     return hipGetLastError();
 }
 
-__global__ void k_center(float* __restrict__ X, long n, int ld, int d, const float* __restrict__ mean)
+// One pass over X at load: the column mean taken off (mean nullable, its pad
+// columns 0), the largest |x| (NaN counts as +inf) into *out as float bits, and
+// ||x||^2 per row in fp32 (norm nullable; the relocation's approximate
+// distances, whose candidate margin covers its rounding).  G lanes a row, a
+// float4 each at a time, so that a wave's loads are consecutive; U rows a
+// lane group in flight.  Three kernels took 65, 38 and 161 us at 500,000 x 100
+// (the norms a thread per row: 64 cache lines a load); this one 73 (5.5 TB/s).
+template <int G>
+__global__ __launch_bounds__(256) void k_load_pass(float* __restrict__ X, long n, int ld,
+                                                   const float* __restrict__ mean, unsigned* out,
+                                                   float* __restrict__ norm)
 {
-    const long total = n * (long)ld;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
-        const int c = (int)(i % ld);
-        if (c < d) X[i] = X[i] - mean[c];
-    }
-}
-
-hipError_t launch_center(float* X, long n, int ld, int d, const float* mean, hipStream_t s)
-{
-    const long total = n * (long)ld;
-    long blocks = (total + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_center, dim3((unsigned)blocks), dim3(256), 0, s, X, n, ld, d, mean);
-    return hipGetLastError();
-}
-
-// Largest |x| over `count` floats (NaN counts as +inf) into *out as float
-// bits: non-negative floats order like their bit patterns, so an unsigned
-// atomic max per wave combines them.
-__global__ __launch_bounds__(256) void k_absmax(const float* __restrict__ X, long count, unsigned* out)
-{
+    constexpr int RB = 256 / G;  // rows per block at a time
+    constexpr int U = 4;
+    const int g = threadIdx.x / G, q0 = threadIdx.x % G;
+    const int nq = ld >> 2;
     float m = 0.f;
-    const long stride = (long)gridDim.x * 256;
-    const long c4 = count >> 2;  // 16-byte loads over the multiple-of-4 part
-    const float4* X4 = reinterpret_cast<const float4*>(X);
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < c4; i += stride) {
-        const float4 v4 = X4[i];
-        const float e[4] = {fabsf(v4.x), fabsf(v4.y), fabsf(v4.z), fabsf(v4.w)};
+    for (long r0 = (long)blockIdx.x * (RB * U) + g; r0 < n; r0 += (long)gridDim.x * (RB * U)) {
+        float s[U];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) m = e[u] != e[u] ? INFINITY : fmaxf(m, e[u]);
-    }
-    for (long i = 4 * c4 + (long)blockIdx.x * 256 + threadIdx.x; i < count; i += stride) {
-        const float v = fabsf(X[i]);
-        m = v != v ? INFINITY : fmaxf(m, v);
+        for (int u = 0; u < U; ++u) s[u] = 0.f;
+        for (int q = q0; q < nq; q += G) {
+            f4v v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const long r = min(r0 + (long)u * RB, n - 1);
+                v[u] = *reinterpret_cast<const f4v*>(X + r * ld + 4 * q);
+            }
+            if (mean != nullptr) {
+                const f4v mu = *reinterpret_cast<const f4v*>(mean + 4 * q);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const long r = r0 + (long)u * RB;
+                    v[u] = v[u] - mu;
+                    if (r < n) *reinterpret_cast<f4v*>(X + r * ld + 4 * q) = v[u];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (r0 + (long)u * RB >= n) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float x = fabsf(v[u][e]);
+                    m = x != x ? INFINITY : fmaxf(m, x);
+                    s[u] = fmaf(x, x, s[u]);
+                }
+            }
+        }
+        if (norm != nullptr) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+#pragma unroll
+                for (int off = 1; off < G; off <<= 1) s[u] += __shfl_xor(s[u], off, 64);
+                if (q0 == 0 && r0 + (long)u * RB < n) norm[r0 + (long)u * RB] = s[u];
+            }
+        }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
@@ -2397,60 +2529,53 @@ __global__ __launch_bounds__(256) void k_absmax(const float* __restrict__ X, lon
     if (threadIdx.x == 0) atomicMax(out, __float_as_uint(fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]))));
 }
 
-hipError_t launch_absmax(const float* X, long count, unsigned* out, hipStream_t s)
+hipError_t launch_load_pass(float* X, long n, int ld, const float* mean, unsigned* out, float* norm, hipStream_t s)
 {
     const hipError_t e = hipMemsetAsync(out, 0, sizeof(unsigned), s);
     if (e != hipSuccess) return e;
-    long blocks = (count / 4 + 255) / 256;
-    if (blocks > 1024) blocks = 1024;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_absmax, dim3((unsigned)blocks), dim3(256), 0, s, X, count, out);
-    return hipGetLastError();
-}
-
-// ||x_r||^2 in fp32, one thread per row (the relocation's approximate
-// distances; their candidate margin covers its rounding).
-__global__ __launch_bounds__(256) void k_rownorm(const float* __restrict__ X, long n, int ld, int d,
-                                                 float* __restrict__ out)
-{
-    const long r = (long)blockIdx.x * 256 + threadIdx.x;
-    if (r >= n) return;
-    const float4* x4 = reinterpret_cast<const float4*>(X + r * ld);
-    float s = 0.f;
-    const int nfull = d >> 2;
-    for (int g = 0; g < nfull; ++g) {
-        const float4 v = x4[g];
-        s = fmaf(v.x, v.x, s);
-        s = fmaf(v.y, v.y, s);
-        s = fmaf(v.z, v.z, s);
-        s = fmaf(v.w, v.w, s);
+    const int nq = ld / 4;
+    const int G = nq <= 1 ? 1 : nq <= 2 ? 2 : nq <= 4 ? 4 : nq <= 8 ? 8 : nq <= 16 ? 16 : nq <= 32 ? 32 : 64;
+    const long rows = 256 / G * 4;
+    const long blocks = max(1L, min(4096L, (n + rows - 1) / rows));
+    const dim3 g((unsigned)blocks), b(256);
+    switch (G) {
+    case 1: hipLaunchKernelGGL(k_load_pass<1>, g, b, 0, s, X, n, ld, mean, out, norm); break;
+    case 2: hipLaunchKernelGGL(k_load_pass<2>, g, b, 0, s, X, n, ld, mean, out, norm); break;
+    case 4: hipLaunchKernelGGL(k_load_pass<4>, g, b, 0, s, X, n, ld, mean, out, norm); break;
+    case 8: hipLaunchKernelGGL(k_load_pass<8>, g, b, 0, s, X, n, ld, mean, out, norm); break;
+    case 16: hipLaunchKernelGGL(k_load_pass<16>, g, b, 0, s, X, n, ld, mean, out, norm); break;
+    case 32: hipLaunchKernelGGL(k_load_pass<32>, g, b, 0, s, X, n, ld, mean, out, norm); break;
+    default: hipLaunchKernelGGL(k_load_pass<64>, g, b, 0, s, X, n, ld, mean, out, norm); break;
     }
-    for (int c = 4 * nfull; c < d; ++c) s = fmaf(X[r * ld + c], X[r * ld + c], s);
-    out[r] = s;
-}
-
-hipError_t launch_rownorm(const float* X, long n, int ld, int d, float* out, hipStream_t s)
-{
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rownorm, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, X, n, ld, d, out);
     return hipGetLastError();
 }
 
-__global__ void k_cnorm(const float* __restrict__ C, int k, int ld, float* __restrict__ cnorm)
+// Centres given by the caller: their mean taken off (mean nullable) and
+// ||c||^2, fp64 sums over the lanes of a wave per centre.  (One thread per
+// centre over its floats one by one took 12 us at 50 x 100 and 105 us at
+// 2,048 x 768; now 3 to 6.)
+__global__ __launch_bounds__(256) void k_cnorm(float* __restrict__ C, int k, int ld, int d,
+                                               const float* __restrict__ mean, float* __restrict__ cnorm)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = (int)blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (j >= k) return;
+    float* const row = C + (long)j * ld;
     double s = 0.0;
-    for (int c = 0; c < ld; ++c) {
-        const double v = (double)C[(long)j * ld + c];
-        s += v * v;
+    for (int c = lane; c < ld; c += 64) {
+        float v = row[c];
+        if (mean != nullptr && c < d) {
+            v = v - mean[c];
+            row[c] = v;
+        }
+        s += (double)v * (double)v;
     }
-    cnorm[j] = (float)s;
+    s = wave_sum(s);
+    if (lane == 0) cnorm[j] = (float)s;
 }
 
-hipError_t launch_cnorm(const float* C, int k, int ld, float* cnorm, hipStream_t s)
+hipError_t launch_cnorm(float* C, int k, int ld, int d, const float* mean, float* cnorm, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_cnorm, dim3((k + 255) / 256), dim3(256), 0, s, C, k, ld, cnorm);
+    hipLaunchKernelGGL(k_cnorm, dim3((k + 3) / 4), dim3(256), 0, s, C, k, ld, d, mean, cnorm);
     return hipGetLastError();
 }
 

@@ -522,7 +522,7 @@ struct Lloyd {
             TRY(measure_xmax());
             split_on = split_range_ok(xmax);
         }
-        HIP_TRY(launch_cnorm(cen[0], k, ld, cnorm, s), "cnorm launch");
+        HIP_TRY(launch_cnorm(cen[0], k, ld, d, nullptr, cnorm, s), "cnorm launch");
         return 0;
     }
 
@@ -620,11 +620,14 @@ struct Lloyd {
             const int nb = colsum_grid(n);
             HIP_TRY(launch_colsum(X, n, ld, d, colpart, nb, s), "colsum launch");
             HIP_TRY(launch_colmean(colpart, nb, n, d, mean, s), "colmean launch");
-            HIP_TRY(launch_center(X, n, ld, d, mean, s), "center launch");
+            HIP_TRY(launch_load_pass(X, n, ld, mean, absmax, xnorm, s), "load pass launch");
+            absmax_set = true;
             TRY(download_bytes(*C, mean, size_t(d) * sizeof(float), h_mean.data(), s));
         } else {
             std::fill(h_mean.begin(), h_mean.end(), 0.f);
             HIP_TRY(hipMemsetAsync(mean, 0, size_t(ld) * sizeof(float), s), "hipMemsetAsync");
+            absmax_set = f3cap || a3cap || xnorm != nullptr;
+            if (absmax_set) HIP_TRY(launch_load_pass(X, n, ld, nullptr, absmax, xnorm, s), "load pass launch");
         }
         xmax_known = false;
         split_on = false;
@@ -632,16 +635,17 @@ struct Lloyd {
             TRY(measure_xmax());
             split_on = split_range_ok(xmax);
         }
-        if (xnorm != nullptr) HIP_TRY(launch_rownorm(X, n, ld, d, xnorm, s), "rownorm launch");
         return 0;
     }
 
     // max |x| of the loaded X (NaN counted as +inf) into xmax
     bool xmax_known = false;
+    bool absmax_set = false;  // the load pass left it in absmax
     int measure_xmax()
     {
+        if (!absmax_set) HIP_TRY(launch_load_pass(X, n, ld, nullptr, absmax, nullptr, s), "load pass launch");
+        absmax_set = true;
         unsigned bits = 0;
-        HIP_TRY(launch_absmax(X, n * (long)ld, absmax, s), "absmax launch");
         TRY(download_bytes(*C, absmax, sizeof(unsigned), &bits, s));
         std::memcpy(&xmax, &bits, sizeof(float));
         xmax_known = true;
@@ -652,8 +656,7 @@ struct Lloyd {
     int set_centers(const float* host)
     {
         TRY(upload_rows(*C, host, k, d, ld, cen[cur], s));
-        if (centred) HIP_TRY(launch_center(cen[cur], k, ld, d, mean, s), "center launch");
-        HIP_TRY(launch_cnorm(cen[cur], k, ld, cnorm, s), "cnorm launch");
+        HIP_TRY(launch_cnorm(cen[cur], k, ld, d, centred ? mean : nullptr, cnorm, s), "cnorm launch");
         return 0;
     }
 
@@ -832,9 +835,15 @@ struct Lloyd {
             HIP_TRY(launch_finalize_reloc(f, r, s), "finalize launch");
         } else {
             HIP_TRY(launch_finalize(f, s, false), "finalize launch");
-            if (reloc_inline) HIP_TRY(launch_reloc_inline(r, s), "relocation launch");
+            if (reloc_inline) {
+                if (f.rec_off != nullptr) {
+                    r.fold_shift = shift_sq;
+                    r.fold_cnorm = cnorm;
+                }
+                HIP_TRY(launch_reloc_inline(r, f, fblocks == 0, s), "relocation launch");
+            }
         }
-        if (fblocks == 0 || last) HIP_TRY(launch_finalize_loop(f, s), "finalize launch");
+        if (fblocks == 0 ? !reloc_inline : last) HIP_TRY(launch_finalize_loop(f, s), "finalize launch");
         if (ev) HIP_TRY(hipEventRecord(ev[3], s), "hipEventRecord");
         cur ^= 1;
         return 0;
@@ -1115,7 +1124,7 @@ struct Lloyd {
             HIP_TRY(launch_pp_dist(pp, c, s), "pp dist launch");
         }
         HIP_TRY(launch_pp_select(pp, k, s), "pp select launch");
-        HIP_TRY(launch_cnorm(cen[cur], k, ld, cnorm, s), "cnorm launch");
+        HIP_TRY(launch_cnorm(cen[cur], k, ld, d, nullptr, cnorm, s), "cnorm launch");
         TRY(download_bytes(*C, pp.idx, size_t(k) * sizeof(long), idx_out, s));
         return 0;
     }
