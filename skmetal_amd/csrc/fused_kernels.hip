@@ -6,6 +6,8 @@
 //   k_fused     E-step on fp32 MFMA, per-cluster sums by a VALU walker; 8
 //               waves per block (d <= 16, data outside the split's range of
 //               split_kernels.hip's k_fused3, or the fp32 switch).
+//   k_fused_low E-step and sums on the VALU, every wave by itself (d <= 16,
+//               few centres or many rows: low_takes).
 //
 // The fused kernels are used when k <= 64 and d <= 100; X's row stride ld is
 // then padded (with zeros) to 4*NQ floats for one of the compiled NQ, so the
@@ -362,7 +364,255 @@ __global__ __launch_bounds__(512, 1) void k_fused(FusedArgs a)
     combine_sums<CPC>(zrow + XS, ld, k, psum, pcnt, sCnt, tid, &st->present[a.iter & 1]);
 }
 
+// ---------------------------------------------------------------------------
+// k_fused_low: rows of at most 16 floats
+// ---------------------------------------------------------------------------
+//
+// Short rows leave little arithmetic per row, and k_fused's round (load, E-step,
+// argmin, hand-over to the walker) is latency with two waves a SIMD: 33 us at
+// 1M x 3, k = 64 and 71 us at 1M x 16, k = 20, for 16 and 64 MB.  Here every
+// wave works alone, four a SIMD, with no hand-over: 64 R rows at a time, R
+// rows a lane, the next ones in flight.  The E-step runs on the VALU (x.c as
+// the fma chain over the features that the fp32 MFMAs make, then ||c||^2 - 2
+// x.c and a strict '<' scan), the centres read from LDS as broadcasts, once
+// per R rows (at R = 1 those reads take as long as the arithmetic).  The sums:
+// per 64 rows an LDS bit mask of each cluster's rows; lane (cluster c, slice
+// s) of 64 / KP slices (KP = k rounded up to a power of two) walks the slice's
+// rows of c in ascending order.  Slices meet by an xor butterfly, waves in
+// order: bitwise reproducible.  Bound by the VALU (k = 64) or HBM (k <= 8).
+// LDS: centres [64][4 NQ] | per wave: rows [65][4 NQ] (the last one zeros), masks [64]
+template <int NQ>
+constexpr size_t low_wave_bytes()
+{
+    return 65 * 16 * NQ + 64 * sizeof(unsigned long long);
+}
+
+template <int NQ, int R>
+__global__ __launch_bounds__(1024) void k_fused_low(FusedArgs a)
+{
+    constexpr int LD = 4 * NQ;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ __attribute__((aligned(16))) float sN[64];
+    __shared__ int sCnt[16][64];
+    __shared__ int sDone, sChg;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = (int)(blockDim.x >> 6);
+    const int k = a.k;
+    const long n = a.n;
+    float* const sC = lds;
+    char* const mine = reinterpret_cast<char*>(lds + 64 * LD) + wave * low_wave_bytes<NQ>();
+    f4v* const tile = reinterpret_cast<f4v*>(mine);
+    unsigned long long* const mask = reinterpret_cast<unsigned long long*>(mine + 65 * 16 * NQ);
+    // this wave's chunks of 64 R rows: c0, c0 + cstep, ..
+    const long cstep = (long)gridDim.x * nw * (64 * R);
+    long c0 = ((long)blockIdx.x * nw + wave) * (64 * R);
+    f4v x[R][NQ], xn[R][NQ];
+    int old[R], oldn[R];
+    auto load = [&](long c) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const long row = min(c + 64 * r + lane, n - 1);
+            const f4v* p = reinterpret_cast<const f4v*>(a.X + row * LD);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) xn[r][q] = p[q];
+            oldn[r] = a.labels[row];
+        }
+    };
+    if (c0 < n) load(c0);
+    // centres (zeros past k: their norms are +inf), the zero row, norms and
+    // the previous step's decision
+    for (int i = tid; i < 64 * NQ; i += (int)blockDim.x) {
+        const int j = i / NQ;
+        f4v v = {0.f, 0.f, 0.f, 0.f};
+        if (j < k) v = *reinterpret_cast<const f4v*>(a.C + (long)i * 4);
+        *reinterpret_cast<f4v*>(sC + 4 * i) = v;
+    }
+    if (lane < NQ) tile[64 * NQ + lane] = f4v{0.f, 0.f, 0.f, 0.f};
+    if (wave == 0) {
+        const int prev = a.state->done;  // an earlier step halted the loop
+        if (prev != 0) {
+            if (lane == 0) sDone = prev;
+        } else {
+            step_norms<64>(a, lane, sN, &sDone);
+        }
+        if (lane == 0) sChg = 0;
+    }
+    __syncthreads();
+    if (sDone != 0) return;
+    int lk = 0;
+    while ((1 << lk) < k) ++lk;
+    const int KP = 1 << lk;
+    const int c = lane & (KP - 1), sl = lane >> lk;
+    const unsigned long long smask = KP == 64 ? ~0ull : (1ull << KP) - 1ull;  // a slice is KP rows
+    f4v S[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) S[q] = f4v{0.f, 0.f, 0.f, 0.f};
+    int cnt = 0, changed = 0;
+    const int k4 = (k + 3) & ~3;
+    for (; c0 < n; c0 += cstep) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) x[r][q] = xn[r][q];
+            old[r] = oldn[r];
+        }
+        if (c0 + cstep < n) load(c0 + cstep);  // in flight while this chunk is worked on
+        float best[R];
+        int bi[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            best[r] = INFINITY;
+            bi[r] = 0;
+        }
+        for (int j = 0; j < k4; j += 4) {
+            const f4v cn = *reinterpret_cast<const f4v*>(sN + j);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                f4v cv[NQ];
+#pragma unroll
+                for (int q = 0; q < NQ; ++q) cv[q] = *reinterpret_cast<const f4v*>(sC + (j + u) * LD + 4 * q);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    float acc = 0.f;
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc = fmaf(x[r][q][e], cv[q][e], acc);
+                    }
+                    const float d = fmaf(-2.0f, acc, cn[u]);  // NaN compares false
+                    const bool take = d < best[r];
+                    best[r] = take ? d : best[r];
+                    bi[r] = take ? j + u : bi[r];
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const long row = c0 + 64 * r + lane;
+            const bool valid = row < n;
+            if (valid) a.labels[row] = bi[r];
+            changed += (int)__popcll(__ballot(valid && old[r] != bi[r]));
+            // the 64 rows to LDS and the masks of each cluster's rows (a
+            // wave's LDS accesses are performed in order)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) tile[lane * NQ + q] = x[r][q];
+            if (lane < KP) mask[lane] = 0ull;
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_wave_barrier();
+            if (valid) atomicOr(&mask[bi[r]], 1ull << lane);
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_wave_barrier();
+            const int r0 = sl << lk;
+            unsigned long long m = (mask[c] >> r0) & smask;
+            cnt += (int)__popcll(m);
+            while (__ballot(m != 0ull) != 0ull) {
+                // two rows at a time; past the last one the row of zeros
+                int rr[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    rr[u] = m != 0ull ? r0 + __ffsll((long long)m) - 1 : 64;
+                    m &= m - 1ull;
+                }
+                f4v v[2][NQ];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) v[u][q] = tile[rr[u] * NQ + q];
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) S[q] += v[u][q];
+                }
+            }
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    // the slices of a cluster, then the waves in order
+    for (int off = KP; off < 64; off <<= 1) {
+        cnt += __shfl_xor(cnt, off, 64);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S[q][e] += __shfl_xor(S[q][e], off, 64);
+        }
+    }
+    if (lane == 0 && changed != 0) atomicAdd(&sChg, changed);
+    __syncthreads();  // every wave is done with its rows
+    float* const red = lds + 64 * LD;  // [wave][KP][LD]
+    if (lane < KP) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) *reinterpret_cast<f4v*>(red + (wave * KP + lane) * LD + 4 * q) = S[q];
+        sCnt[wave][lane] = cnt;
+    }
+    __syncthreads();
+    if (tid == 0 && sChg != 0) atomicAdd(a.changed, sChg);
+    float* const out = a.psum + (long)blockIdx.x * k * LD;
+    for (int i = tid; i < k * LD; i += (int)blockDim.x) {
+        float t = red[i];
+        for (int w = 1; w < nw; ++w) t += red[w * KP * LD + i];
+        out[i] = t;
+    }
+    if (tid < 64) {
+        int t = 0;
+        if (tid < k) {
+            for (int w = 0; w < nw; ++w) t += sCnt[w][tid];
+            a.pcnt[(long)blockIdx.x * k + tid] = t;
+        }
+        const unsigned long long m = __ballot(t > 0);
+        if (tid == 0 && m != 0ull) atomicOr(&a.state->present[a.iter & 1], m);
+    }
+}
+
 typedef void (*fused_fn)(FusedArgs);
+
+// Whether k_fused_low takes the shape.  Its E-step is k (ld + 3) VALU
+// instructions a row and wave, where k_fused's MFMA wave has the VALU to its
+// argmin: few centres or features, and, while the walkers' rounds are what
+// k_fused waits for, more rows.  Kernel times, k_fused / k_fused_low: 1M x 3:
+// k = 64 33 / 24 us, k = 16 43 / 15, k = 4 28 / 13; 1M x 8: k = 64 39 / 32,
+// k = 20 62 / 20; 1M x 16: k = 64 51 / 52, k = 20 71 / 31, k = 8 39 / 27;
+// 50,000 rows: 3 floats, k = 64 8.1 / 9.7, k = 16 8.8 / 7.8; 8 floats, k = 64
+// 8.3 / 10.7, k = 20 10.0 / 8.6; 16 floats, k = 64 9.6 / 13.0, k = 20 10.6 /
+// 9.7.
+static bool low_takes(long n, int ld, int k)
+{
+    const int ops = k * (ld + 3);
+    return ld <= 16 && (ops <= 400 || (n >= 150000 && ops <= 750));
+}
+
+// Waves a block and rows a lane for n rows: four-wave blocks while every CU
+// has at most one of them (the E-step's VALU time is per wave), else sixteen
+// waves, and two rows a lane (which halve the LDS reads of the centres) once
+// every wave has two tiles of 64.  Four rows a lane were no faster from 1M to
+// 4M rows.
+struct LowShape {
+    int waves, rows;
+};
+static LowShape low_shape(long n, int num_cu)
+{
+    const long tiles = (n + 63) / 64;
+    if (tiles <= 4L * num_cu) return {4, 1};
+    return {16, tiles <= 32L * num_cu ? 1 : 2};
+}
+
+static fused_fn low_kernel(int ld, int rows)
+{
+    switch (ld) {
+    case 4: return rows == 1 ? &k_fused_low<1, 1> : &k_fused_low<1, 2>;
+    case 8: return rows == 1 ? &k_fused_low<2, 1> : &k_fused_low<2, 2>;
+    case 16: return rows == 1 ? &k_fused_low<4, 1> : &k_fused_low<4, 2>;
+    default: return nullptr;
+    }
+}
+
+static size_t low_dyn_lds(int ld, int waves)
+{
+    const size_t per = ld == 4 ? low_wave_bytes<1>() : ld == 8 ? low_wave_bytes<2>() : low_wave_bytes<4>();
+    return 64 * (size_t)ld * sizeof(float) + (size_t)waves * per;
+}
 
 template <int NQ, int... KGs>
 struct FusedTable {
@@ -412,6 +662,16 @@ int fused_ld(int d, int k)
     static const int kLds[] = {4, 8, 16, 32, 48, 64, 80, 100};
     for (int ld : kLds) {
         if (ld < d) continue;
+        if (ld <= 16) {
+            for (const int rows : {1, 2}) {
+                if (hipFuncSetAttribute(reinterpret_cast<const void*>(low_kernel(ld, rows)),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)low_dyn_lds(ld, 16)) !=
+                    hipSuccess) {
+                    (void)hipGetLastError();
+                    return 0;
+                }
+            }
+        }
         fused_fn f = fused_kernel(k, ld);
         const size_t dyn = fused_dyn_lds(k, ld);
         const size_t stat = 4 * 64 * (sizeof(unsigned long long) + sizeof(int)) + 64 * sizeof(float);  // sMask, sCnt, sN
@@ -428,8 +688,13 @@ int fused_ld(int d, int k)
 
 int fused_blocks(long n, int ld, int k, int num_cu)
 {
-    if (fused_kernel(k, ld) == nullptr) return 0;
     const long tiles = (n + 63) / 64;
+    if (low_takes(n, ld, k)) {
+        const LowShape g = low_shape(n, num_cu);
+        const long blocks = (tiles + g.waves * g.rows - 1) / (g.waves * g.rows);
+        return (int)(blocks < 1 ? 1 : blocks < num_cu ? blocks : num_cu);
+    }
+    if (fused_kernel(k, ld) == nullptr) return 0;
     long blocks = (tiles + 3) / 4;
     if (blocks > num_cu) blocks = num_cu;
     return (int)(blocks < 1 ? 1 : blocks);
@@ -438,6 +703,14 @@ int fused_blocks(long n, int ld, int k, int num_cu)
 hipError_t launch_fused(const FusedArgs& a, hipStream_t s)
 {
     if (a.split) return launch_fused3(a, s);
+    if (low_takes(a.n, a.ld, a.k)) {
+        if (a.blocks < 1 || a.k < 1 || a.k > 64) return hipErrorInvalidValue;
+        const LowShape g = low_shape(a.n, a.num_cu);
+        const fused_fn f = low_kernel(a.ld, g.rows);
+        if (f == nullptr) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(f, dim3(a.blocks), dim3(64 * g.waves), low_dyn_lds(a.ld, g.waves), s, a);
+        return hipGetLastError();
+    }
     fused_fn f = fused_kernel(a.k, a.ld);
     if (f == nullptr || a.blocks < 1) return hipErrorInvalidValue;
     hipLaunchKernelGGL(f, dim3(a.blocks), dim3(512), fused_dyn_lds(a.k, a.ld), s, a);

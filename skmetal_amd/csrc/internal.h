@@ -187,6 +187,7 @@ struct FusedArgs {
     // k_fused3, nullable: each row's minimum ||c||^2 - 2 x.c (the distance to
     // its new centre less ||x||^2), for the relocation's candidate search
     float* emin = nullptr;
+    int num_cu = 256;      // compute units of the device (as fused_blocks was given)
 };
 // Row stride (floats) X must have for the fused kernel, or 0 when (d, k) does
 // not qualify; the pad columns are zero.

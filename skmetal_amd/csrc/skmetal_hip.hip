@@ -787,6 +787,7 @@ struct Lloyd {
                     decide ? 1 : 0, iter, tol, flags, part, finalize_col_chunks(d, fblocks), counts,
                     &st->chg[(iter + 1) & 1], cnorm, shift_sq};
         a.split = split_on && f3cap ? 1 : 0;
+        a.num_cu = C->num_cu;
         if (a.split) a.emin = emin;
         HIP_TRY(launch_fused(a, s), "fused launch");
         return 0;
