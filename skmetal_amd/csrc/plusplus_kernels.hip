@@ -572,9 +572,8 @@ __global__ __launch_bounds__(1024) void k_pp_select(PPArgs a, int c)
 {
     constexpr int RPL = kPPRows / 64;  // rows per lane in the row search
     static_assert(kPPRows % 64 == 0, "the row search gives each lane whole rows");
-    constexpr int TB = 8;  // candidates whose partials are summed together
     __shared__ double wsum[16];
-    __shared__ double wpot[16][TB];
+    __shared__ double wpot[16];
     __shared__ double rv[kPPMaxTrials];
     __shared__ int found[kPPMaxTrials];
     __shared__ long picks[kPPMaxTrials];
@@ -583,60 +582,45 @@ __global__ __launch_bounds__(1024) void k_pp_select(PPArgs a, int c)
     const int Tq = c == 1 ? 1 : a.T;
 
     // centre c - 1: the candidate of least potential (first one on ties).
-    // Each potential is a fixed-order sum of the block partials: thread i adds
-    // its blocks (the loads of TB candidates in flight together), then a
-    // butterfly per wave, then the 16 waves in order.  With at most TB
-    // candidates and 2048 blocks, thread i owns blocks [m i, m i + m), the
-    // same blocks as in the running sum below, which then takes the chosen
-    // candidate's values from these registers instead of loading them again;
-    // otherwise thread i adds blocks i, i + 1024, ...
+    // Each potential is a fixed-order sum of the block partials: wave wv adds
+    // share wv / TW of candidate t0 + wv % TW (TW candidates at a time, 16 / TW
+    // waves each; lane l blocks l, l + 64, .. of the share), one butterfly a
+    // wave, then a candidate's waves in order.  (Every thread adding its
+    // blocks of all candidates took eight butterflies in each of the 16 waves,
+    // 1,500 LDS permutes on one CU: 13.7 us a call at 300,000 rows, T = 7, and
+    // 11.8 at 2,000 rows, T = 4; now 9.8 and 7.3.)
     const int m = (a.nb + 1023) / 1024;
     const int b0 = m * tid, b1 = min(a.nb, b0 + m);
-    const bool regs = Tq <= TB && m <= 2;  // block-uniform
-    double pv[TB][2];
-    for (int t0 = 0; t0 < Tq; t0 += TB) {
-        double v[TB];
+    double bestpot = 0.0;
+    int best = 0;
+    for (int t0 = 0; t0 < Tq; t0 += 16) {
+        const int TW = min(16, Tq - t0), ns = 16 / TW;
+        const int t = wv % TW, sh = wv / TW;
+        double v = 0.0;
+        if (sh < ns) {
+            const double* P = a.P[q] + (long)(t0 + t) * a.nb;
+            constexpr int U = 8;
+            for (int b = 64 * sh + lane; b < a.nb; b += 64 * ns * U) {
+                double x[U];
 #pragma unroll
-        for (int t = 0; t < TB; ++t) v[t] = 0.0;
-        if (regs) {
+                for (int u = 0; u < U; ++u) x[u] = b + 64 * ns * u < a.nb ? P[b + 64 * ns * u] : 0.0;
 #pragma unroll
-            for (int t = 0; t < TB; ++t)
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    pv[t][i] = t < Tq && b0 + i < b1 ? a.P[q][(long)t * a.nb + b0 + i] : 0.0;
-#pragma unroll
-            for (int t = 0; t < TB; ++t)
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    if (b0 + i < b1) v[t] += pv[t][i];
-        } else {
-            for (int b = tid; b < a.nb; b += 1024) {
-#pragma unroll
-                for (int t = 0; t < TB; ++t)
-                    if (t0 + t < Tq) v[t] += a.P[q][(long)(t0 + t) * a.nb + b];
+                for (int u = 0; u < U; ++u) v += x[u];
             }
         }
-#pragma unroll
-        for (int t = 0; t < TB; ++t) {
-            const double w = wave_sum(v[t]);
-            if (lane == 0) wpot[wv][t] = w;
-        }
+        v = wave_sum(v);
+        if (lane == 0) wpot[wv] = v;
         __syncthreads();
-        if (tid < TB && t0 + tid < Tq) {
-            double w = 0.0;
-            for (int i = 0; i < 16; ++i) w += wpot[i][tid];
-            rv[t0 + tid] = w;
+        for (int x = 0; x < TW; ++x) {
+            double w = wpot[x];
+            for (int y = 1; y < ns; ++y) w += wpot[x + TW * y];
+            if ((t0 == 0 && x == 0) || w < bestpot) {
+                bestpot = w;
+                best = t0 + x;
+            }
         }
         __syncthreads();
     }
-    double bestpot = rv[0];
-    int best = 0;
-    for (int t = 1; t < Tq; ++t)
-        if (rv[t] < bestpot) {
-            bestpot = rv[t];
-            best = t;
-        }
-    __syncthreads();
     const long crow = a.cand[best];
     if (tid == 0) {
         a.idx[c - 1] = crow;
@@ -657,16 +641,9 @@ __global__ __launch_bounds__(1024) void k_pp_select(PPArgs a, int c)
     // [m i, m i + m); its start is the scan of the thread totals before it.
     // found[t] = the first block whose running sum reaches r_t.
     const double* S = a.P[q] + (long)best * a.nb;
-    double sv0 = 0.0, sv1 = 0.0;  // the register path's values of S[b0], S[b0 + 1]
-    if (regs) {
-#pragma unroll
-        for (int t = 0; t < TB; ++t)
-            if (t == best) {
-                sv0 = pv[t][0];
-                sv1 = pv[t][1];
-            }
-    }
-    auto sval = [&](int b) { return regs ? (b == b0 ? sv0 : sv1) : S[b]; };
+    // (up to two blocks a thread: their values in registers)
+    double sv0 = b0 < b1 ? S[b0] : 0.0, sv1 = b0 + 1 < b1 ? S[b0 + 1] : 0.0;
+    auto sval = [&](int b) { return b == b0 ? sv0 : b == b0 + 1 ? sv1 : S[b]; };
     double own = 0.0;
     for (int b = b0; b < b1; ++b) own += sval(b);
     const double incl = wave_scan(own, lane);
