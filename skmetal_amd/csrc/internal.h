@@ -413,6 +413,7 @@ struct WSArgs {
     long long* nnz;             // [1] rows with p > 0
     double* cst;                // [ws_chunks(n) + 1] numpy's cumsum before each chunk, then the total (exact search)
     int* cseq;                  // [ws_chunks(n)] 1: the chunk's sums come from a walk in row order
+    long long* cq; int* ce;     // [ws_chunks(n)] each chunk's sum in units of its binade's grid, and the binade (exact search)
     const double* u; int m;     // this pass's uniforms
     double dmin;                // the certified search's least margin (0; larger sends more draws to the exact search)
     const long* zero; int nz;   // rows whose p is zeroed before the pass

@@ -439,68 +439,123 @@ __device__ __forceinline__ bool grid_q(double v, int e, long long& q)
     return true;
 }
 
-__global__ __launch_bounds__(kWSThreads) void k_ws_chain(WSArgs a, int nc)
+// The chunks' integer sums for the binade that the prefix of another order
+// puts the running sum in: cq[c] = Q, ce[c] = its exponent, or INT_MIN where
+// a value ends in .5 of the grid (or the sum is 0).  k_ws_chain uses them
+// where that binade is the running sum's: the chunks then cost it a few
+// cycles, and only those that cross a binade or hold a tie are walked (807 ->
+// 144 us at 500,000 rows, against every chunk's values loaded by the one block).
+__global__ __launch_bounds__(kWSThreads) void k_ws_grid(WSArgs a)
 {
     constexpr int PT = kWSChunk / kWSThreads;
-    __shared__ double tile[kWSChunk];
     __shared__ long long qred[kWSThreads / 64];
     __shared__ int bred[kWSThreads / 64];
-    __shared__ double walked;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    double s = 0.0;
-    for (int c = 0; c < nc; ++c) {
-        const long c0 = (long)c * kWSChunk;
-        const int len = (int)min((long)kWSChunk, a.n - c0);
-        double v[PT];
+    const long c0 = (long)blockIdx.x * kWSChunk;
+    const int len = (int)min((long)kWSChunk, a.n - c0);
+    const double s = a.pfx[blockIdx.x];
+    long long q = 0;
+    int bad = s > 0.0 ? 0 : 1;
+    const int e = s > 0.0 ? ilogb(s) : 0;
+    if (!bad) {
 #pragma unroll
         for (int j = 0; j < PT; ++j) {
             const int i = tid + kWSThreads * j;
-            v[j] = i < len ? a.p[c0 + i] : 0.0;
-            tile[i] = v[j];
+            long long qj = 0;
+            if (!grid_q(i < len ? a.p[c0 + i] : 0.0, e, qj)) bad = 1;
+            q += qj;
         }
-        long long q = 0;
-        int bad = s > 0.0 ? 0 : 1;
-        const int e = s > 0.0 ? ilogb(s) : 0;
-        if (!bad) {
+    }
 #pragma unroll
-            for (int j = 0; j < PT; ++j) {
-                long long qj = 0;
-                if (!grid_q(v[j], e, qj)) bad = 1;
-                q += qj;
-            }
-        }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            q += __shfl_xor(q, off, 64);
-            bad |= __shfl_xor(bad, off, 64);
-        }
-        if (lane == 0) {
-            qred[wv] = q;
-            bred[wv] = bad;
+    for (int off = 1; off < 64; off <<= 1) {
+        q += __shfl_xor(q, off, 64);
+        bad |= __shfl_xor(bad, off, 64);
+    }
+    if (lane == 0) {
+        qred[wv] = q;
+        bred[wv] = bad;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        a.cq[blockIdx.x] = (qred[0] + qred[1]) + (qred[2] + qred[3]);
+        a.ce[blockIdx.x] = (bred[0] | bred[1] | bred[2] | bred[3]) == 0 ? e : INT_MIN;
+    }
+}
+
+__global__ __launch_bounds__(kWSThreads) void k_ws_chain(WSArgs a, int nc)
+{
+    constexpr int PT = kWSChunk / kWSThreads;
+    constexpr int TC = 256;  // chunks whose integer sums are in LDS at a time
+    __shared__ double tile[kWSChunk];
+    __shared__ long long tq[TC];
+    __shared__ int te[TC];
+    __shared__ double sums[TC + 1];  // the sum before each of the tile's chunks
+    __shared__ int stop;             // the first of them that has to be walked
+    const int tid = threadIdx.x;
+    double s = 0.0;
+    for (int t0 = 0; t0 < nc; t0 += TC) {
+        const int m = min(TC, nc - t0);
+        if (tid < m) {
+            tq[tid] = a.cq[t0 + tid];
+            te[tid] = a.ce[t0 + tid];
         }
         __syncthreads();
-        const long long Q = (qred[0] + qred[1]) + (qred[2] + qred[3]);
-        bool ok = (bred[0] | bred[1] | bred[2] | bred[3]) == 0 && Q < (1LL << 53);
-        double next = s;
-        if (ok) {
-            next = s + ldexp((double)Q, e - 52);  // a multiple of g: exact while below 2^(e+1)
-            ok = next < ldexp(1.0, e + 1);
-        }
-        if (tid == 0) {
-            a.cst[c] = s;
-            a.cseq[c] = ok ? 0 : 1;
-        }
-        if (!ok) {
+        for (int c = 0; c < m;) {
+            // as far as the integer sums go
             if (tid == 0) {
                 double r = s;
-                for (int i = 0; i < len; ++i) r += tile[i];
-                walked = r;
+                int x = c;
+                for (; x < m; ++x) {
+                    sums[x] = r;
+                    const int e = r > 0.0 ? ilogb(r) : INT_MIN;
+                    const long long Q = tq[x];
+                    if (e == INT_MIN || te[x] != e || Q >= (1LL << 53)) break;
+                    // a multiple of the grid: exact while below 2^(e+1)
+                    const double next = r + ldexp((double)Q, e - 52);
+                    if (!(next < ldexp(1.0, e + 1))) break;
+                    r = next;
+                }
+                sums[x] = r;
+                stop = x;
             }
             __syncthreads();
-            next = walked;
+            const int x = stop;
+            for (int y = c + tid; y < x; y += kWSThreads) {
+                a.cst[t0 + y] = sums[y];
+                a.cseq[t0 + y] = 0;
+            }
+            s = sums[x];
+            c = x;
+            if (x < m) {  // walked in row order
+                const long c0 = (long)(t0 + x) * kWSChunk;
+                const int len = (int)min((long)kWSChunk, a.n - c0);
+#pragma unroll
+                for (int j = 0; j < PT; ++j) {
+                    const int i = tid + kWSThreads * j;
+                    tile[i] = i < len ? a.p[c0 + i] : 0.0;
+                }
+                __syncthreads();
+                if (tid == 0) {
+                    a.cst[t0 + x] = s;
+                    a.cseq[t0 + x] = 1;
+                    double r = s;
+                    int i = 0;
+                    for (; i + 16 <= len; i += 16) {
+                        double v[16];
+#pragma unroll
+                        for (int u = 0; u < 16; ++u) v[u] = tile[i + u];
+#pragma unroll
+                        for (int u = 0; u < 16; ++u) r += v[u];
+                    }
+                    for (; i < len; ++i) r += tile[i];
+                    sums[TC] = r;
+                }
+                __syncthreads();
+                s = sums[TC];
+                ++c;
+            }
+            __syncthreads();  // sums, stop and the tile are reused
         }
-        s = next;
-        __syncthreads();  // the tile and the reductions are reused
     }
     if (tid == 0) a.cst[nc] = s;
 }
@@ -617,6 +672,7 @@ hipError_t launch_ws_search(const WSArgs& a, hipStream_t s)
 hipError_t launch_ws_exact(const WSArgs& a, int all, hipStream_t s)
 {
     const int nc = ws_chunks(a.n);
+    hipLaunchKernelGGL(k_ws_grid, dim3(nc), dim3(kWSThreads), 0, s, a);
     hipLaunchKernelGGL(k_ws_chain, dim3(1), dim3(kWSThreads), 0, s, a, nc);
     hipLaunchKernelGGL(k_ws_exact_search, dim3(a.m), dim3(kWSThreads), 0, s, a, nc, all);
     return hipGetLastError();

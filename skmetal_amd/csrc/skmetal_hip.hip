@@ -1278,6 +1278,8 @@ struct Lloyd {
             if (ws.cst == nullptr) {
                 TRY(grab((void**)&ws.cst, size_t(ws_chunks(n) + 1) * sizeof(double)));
                 TRY(grab((void**)&ws.cseq, size_t(ws_chunks(n)) * sizeof(int)));
+                TRY(grab((void**)&ws.cq, size_t(ws_chunks(n)) * sizeof(long long)));
+                TRY(grab((void**)&ws.ce, size_t(ws_chunks(n)) * sizeof(int)));
             }
             HIP_TRY(launch_ws_exact(ws, exact == 1 ? 1 : 0, s), "sampling exact launch");
         }
