@@ -406,7 +406,13 @@ __global__ __launch_bounds__(512, 2) void k_screen_wide(WideArgs a)
             const f4v v = raw[u];
             *reinterpret_cast<v2u*>(dst + (lr + 4 * u) * kWideStr + 4 * q16) =
                 v2u{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
-            if (cg == 0) xx[u] = fmaf(fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w))), in, xx[u]);
+        }
+        if (cg == 0) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const f4v v = raw[u];
+                xx[u] = fmaf(fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w))), in, xx[u]);
+            }
         }
     };
     load_rows(0);
@@ -427,13 +433,20 @@ __global__ __launch_bounds__(512, 2) void k_screen_wide(WideArgs a)
         acc[c][1] = acc[c][0];
     }
     put_rows(0, 0);
+    if (nks > 1) load_rows(1);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     for (int ks = 0; ks < nks; ++ks) {
         const int cur = ks & 1;
         if (ks + 1 < nks) {
+            // the next stage: its rows, loaded a stage ago, to LDS, and its
+            // centres; then the rows of the one after it (their wait at the
+            // end of the stage left half of it idle)
+            put_rows(ks + 1, cur ^ 1);
             copy_centres(ks + 1, cur ^ 1);
-            load_rows(ks + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (ks + 2 < nks) load_rows(ks + 2);
+            __builtin_amdgcn_sched_barrier(0);
         }
         const __bf16* const xb =
             reinterpret_cast<const __bf16*>(smem + cur * stage_bytes) + (64 * wr + r32) * kWideStr + 8 * h;
@@ -453,10 +466,16 @@ __global__ __launch_bounds__(512, 2) void k_screen_wide(WideArgs a)
             }
         }
         if (ks + 1 < nks) {
-            put_rows(ks + 1, cur ^ 1);
-            // the next stage is in and this one is read: swap
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
+            // the next stage is in and this one is read: swap.  vmcnt(8):
+            // everything but the eight row loads issued last (loads complete
+            // in order); lgkmcnt(0): this wave's LDS writes.
+            if (ks + 2 < nks)
+                __builtin_amdgcn_s_waitcnt(0x0078);
+            else
+                __builtin_amdgcn_s_waitcnt(0);
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            __builtin_amdgcn_s_barrier();
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
         }
     }
 #pragma unroll
