@@ -79,10 +79,12 @@ __device__ __forceinline__ int place_centre(int p, int h)
     return 32 * (p >> 4) + 8 * ((p & 15) >> 2) + 4 * h + (p & 3);
 }
 
-// A block of 8 waves owns 512 rows, 64 per wave in two 32-row groups whose
-// high parts stay in registers (rows of at most 128 floats) while the
-// centres pass by in LDS stages of kScreenSC (the next stage copied in with
-// direct-to-LDS loads while the current one is used).  Per 32 centres a wave
+// A wave takes 64 rows at a time, in two 32-row groups whose high parts stay
+// in registers (rows of at most 128 floats) while the centres pass by in LDS
+// stages of kScreenSC: all of them resident, and the waves free to drift
+// apart, where LDS holds them, else the next stage copied in with
+// direct-to-LDS loads while the current one is used.  Each 32 x 32 tile's
+// MFMAs are issued before the values of the tile before it are taken.  Per 32 centres a wave
 // reads 2 NK 1 KB operands for 4 NK MFMAs; the accumulators start from
 // -||c||^2 / 2, so that they end as the value to maximise.  Lane l keeps the
 // two largest over its centres of row l%32 of each group, the centre's place
@@ -92,10 +94,15 @@ __device__ __forceinline__ int place_centre(int p, int h)
 // wave and SIMD alone, 106 together; the same work in 32x32x16 MFMAs 81.
 // So the rows' K steps take features 32 s + 16 (l/32) + 8 t + j: each lane's
 // 64 bytes of a row in a row.
+// As many waves as the registers leave (2M x 64, k = 1,024: 281 us with
+// twelve, 290 with eight and both groups of the next rows in flight; 1M x 128,
+// k = 256: sixteen without prefetch 149, eight with 107).
+constexpr int screen_waves(int nk) { return nk <= 2 ? 12 : 8; }
 template <int NK>
-__global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
+__global__ __launch_bounds__(64 * screen_waves(NK), screen_waves(NK) / 4) void k_screen(ScreenArgs a, int resident)
 {
     using G = ScreenGeom<NK>;
+    constexpr int NW = screen_waves(NK);
     constexpr bool PIPE = true;
     const LoopState* st = a.state;
     if (st != nullptr && (st->done != 0 || st->screen_off != 0)) return;
@@ -114,7 +121,7 @@ __global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.img), (short)0, nst * stage_bytes, 0x00020000);
     auto copy_stage = [&](int stg, int b) {
         char* dst = smem + b * stage_bytes;
-        for (int i = wave; i < stage_bytes / 1024; i += 8) {
+        for (int i = wave; i < stage_bytes / 1024; i += NW) {
             const int soff = stg * stage_bytes + i * 1024;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16,
                                                      lane * 16, soff, 0, 0);
@@ -129,7 +136,7 @@ __global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
     int cur = 0;
     // (resident: a wave stops at its own last rows; else all waves take part
     // in the stages of the block's)
-    const long wstep = (long)gridDim.x * 512;
+    const long wstep = (long)gridDim.x * (64 * NW);
     auto rows_at = [&](long base) { return resident ? base : base + (long)gridDim.x * 64 * wave; };
     auto rows_rsrc = [&](long wrow) {
         const long nrow = n - wrow < 64 ? (n - wrow > 0 ? n - wrow : 0) : 64;
@@ -138,10 +145,9 @@ __global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
     };
     // group g's rows (a lane past the rows' end loads 0, one past a row's end
     // the next row's values: these meet zero centre parts and are kept out of
-    // the norm).  PG of the next 64 rows' groups are in flight while the
-    // current ones meet the centres: registers for no more.
-    constexpr int PG = NK <= 2 ? 2 : 1;
-    f4v raw[PG][NK][4];
+    // the norm).  Group 0 of the next 64 rows is in flight while the current
+    // ones meet the centres: registers for no more.
+    f4v raw[NK][4];
     auto load = [&](f4v(&q)[NK][4], __amdgpu_buffer_rsrc_t rs, int g) {
 #pragma unroll
         for (int s = 0; s < NK; ++s) {
@@ -154,11 +160,7 @@ __global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
         }
     };
     const long first = (long)blockIdx.x * 64 + (resident ? (long)gridDim.x * 64 * wave : 0);
-    {
-        const __amdgpu_buffer_rsrc_t rs = rows_rsrc(rows_at(first));
-#pragma unroll
-        for (int g = 0; g < PG; ++g) load(raw[g], rs, g);
-    }
+    load(raw, rows_rsrc(rows_at(first)), 0);
     for (long base = first; base < n; base += wstep) {
         const long wrow = rows_at(base);
         const long nrow = n - wrow < 64 ? (n - wrow > 0 ? n - wrow : 0) : 64;
@@ -186,18 +188,10 @@ __global__ __launch_bounds__(512, 2) void k_screen(ScreenArgs a, int resident)
             // alive)
             asm volatile("" : "+v"(xx[g]));
         };
-        parts(raw[0], 0);
-        if constexpr (PG == 2) {
-            parts(raw[1], 1);
-        } else {
-            load(raw[0], rows_rsrc(wrow), 1);
-            parts(raw[0], 1);
-        }
-        if (base + wstep < n) {
-            const __amdgpu_buffer_rsrc_t rs = rows_rsrc(rows_at(base + wstep));
-#pragma unroll
-            for (int g = 0; g < PG; ++g) load(raw[g], rs, g);
-        }
+        parts(raw, 0);
+        load(raw, rows_rsrc(wrow), 1);
+        parts(raw, 1);
+        if (base + wstep < n) load(raw, rows_rsrc(rows_at(base + wstep)), 0);
         __builtin_amdgcn_sched_barrier(0);
         float m1[2], m2[2];
         int ms[2];
@@ -337,8 +331,9 @@ static hipError_t launch_screen_nk(const ScreenArgs& a, int num_cu, hipStream_t 
     if (e != hipSuccess) return e;
     const int nst = (a.k + kScreenSC - 1) / kScreenSC;
     const int resident = nst <= G::RES;
-    const long blocks = (a.n + 511) / 512;
-    hipLaunchKernelGGL(k_screen<NK>, dim3((unsigned)(blocks < num_cu ? blocks : num_cu)), dim3(512),
+    constexpr int NW = screen_waves(NK);
+    const long blocks = (a.n + 64 * NW - 1) / (64 * NW);
+    hipLaunchKernelGGL(k_screen<NK>, dim3((unsigned)(blocks < num_cu ? blocks : num_cu)), dim3(64 * NW),
                        (size_t)(resident ? nst : 2) * G::STAGE, s, a, resident);
     return hipGetLastError();
 }
