@@ -118,6 +118,7 @@ struct Context {
     void* scratch = nullptr;  // device address of this device's `scratch` array
     void* pin[2] = {nullptr, nullptr};
     hipEvent_t pin_ev[2] = {nullptr, nullptr};
+    LoopState* pin_state = nullptr;  // pinned: the loop state's read-backs
     std::multimap<size_t, void*> free_blocks;
     std::map<void*, size_t> sizes;
 
@@ -144,6 +145,8 @@ struct Context {
             HIP_TRY(hipHostMalloc(&pin[i], kPinBytes, hipHostMallocDefault), "hipHostMalloc(staging)");
             HIP_TRY(hipEventCreateWithFlags(&pin_ev[i], hipEventDisableTiming), "hipEventCreate");
         }
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&pin_state), sizeof(LoopState), hipHostMallocDefault),
+                "hipHostMalloc(state)");
         ready = true;
         return 0;
     }
@@ -673,8 +676,9 @@ struct Lloyd {
 
     int read_state(LoopState* h)
     {
-        HIP_TRY(hipMemcpyAsync(h, st, sizeof(LoopState), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(state)");
+        HIP_TRY(hipMemcpyAsync(C->pin_state, st, sizeof(LoopState), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(state)");
         HIP_TRY(hipStreamSynchronize(s), "hipStreamSynchronize");
+        *h = *C->pin_state;
         return 0;
     }
 
@@ -1208,19 +1212,21 @@ struct Lloyd {
             TRY(grab((void**)&ws.total, sizeof(float)));
             TRY(grab((void**)&ws.ctot, size_t(nc) * sizeof(double)));
             TRY(grab((void**)&ws.cnz, size_t(nc) * sizeof(int)));
-            TRY(grab((void**)&ws.pfx, size_t(nc + 1) * sizeof(double)));
-            TRY(grab((void**)&ws.nnz, sizeof(long long)));
+            // (the count of rows with p > 0 behind the prefix: one read-back)
+            TRY(grab((void**)&ws.pfx, size_t(nc + 1) * sizeof(double) + sizeof(long long)));
+            ws.nnz = reinterpret_cast<long long*>(ws.pfx + nc + 1);
         }
         ws.n = n;
         ws.w = weights == 0 ? kp_mind : nullptr;
         ws.floor = 1e-30f;
         HIP_TRY(launch_ws_prepare(ws, s), "sampling prepare launch");
-        double st[1];
-        long long z = 0;
-        TRY(download_bytes(*C, ws.pfx + ws_chunks(n), sizeof(double), st, s));
-        TRY(download_bytes(*C, ws.nnz, sizeof(long long), &z, s));
-        *psum = st[0];
-        *nnz = z;
+        struct {
+            double sum;
+            long long nz;
+        } back;
+        TRY(download_bytes(*C, ws.pfx + ws_chunks(n), sizeof(back), &back, s));
+        *psum = back.sum;
+        *nnz = back.nz;
         ws_ready = true;
         return 0;
     }
@@ -1246,15 +1252,14 @@ struct Lloyd {
         const long need = std::max(m, nz);
         if (need > ws_mcap) {
             const long cap = std::max<long>(need, 2 * ws_mcap);
-            for (void* q : {(void*)ws.u, (void*)ws.out, (void*)ws.unsure, (void*)ws.zero}) {
+            for (void* q : {(void*)ws.u, (void*)ws.out, (void*)ws.zero}) {
                 if (q == nullptr) continue;
                 const auto it = std::find(owned.begin(), owned.end(), q);
                 if (it != owned.end()) owned.erase(it);
                 C->release(q);
             }
             TRY(grab((void**)&ws.u, size_t(cap) * sizeof(double)));
-            TRY(grab((void**)&ws.out, size_t(cap) * sizeof(long)));
-            TRY(grab((void**)&ws.unsure, size_t(cap) * sizeof(int)));
+            TRY(grab((void**)&ws.out, size_t(cap) * (sizeof(long) + sizeof(int))));
             TRY(grab((void**)&ws.zero, size_t(cap) * sizeof(long)));
             ws_mcap = cap;
         }
@@ -1262,18 +1267,25 @@ struct Lloyd {
         ws.m = (int)m;
         ws.nz = (int)nz;
         ws.dmin = exact == 2 ? 0.25 / (double)n : 0.0;
+        ws.unsure = reinterpret_cast<int*>(ws.out + m);  // behind the rows: one read-back
         if (nz > 0) {
             TRY(upload_bytes(*C, zero, size_t(nz) * sizeof(long), const_cast<long*>(ws.zero), s));
             HIP_TRY(launch_ws_zero(ws, s), "sampling zero launch");
         }
         TRY(upload_bytes(*C, u, size_t(m) * sizeof(double), const_cast<double*>(ws.u), s));
-        std::vector<int> uns(size_t(m), 1);
+        long left = m;
         if (exact != 1) {
             HIP_TRY(launch_ws_search(ws, s), "sampling search launch");
-            TRY(download_bytes(*C, ws.unsure, size_t(m) * sizeof(int), uns.data(), s));
+            std::vector<char> back(size_t(m) * (sizeof(long) + sizeof(int)));
+            TRY(download_bytes(*C, ws.out, back.size(), back.data(), s));
+            std::memcpy(out, back.data(), size_t(m) * sizeof(long));
+            left = 0;
+            for (long i = 0; i < m; ++i) {
+                int unsure;
+                std::memcpy(&unsure, back.data() + size_t(m) * sizeof(long) + size_t(i) * sizeof(int), sizeof(int));
+                left += unsure != 0;
+            }
         }
-        long left = 0;
-        for (long i = 0; i < m; ++i) left += uns[i] != 0;
         if (left > 0) {
             if (ws.cst == nullptr) {
                 TRY(grab((void**)&ws.cst, size_t(ws_chunks(n) + 1) * sizeof(double)));
@@ -1282,8 +1294,8 @@ struct Lloyd {
                 TRY(grab((void**)&ws.ce, size_t(ws_chunks(n)) * sizeof(int)));
             }
             HIP_TRY(launch_ws_exact(ws, exact == 1 ? 1 : 0, s), "sampling exact launch");
+            TRY(download_bytes(*C, ws.out, size_t(m) * sizeof(long), out, s));
         }
-        TRY(download_bytes(*C, ws.out, size_t(m) * sizeof(long), out, s));
         *n_exact = (int)left;
         return 0;
     }
@@ -1741,8 +1753,9 @@ int skmetal_hip_lloyd_mindists(skmetal_hip_lloyd* h, const int64_t* rows, size_t
     Guard g(c);
     if (!h) return fail(SKMETAL_EINVAL, "null pointer argument");
     if (m > (size_t(1) << 30)) return fail(SKMETAL_ERANGE, "m=%zu candidate rows out of range", m);
+    // (without a download nothing waits: the rows went through the pinned
+    // staging, and whatever reads the distances follows on the stream)
     TRY(h->L.mindists(reinterpret_cast<const long*>(rows), (long)m, reset, dists_out));
-    HIP_TRY(hipStreamSynchronize(h->L.s), "hipStreamSynchronize");
     return 0;
 }
 
