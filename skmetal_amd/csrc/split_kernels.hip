@@ -815,10 +815,9 @@ __global__ __launch_bounds__(256) void k_centre_images(const float* __restrict__
 // acc += one K step (32 features) of the wave's 32 rows (xp, two 16-row
 // groups) against 16 CB centres: cbase is the K step of this lane's centre
 // row in the stage's high parts.
-template <int CB>
+template <int CB, typename G = Assign3Geom<CB>>
 __device__ __forceinline__ void six_products(v4f (&acc)[2][CB], const Parts8 (&xp)[2], const __bf16* cbase)
 {
-    using G = Assign3Geom<CB>;
     // four centre blocks at a time, product-major over their
     // eight accumulators: consecutive MFMAs write different
     // accumulators (a block's six products back to back wait
@@ -857,11 +856,11 @@ __device__ __forceinline__ void six_products(v4f (&acc)[2][CB], const Parts8 (&x
 // l's label and minimum ||c||^2 - 2 x.c.  xr holds the rows' first K step
 // (rows 16g + l%16, features 8h..) and `cur` the LDS stage with stage 0 of
 // the image; xload(f) loads the rows' K step at feature f into xr, next()
-// the next block's first.
+// the next block's first.  A wave without rows (active false) only copies.
 template <int CB, typename Copy, typename XLoad, typename Next>
 __device__ __forceinline__ void assign3_rows(char* smem, int ld, int npass, int nseg, int h, int r16, int& cur,
-                                             float4 (&xr)[2][2], Copy copy_stage, XLoad xload, Next next, int& mylab,
-                                             float& mymin)
+                                             float4 (&xr)[2][2], Copy copy_stage, XLoad xload, Next next, bool active,
+                                             int& mylab, float& mymin)
 {
     using G = Assign3Geom<CB>;
     constexpr int CPC = G::CPC, SEG = G::SEG, NKS = G::NKS, CSTR = G::CSTR, CPART = G::CPART;
@@ -883,7 +882,8 @@ __device__ __forceinline__ void assign3_rows(char* smem, int ld, int npass, int 
             for (int ks = 0; ks < nks; ++ks) {
                 Parts8 xp[2];
 #pragma unroll
-                for (int g = 0; g < 2; ++g) xp[g] = split8(xr[g][0], xr[g][1]);
+                for (int g = 0; g < 2; ++g)
+                    if (active) xp[g] = split8(xr[g][0], xr[g][1]);
                 // the next K step's rows: this stage's next, the next
                 // segment's or pass's first (same rows), or the next row
                 // block's first
@@ -899,7 +899,7 @@ __device__ __forceinline__ void assign3_rows(char* smem, int ld, int npass, int 
                 // the next stage's copy goes out behind the X loads that
                 // this stage still waits on (loads complete in order)
                 if (ks == nks - 1 && nst > 1) copy_stage(stg + 1 < nst ? stg + 1 : 0, cur ^ 1);
-                six_products<CB>(acc, xp, cbase + 32 * ks);
+                if (active) six_products<CB>(acc, xp, cbase + 32 * ks);
             }
             if (nst > 1) {
                 // the next stage is in (every wave's copies) and this one
@@ -1026,7 +1026,7 @@ __global__ __launch_bounds__(512, 1) void k_assign3(const float* __restrict__ X,
             [&]() {
                 if (base + (long)gridDim.x * 256 < n) xload(rows_rsrc(base + (long)gridDim.x * 256), 0);
             },
-            mylab, mymin);
+            true, mylab, mymin);
         const bool valid = lane < nrow;
         const long row = wrow + lane;
         int moved = 0;
@@ -1214,7 +1214,7 @@ __global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict
                         xload(0);
                     }
                 },
-                mylab, mymin);
+                pos + 32 * wave < cnt, mylab, mymin);
             const int i = pos + 32 * wave + lane;
             const bool valid = lane < 32 && i < cnt;
             int moved = 0;
@@ -1259,21 +1259,27 @@ __device__ __forceinline__ unsigned order_bits(float v)
     return b ^ ((b >> 31) != 0u ? 0xffffffffu : 0x80000000u);
 }
 
-__global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restrict__ X, long n, int ld,
-                                                          const char* __restrict__ img,
-                                                          const float* __restrict__ cnorm, int k,
-                                                          const unsigned* __restrict__ list, const int* nlist,
-                                                          LoopState* st, unsigned long long* __restrict__ keys)
+// A unit's centres in LDS: 16 CB of a stage's 256 rows, part by part.
+template <int CB>
+struct UnitGeom {
+    static constexpr int CSTR = Assign3Geom<16>::CSTR;
+    static constexpr int CPART = 16 * CB * CSTR;
+    static constexpr int PKB = CPART * 2 / 1024;  // KB of a part
+    static constexpr int STAGE = 3 * CPART * 2;
+    static_assert(CPART * 2 % 1024 == 0 && Assign3Geom<16>::NKS == 1, "whole KB, one K step a stage");
+};
+
+template <int CB>
+__device__ __forceinline__ void assign3_units(const float* __restrict__ X, int ld, const char* __restrict__ img,
+                                              const float* __restrict__ cnorm, int k,
+                                              const unsigned* __restrict__ list, bool all, long cnt,
+                                              unsigned long long* __restrict__ keys, char* smem)
 {
-    if (st != nullptr && st->done != 0) return;
-    constexpr int CB = 16;
-    using G = Assign3Geom<CB>;
-    constexpr int CPC = G::CPC;
-    static_assert(G::NKS == 1, "one K step a stage");
-    const bool all = st != nullptr && st->screen_off != 0;
-    const long cnt = all ? n : (long)*nlist;
-    if (st != nullptr && !all && blockIdx.x == 0 && threadIdx.x == 0) st->unsure = (int)min(cnt, 0x7fffffffL);
-    const int npass = (k + CPC - 1) / CPC;
+    using A = Assign3Geom<16>;
+    using G = UnitGeom<CB>;
+    constexpr int CPC = 16 * CB;
+    constexpr int SUB = 16 / CB;  // units a stage's centres make
+    const int npass = (k + 255) / 256 * SUB;
     const int nseg = (ld + 31) / 32;
     const long nb = (cnt + 255) / 256;
     // XCD x takes the row blocks x, x + 8, ..: its unit i is pass i % npass
@@ -1282,18 +1288,19 @@ __global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restric
     long i = blockIdx.x >> 3;
     auto block_of = [&](long j) { return xcd + 8 * (j / npass); };
     if (block_of(i) >= nb) return;
-    extern __shared__ __attribute__((aligned(1024))) char smem[];  // two stages
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 4, r16 = lane & 15;
-    const __amdgpu_buffer_rsrc_t irs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(img), (short)0,
-                                                                         npass * nseg * G::STAGE, 0x00020000);
-    const int stage_bytes = G::STAGE;
-    auto copy_stage = [&](int stg, int b) {
+    const __amdgpu_buffer_rsrc_t irs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(img), (short)0, (k + 255) / 256 * nseg * A::STAGE, 0x00020000);
+    const int stage_bytes = G::STAGE, image_stage = A::STAGE, part_bytes = A::CPART * 2, part_kb = G::PKB;
+    // K step sg of pass p: the three parts of its 16 CB centres
+    auto copy_stage = [&](int p, int sg, int b) {
         char* dst = smem + b * stage_bytes;
-        for (int q = wave; q < stage_bytes / 1024; q += 8) {
-            const int soff = stg * stage_bytes + q * 1024;
+        const int from = (p / SUB * nseg + sg) * image_stage + p % SUB * part_kb * 1024;
+        for (int q = wave; q < 3 * part_kb; q += 8) {
+            const int soff = from + q / part_kb * part_bytes + q % part_kb * 1024;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (__attribute__((address_space(3))) void*)(dst + q * 1024), 16,
                                                      lane * 16, soff, 0, 0);
         }
@@ -1320,7 +1327,7 @@ __global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restric
     };
     rows_at(i);
     xload(0);
-    copy_stage((int)(i % npass) * nseg, 0);
+    copy_stage((int)(i % npass), 0, 0);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     int cur = 0;
@@ -1329,6 +1336,7 @@ __global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restric
         const long row0 = block_of(i) * 256 + 32 * wave;
         const long nx = i + slots;
         const bool more = block_of(nx) < nb;
+        const bool active = row0 < cnt;  // (a wave without rows only copies)
         v4f acc[2][CB];
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -1339,16 +1347,17 @@ __global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restric
             const __bf16* const cbase = reinterpret_cast<const __bf16*>(smem + cur * G::STAGE) + r16 * G::CSTR + 8 * h;
             Parts8 part[2];
 #pragma unroll
-            for (int g = 0; g < 2; ++g) part[g] = split8(xr[g][0], xr[g][1]);
+            for (int g = 0; g < 2; ++g)
+                if (active) part[g] = split8(xr[g][0], xr[g][1]);
             if (sg + 1 < nseg) {
                 xload(32 * (sg + 1));
-                copy_stage(p * nseg + sg + 1, cur ^ 1);
+                copy_stage(p, sg + 1, cur ^ 1);
             } else if (more) {
                 rows_at(nx);
                 xload(0);
-                copy_stage((int)(nx % npass) * nseg, cur ^ 1);
+                copy_stage((int)(nx % npass), 0, cur ^ 1);
             }
-            six_products<CB>(acc, part, cbase);
+            if (active) six_products<CB, G>(acc, part, cbase);
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             cur ^= 1;
@@ -1388,6 +1397,25 @@ __global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restric
         if (!more) break;
         i = nx;
     }
+}
+
+// Units of 256 centres, or of 64 while those would leave half the CUs without
+// one: a unit's K steps are a chain of 12 us per 100 features at 256 centres.
+__global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restrict__ X, long n, int ld,
+                                                          const char* __restrict__ img,
+                                                          const float* __restrict__ cnorm, int k,
+                                                          const unsigned* __restrict__ list, const int* nlist,
+                                                          LoopState* st, unsigned long long* __restrict__ keys)
+{
+    if (st != nullptr && st->done != 0) return;
+    extern __shared__ __attribute__((aligned(1024))) char smem[];  // two stages
+    const bool all = st != nullptr && st->screen_off != 0;
+    const long cnt = all ? n : (long)*nlist;
+    if (st != nullptr && !all && blockIdx.x == 0 && threadIdx.x == 0) st->unsure = (int)min(cnt, 0x7fffffffL);
+    if ((cnt + 255) / 256 * ((k + 255) / 256) * 2 <= (long)gridDim.x)
+        assign3_units<4>(X, ld, img, cnorm, k, list, all, cnt, keys, smem);
+    else
+        assign3_units<16>(X, ld, img, cnorm, k, list, all, cnt, keys, smem);
 }
 
 // The labels of the units' rows from their keys.
@@ -1562,14 +1590,14 @@ hipError_t launch_assign3_units(const AssignArgs& a, const unsigned* list, const
     if (a.n <= 0) return hipSuccess;
     static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_assign3_units),
                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                    (int)Assign3Geom<16>::LDS);
+                                                    2 * UnitGeom<16>::STAGE);
     if (e != hipSuccess) return e;
     // whole rounds of the eight XCDs, one block per CU
-    const long units = (a.n + 255) / 256 * ((a.k + 255) / 256);
+    const long units = (a.n + 255) / 256 * ((a.k + 255) / 256) * 4;
     long blocks = num_cu < units ? num_cu : units;
     blocks = (blocks + 7) / 8 * 8;
-    hipLaunchKernelGGL(k_assign3_units, dim3((unsigned)blocks), dim3(512), Assign3Geom<16>::LDS, s, a.X, a.n, a.ld,
-                       a.img, a.cnorm, a.k, list, nlist, a.state, keys);
+    hipLaunchKernelGGL(k_assign3_units, dim3((unsigned)blocks), dim3(512), 2 * UnitGeom<16>::STAGE, s, a.X, a.n,
+                       a.ld, a.img, a.cnorm, a.k, list, nlist, a.state, keys);
     const long fb = (a.n + 255) / 256;
     hipLaunchKernelGGL(k_units_finish, dim3((unsigned)(fb < num_cu ? fb : num_cu)), dim3(256), 0, s, a.n, list, nlist,
                        keys, a.labels, a.state, a.changed);
