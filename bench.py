@@ -279,13 +279,15 @@ def main():
             "mfma_per_32_rows": {"e_step": 2 * e16, "sums": s32},
         }
     elif asplit:
-        # MFMA roofline of the split E-step: six bf16 products per x.c term,
-        # over the padded centres (multiples of 16 per pass) and features (32)
+        # MFMA roofline of the split E-step over the padded centres (multiples
+        # of 16 per pass) and features (32): one bf16 product per x.c term, which
+        # every row takes (the certified screen; the rows it leaves, and shapes
+        # without it, take six)
         kp = -(-k // (16 * (4 if k <= 64 else 8 if k <= 128 else 16))) * (16 * (4 if k <= 64 else 8 if k <= 128 else 16))
         dp = -(-d // 32) * 32
-        mflops = 6.0 * 2.0 * n * kp * dp
+        mflops = 2.0 * n * kp * dp
         roofline = {
-            "kernel": "k_assign3: ||c||^2 - 2 x.c on bf16 MFMAs over the exact three-part split + argmin",
+            "kernel": "k_screen / k_assign3: ||c||^2 - 2 x.c on bf16 MFMAs over the exact three-part split + argmin",
             "bound": "mfma",
             "achieved": round(mflops / assign_s / 1e12, 1),
             "peak": PEAK_BF16_MFMA_TFLOPS,
@@ -331,7 +333,7 @@ def main():
         "step_mode": (f"fused: {kname} (E-step + per-cluster sums) + k_finalize_reloc (finalize and in-stream "
                       "empty-cluster relocation in one launch; the relocation returns at once when no cluster "
                       "is empty)" if fused
-                      else f"{kname} + sorted update + k_finalize_recs + k_reloc + k_finalize_loop"),
+                      else f"{kname} (behind the screen where it pays) + sorted update + k_finalize_recs + k_reloc"),
         "e_step": ("fp32-equivalent: exact three-part bf16 split of x and c (x = hi + mid + lo), 6 of 9 part "
                    "products on v_mfma_f32_16x16x32_bf16, fp32 accumulation; the 3 left out total <= 2^-23 |x_i c_i|"
                    if (split or (asplit and not fused)) else "fp32 MFMA (v_mfma_f32_4x4x1_16b_f32)"),
