@@ -115,7 +115,7 @@ struct ScreenArgs {
     LoopState* state;             // nullable: no early exit
     int* changed;                 // nullable, as AssignArgs
     const char* img;              // launch_centre_images's simg
-    float* emin;                  // nullable: the labelled rows' minima, within 2^-8 (||x||^2 + max ||c||^2)
+    float* emin;                  // nullable: the labelled rows' minima, within 1.1 2^-7 (||x||^2 + max ||c||^2)
     unsigned long long* masks;    // [ceil(n / 64)]
 };
 size_t screen_image_bytes(int k, int ld);
@@ -340,7 +340,7 @@ struct InRelocArgs {
     const float* xnorm = nullptr;
     const float* emin = nullptr;
     // xnorm + emin lies within margin (max ||x||^2 + max ||c||^2) of the
-    // distance (2^-10 for the six products, 2^-7 for the screen's minima)
+    // distance (2^-10 for the six products, 2^-6 for the screen's minima)
     float margin = 0x1p-10f;
     // record mode (both or neither): the clusters' folded shift^2 and ||c||^2
     float* fold_shift = nullptr;

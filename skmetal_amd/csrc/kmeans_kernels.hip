@@ -2037,8 +2037,8 @@ __device__ __forceinline__ bool reloc_body(const InRelocArgs& a, int E)
     // row, the block's E-th largest of them, T, and as candidates the rows
     // within 2M of T, M = margin (max ||x||^2 + max ||c||^2).  The rows
     // wanted are all among them when the approximation and the direct form
-    // together err by at most M.  Screened steps: 1.1 2^-8 and 2^-13 of that
-    // sum, margin 2^-7.  Six-product steps (margin 2^-10): for rows of
+    // together err by at most M.  Screened steps: 1.1 2^-7 and 2^-13 of that
+    // sum, margin 2^-6.  Six-product steps (margin 2^-10): for rows of
     // at most 128 floats the approximation and the direct form each lie
     // within 2^-13 of that sum of the true distance (fp32 norms, the split's
     // dropped terms, the fp32 accumulation of at most 768 part products, and

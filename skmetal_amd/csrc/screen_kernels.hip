@@ -4,7 +4,7 @@
 // k_assign3 takes six bf16 part products for every x.c and is bound by them.
 // For most rows one of the six settles the label: the product of the high
 // parts, hh, differs from the six-product value by less than
-//   e = 1.05 (2^-8 + ..) ||x|| max ||c||   (screen_slack below),
+//   e = 1.05 (2^-7 + ..) ||x|| max ||c||   (screen_slack below),
 // so when a row's largest hh.. value leads its second largest by more than
 // 2 e, the six products have their first minimum at the same centre, and no
 // other centre can tie with it.  k_screen labels those rows and leaves the
@@ -18,17 +18,18 @@ namespace skm {
 // A bound on how far a screen value lies from x.c - ||c||^2 / 2 as the six
 // products give it, for a row with ||x||^2 = xx (fp32 sum) and C2 = the
 // largest ||c||^2, ldp features with the padding:
-//   rounding x and c to bf16 and the index in the low six or seven bits:
-//   2^-8 + 2^-18 + 2^-16 of ||x|| ||c||; the screen's fp32 accumulation, ldp + 1
+//   rounding x and c to bf16, 2^-8 of each value at most (8 significant bits),
+//   and the index in the low six or seven bits: 2^-7 + 2^-16 + 2^-16 of
+//   ||x|| ||c||; the screen's fp32 accumulation, ldp + 1
 //   terms, and the six products', 6 ldp terms, at most 2^-23 of the terms'
 //   magnitudes each (the terms of one row and centre total at most ||x||
 //   ||c|| by Cauchy-Schwarz); the products left out, 2^-22; the same for
 //   ||c||^2 / 2; and what a flush of subnormal parts and products can take.
-// The factors 1.05 and 1.01 cover the norms' own rounding.
+// The factor 1.05 covers the norms' own rounding.
 __device__ __forceinline__ float screen_slack(float xx, float C2, int ldp)
 {
     const float xn = sqrtf(xx), cn = sqrtf(C2);
-    const float a = 0x1p-8f + 0x1p-15f + 8.f * (float)ldp * 0x1p-23f;
+    const float a = 0x1p-7f + 0x1p-14f + 8.f * (float)ldp * 0x1p-23f;
     const float b = 0x1p-15f + (float)(ldp + 2) * 0x1p-23f;
     return 1.05f * (a * xn * cn + b * 0.5f * C2) + 0x1p-100f * (xn + cn) + 0x1p-100f;
 }

@@ -833,7 +833,7 @@ struct Lloyd {
             // this step's E-step was k_fused3 or k_assign3, which wrote its row minima
             r.xnorm = xnorm;
             r.emin = emin;
-            if (fblocks == 0 && screened()) r.margin = 0x1p-7f;
+            if (fblocks == 0 && screened()) r.margin = 0x1p-6f;
         }
         if (reloc_inline && fblocks > 0 && k <= 64 && 8 * ((k * r.nch + 7) / 8) <= kRelocInlineBlocks) {
             // the fused kernel's presence bits name the empty clusters: one launch

@@ -98,3 +98,26 @@ def test_screen_relocation(monkeypatch, n, d, k):
     C[[4, 20, k - 1]] += 300.0
     lab = _both(monkeypatch, X, C)
     assert len(np.unique(lab)) == k
+
+
+# Every value rounds to bf16 by 2^-8 of itself, in the direction that moves the
+# high-part product of one centre up and of the other down: the pair's screen
+# gap is wrong by nearly 4 * 2^-8 ||x|| ||c||, the most there is, and of the
+# wrong sign.  The bound has to leave such rows to the six products.
+@pytest.mark.parametrize("d", [128, 512])
+def test_screen_worst_rounding(monkeypatch, d):
+    up, down = 1 + 2.0**-8, 1 + 3 * 2.0**-8  # ties: to 1 and to 1 + 2^-6
+    half = (d - 4) // 2
+    x = np.r_[np.full(half, up), np.full(half, -down), 1, 0, 0, 0]
+    c1 = np.r_[np.full(half, up), np.full(half, down), 1.2 * d * 2.0**-7, 0, 0, 0]
+    c1[-4] = np.round(c1[-4] * 64) / 64
+    C = np.empty((160, d), np.float32)
+    C[:] = -0.9 * x * (1 - 1e-3 * np.arange(160)[:, None])
+    C[70], C[7] = c1, -c1
+    X = np.repeat(x[None], 1000, 0).astype(np.float32)
+    _both(monkeypatch, X, C, steps=1)
+    from skmetal_amd import _bridge
+
+    lab = np.empty(len(X), np.int32)  # with the screen
+    _bridge.kmeans_assign(X, C, lab, len(X), d, len(C))
+    assert (lab == 70).all()
