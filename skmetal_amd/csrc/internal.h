@@ -145,15 +145,21 @@ hipError_t launch_screen_wide(const WideArgs& a, hipStream_t s);
 // costs about one round again (nearly every block has a row) and the second
 // launch and its image 20 us, so it is the rounds after the first that are
 // saved.  Timed, a step without / with the screen: 64 floats, k = 1,024:
-// 60,000 rows 95 / 121 us, 120,000 139 / 129, 1,000,000 767 / 318; 128
-// floats, k = 256: 120,000 97 / 101, 250,000 152 / 127, 1,000,000 493 / 308.
+// 60,000 rows 92 / 107 us, 120,000 134 / 111, 1,000,000 693 / 311; 128
+// floats, k = 256: 120,000 91 / 89, 250,000 144 / 114, 1,000,000 442 / 280.
 // Longer rows: the rest goes by units of 256 rows x 256 centres and costs
-// little, but there are two more launches.  768 floats: k = 200 (one unit
-// wide) 64,000 rows 173 / 212 us, 130,000 335 / 306; k = 1,500: 8,000 rows
-// 638 / 156; 300 floats, k = 600: 8,000 rows 168 / 122.
+// little, but there are two more launches.  768 floats, k = 1,500: 8,000 rows
+// 610 / 126; 300 floats: k = 600, 8,000 rows 161 / 87; k = 200, 130,000 rows
+// 158 / 142, 400,000 444 / 337; k = 512, 64,000 rows 150 / 124, 130,000 251 /
+// 175.  The slack grows with the norms: of blobs of 768 floats most rows are
+// left, and with at most two units of centres nothing is saved once
+// k_assign3's blocks fill half the CUs: k = 200, 130,000 rows 326 / 363,
+// 390,000 890 / 958; k = 400, 30,000 rows 242 / 183, 64,000 271 / 302,
+// 130,000 521 / 588.
 inline bool screen_pays(long n, int ld, int k)
 {
     if (n >= (1L << 31) || k <= 128) return false;
+    if (ld > 512 && k <= 512 && n > 32768) return false;
     const double round = (double)((k + 255) / 256 * 256) * ((ld + 31) / 32 * 32);
     const double rounds = (double)((n + 65535) / 65536);
     return ld <= 128 ? (rounds - 1) * round >= 60e3 : rounds * round >= 230e3;
