@@ -25,10 +25,14 @@ namespace skm {
 //   magnitudes each (the terms of one row and centre total at most ||x||
 //   ||c|| by Cauchy-Schwarz); the products left out, 2^-22; the same for
 //   ||c||^2 / 2; and what a flush of subnormal parts and products can take.
-// The factor 1.05 covers the norms' own rounding.
+// The factor 1.05 covers the norms' own rounding, and ldp 2^-125 what their
+// squares lose below the smallest normal number (centres of 2^-80 have
+// ||c||^2 = 0 in fp32, but products with rows of order 1 that the six products
+// tell apart).
 __device__ __forceinline__ float screen_slack(float xx, float C2, int ldp)
 {
-    const float xn = sqrtf(xx), cn = sqrtf(C2);
+    const float lost = (float)ldp * 0x1p-125f;
+    const float xn = sqrtf(xx + lost), cn = sqrtf(C2 + lost);
     const float a = 0x1p-7f + 0x1p-14f + 8.f * (float)ldp * 0x1p-23f;
     const float b = 0x1p-15f + (float)(ldp + 2) * 0x1p-23f;
     return 1.05f * (a * xn * cn + b * 0.5f * C2) + 0x1p-100f * (xn + cn) + 0x1p-100f;

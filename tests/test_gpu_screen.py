@@ -104,8 +104,10 @@ def test_screen_relocation(monkeypatch, n, d, k):
 # high-part product of one centre up and of the other down: the pair's screen
 # gap is wrong by nearly 4 * 2^-8 ||x|| ||c||, the most there is, and of the
 # wrong sign.  The bound has to leave such rows to the six products.
+# So too when ||c||^2 is below fp32's range and its root bounds nothing.
+@pytest.mark.parametrize("scale", [0, -80])
 @pytest.mark.parametrize("d", [128, 512])
-def test_screen_worst_rounding(monkeypatch, d):
+def test_screen_worst_rounding(monkeypatch, d, scale):
     up, down = 1 + 2.0**-8, 1 + 3 * 2.0**-8  # ties: to 1 and to 1 + 2^-6
     half = (d - 4) // 2
     x = np.r_[np.full(half, up), np.full(half, -down), 1, 0, 0, 0]
@@ -114,6 +116,7 @@ def test_screen_worst_rounding(monkeypatch, d):
     C = np.empty((160, d), np.float32)
     C[:] = -0.9 * x * (1 - 1e-3 * np.arange(160)[:, None])
     C[70], C[7] = c1, -c1
+    C *= np.float32(2.0**scale)
     X = np.repeat(x[None], 1000, 0).astype(np.float32)
     _both(monkeypatch, X, C, steps=1)
     from skmetal_amd import _bridge
