@@ -28,6 +28,7 @@
 #include <rocblas/rocblas.h>  // types only: librocblas is opened on the first skmetal_gemm
 
 #include "skmetal_hip.h"
+#include "host_rules.h"
 #include "internal.h"
 
 using namespace skm;
@@ -478,6 +479,21 @@ struct Lloyd {
         return 0;
     }
 
+    // A buffer of grab's given back (null allowed).
+    void drop(void* p)
+    {
+        const auto it = std::find(owned.begin(), owned.end(), p);
+        if (p == nullptr || it == owned.end()) return;
+        owned.erase(it);
+        C->release(p);
+    }
+
+    // A workspace: every buffer of the list, or none.
+    int grab_workspace(std::initializer_list<Buffer> list)
+    {
+        return grab_all(list, [this](void** p, size_t b) { return grab(p, b); }, [this](void* p) { drop(p); });
+    }
+
     // A problem on caller-owned device memory (X [n x d], rows of exactly the
     // fused kernels' stride, used as given; the centres are read from Cdev;
     // labels written to labdev) with every other buffer in the arena.  Only the
@@ -715,12 +731,12 @@ struct Lloyd {
             if (minima) a.emin = emin;
             if (screened() && ld > 128) {
                 if (simg == nullptr) {
-                    TRY(grab((void**)&spart, wide_part_floats(n, k) * sizeof(float)));
-                    TRY(grab((void**)&sxx, size_t(n) * sizeof(float)));
-                    TRY(grab((void**)&slist, size_t(n) * sizeof(unsigned)));
-                    TRY(grab((void**)&snlist, sizeof(int)));
-                    TRY(grab((void**)&smask, size_t(n) * sizeof(unsigned long long)));
-                    TRY(grab((void**)&simg, wide_image_bytes(k, ld)));
+                    TRY(grab_workspace({{(void**)&spart, wide_part_floats(n, k) * sizeof(float)},
+                                        {(void**)&sxx, size_t(n) * sizeof(float)},
+                                        {(void**)&slist, size_t(n) * sizeof(unsigned)},
+                                        {(void**)&snlist, sizeof(int)},
+                                        {(void**)&smask, size_t(n) * sizeof(unsigned long long)},
+                                        {(void**)&simg, wide_image_bytes(k, ld)}}));
                 }
                 const WideArgs wa{X, n, ld, cnorm, k, labels, state, changed, simg, spart, sxx, slist, snlist, smask};
                 HIP_TRY(launch_wide_images(a, simg, snlist, s), "centre image launch");
@@ -730,8 +746,8 @@ struct Lloyd {
             }
             if (screened()) {
                 if (simg == nullptr) {
-                    TRY(grab((void**)&simg, screen_image_bytes(k, ld)));
-                    TRY(grab((void**)&smask, size_t((n + 63) / 64) * sizeof(unsigned long long)));
+                    TRY(grab_workspace({{(void**)&smask, size_t((n + 63) / 64) * sizeof(unsigned long long)},
+                                        {(void**)&simg, screen_image_bytes(k, ld)}}));
                 }
                 const ScreenArgs sa{X, n, ld, k, labels, state, changed, simg, a.emin, smask};
                 HIP_TRY(launch_centre_images(a, simg, s), "centre image launch");
@@ -876,9 +892,9 @@ struct Lloyd {
     {
         if (rowout == nullptr) TRY(grab((void**)&rowout, size_t(n) * sizeof(float)));
         if (r_cand_d == nullptr) {
-            TRY(grab((void**)&r_cand_d, size_t(kRelocCandBlocks) * kMaxReloc * sizeof(float)));
-            TRY(grab((void**)&r_cand_i, size_t(kRelocCandBlocks) * kMaxReloc * sizeof(long)));
-            TRY(grab((void**)&r_amax, sizeof(int)));
+            TRY(grab_workspace({{(void**)&r_cand_d, size_t(kRelocCandBlocks) * kMaxReloc * sizeof(float)},
+                                {(void**)&r_cand_i, size_t(kRelocCandBlocks) * kMaxReloc * sizeof(long)},
+                                {(void**)&r_amax, sizeof(int)}}));
         }
         LoopState w = hs;
         w.done = 0;
@@ -1156,18 +1172,18 @@ struct Lloyd {
         if (kp_mind == nullptr) TRY(grab((void**)&kp_mind, size_t(n) * sizeof(float)));
         if (m > kp_cap) {
             const long cap = std::max<long>(m, 2 * kp_cap);
-            for (void** p : {(void**)&kp_cand, (void**)&kp_ctab, (void**)&kp_ccn})
-                if (*p != nullptr) {
-                    const auto it = std::find(owned.begin(), owned.end(), *p);
-                    if (it != owned.end()) owned.erase(it);
-                    C->release(*p);
-                    *p = nullptr;
-                }
-            TRY(grab((void**)&kp_cand, size_t(cap) * sizeof(long)));
+            kp_cap = 0;
+            for (void** p : {(void**)&kp_cand, (void**)&kp_ctab, (void**)&kp_ccn}) {
+                drop(*p);
+                *p = nullptr;
+            }
             if (pp_rows_min_path(ld)) {  // candidates rounded up to a multiple of 16
                 const size_t capp = size_t(cap + 15) / 16 * 16;
-                TRY(grab((void**)&kp_ctab, capp * ld * sizeof(double)));
-                TRY(grab((void**)&kp_ccn, capp * sizeof(double)));
+                TRY(grab_workspace({{(void**)&kp_cand, size_t(cap) * sizeof(long)},
+                                    {(void**)&kp_ctab, capp * ld * sizeof(double)},
+                                    {(void**)&kp_ccn, capp * sizeof(double)}}));
+            } else {
+                TRY(grab((void**)&kp_cand, size_t(cap) * sizeof(long)));
             }
             kp_cap = cap;
         }
@@ -1207,13 +1223,13 @@ struct Lloyd {
         if (n >= (1L << 31)) return fail(SKMETAL_ERANGE, "sampling supports n < 2^31 rows (n=%ld)", n);
         if (ws.p == nullptr) {
             const int nb = ws_blocks(n), nc = ws_chunks(n);
-            TRY(grab((void**)&ws.p, size_t(n) * sizeof(double)));
-            TRY(grab((void**)&ws.bsum, size_t(nb) * sizeof(float)));
-            TRY(grab((void**)&ws.total, sizeof(float)));
-            TRY(grab((void**)&ws.ctot, size_t(nc) * sizeof(double)));
-            TRY(grab((void**)&ws.cnz, size_t(nc) * sizeof(int)));
             // (the count of rows with p > 0 behind the prefix: one read-back)
-            TRY(grab((void**)&ws.pfx, size_t(nc + 1) * sizeof(double) + sizeof(long long)));
+            TRY(grab_workspace({{(void**)&ws.p, size_t(n) * sizeof(double)},
+                                {(void**)&ws.bsum, size_t(nb) * sizeof(float)},
+                                {(void**)&ws.total, sizeof(float)},
+                                {(void**)&ws.ctot, size_t(nc) * sizeof(double)},
+                                {(void**)&ws.cnz, size_t(nc) * sizeof(int)},
+                                {(void**)&ws.pfx, size_t(nc + 1) * sizeof(double) + sizeof(long long)}}));
             ws.nnz = reinterpret_cast<long long*>(ws.pfx + nc + 1);
         }
         ws.n = n;
@@ -1252,15 +1268,14 @@ struct Lloyd {
         const long need = std::max(m, nz);
         if (need > ws_mcap) {
             const long cap = std::max<long>(need, 2 * ws_mcap);
-            for (void* q : {(void*)ws.u, (void*)ws.out, (void*)ws.zero}) {
-                if (q == nullptr) continue;
-                const auto it = std::find(owned.begin(), owned.end(), q);
-                if (it != owned.end()) owned.erase(it);
-                C->release(q);
+            ws_mcap = 0;
+            for (void** p : {(void**)&ws.u, (void**)&ws.out, (void**)&ws.zero}) {
+                drop(*p);
+                *p = nullptr;
             }
-            TRY(grab((void**)&ws.u, size_t(cap) * sizeof(double)));
-            TRY(grab((void**)&ws.out, size_t(cap) * (sizeof(long) + sizeof(int))));
-            TRY(grab((void**)&ws.zero, size_t(cap) * sizeof(long)));
+            TRY(grab_workspace({{(void**)&ws.u, size_t(cap) * sizeof(double)},
+                                {(void**)&ws.out, size_t(cap) * (sizeof(long) + sizeof(int))},
+                                {(void**)&ws.zero, size_t(cap) * sizeof(long)}}));
             ws_mcap = cap;
         }
         if (exact < 0 || exact > 2) return fail(SKMETAL_EINVAL, "exact=%d is not 0, 1 or 2", exact);
@@ -1288,10 +1303,10 @@ struct Lloyd {
         }
         if (left > 0) {
             if (ws.cst == nullptr) {
-                TRY(grab((void**)&ws.cst, size_t(ws_chunks(n) + 1) * sizeof(double)));
-                TRY(grab((void**)&ws.cseq, size_t(ws_chunks(n)) * sizeof(int)));
-                TRY(grab((void**)&ws.cq, size_t(ws_chunks(n)) * sizeof(long long)));
-                TRY(grab((void**)&ws.ce, size_t(ws_chunks(n)) * sizeof(int)));
+                TRY(grab_workspace({{(void**)&ws.cst, size_t(ws_chunks(n) + 1) * sizeof(double)},
+                                    {(void**)&ws.cseq, size_t(ws_chunks(n)) * sizeof(int)},
+                                    {(void**)&ws.cq, size_t(ws_chunks(n)) * sizeof(long long)},
+                                    {(void**)&ws.ce, size_t(ws_chunks(n)) * sizeof(int)}}));
             }
             HIP_TRY(launch_ws_exact(ws, exact == 1 ? 1 : 0, s), "sampling exact launch");
             TRY(download_bytes(*C, ws.out, size_t(m) * sizeof(long), out, s));
