@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "host_rules.h"
+
 namespace skm {
 
 // Per-fit loop state, resident in device memory.  Every kernel of the
@@ -130,13 +132,13 @@ struct WideArgs {
     LoopState* state;             // nullable: no early exit
     int* changed;                 // nullable, as AssignArgs
     const char* img;              // launch_wide_images's wimg
-    float* part;                  // [2 ceil(k / 256)][n][2]
-    float* xx;                    // [n] ||x||^2
+    float* part;                  // [2 ceil(k / 256)][wide_rows(n, k)][2]
+    float* xx;                    // [wide_rows(n, k)] ||x||^2
     unsigned* list; int* nlist;   // [n], [1]: the rows left
     unsigned long long* keys;     // [n], of the rows left
+    long row0 = 0;                // (of a launch: the first of its rows)
 };
 size_t wide_image_bytes(int k, int ld);
-inline size_t wide_part_floats(long n, int k) { return size_t(n) * size_t(k + 255) / 256 * 4; }
 hipError_t launch_screen_wide(const WideArgs& a, hipStream_t s);
 
 // Where the screen pays.  k_assign3 alone takes its 256-row blocks in rounds

@@ -354,7 +354,7 @@ static hipError_t launch_screen_nk(const ScreenArgs& a, int num_cu, hipStream_t 
 // centres come in with direct-to-LDS loads, and its rows as fp32 into
 // registers, rounded to bf16 on the way to LDS.  Blocks of one row block
 // follow each other on one XCD (block b runs on XCD b % 8), so that X and the
-// image come from its L2.
+// image come from its L2.  A launch takes wide_rows rows.
 __global__ __launch_bounds__(512, 2) void k_screen_wide(WideArgs a)
 {
     const LoopState* st = a.state;
@@ -566,7 +566,7 @@ __global__ __launch_bounds__(256) void k_screen_merge(WideArgs a)
         sAt = sLeft != 0 ? atomicAdd(a.nlist, sLeft) : 0;
     }
     __syncthreads();
-    if (valid && !sure) a.list[sAt + at] = (unsigned)row;
+    if (valid && !sure) a.list[sAt + at] = (unsigned)(a.row0 + row);
 }
 
 size_t wide_image_bytes(int k, int ld)
@@ -581,12 +581,20 @@ hipError_t launch_screen_wide(const WideArgs& a, hipStream_t s)
     static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_screen_wide),
                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 4 * kWideStage);
     if (e != hipSuccess) return e;
-    const long nrb = (a.n + 255) / 256, ncg = (a.k + 255) / 256;
-    const long grid = 8 * ((nrb + 7) / 8) * ncg;
-    if (grid >= (1L << 31)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_screen_wide, dim3((unsigned)grid), dim3(512), 4 * kWideStage, s, a);
-    hipLaunchKernelGGL(k_screen_merge, dim3((unsigned)nrb), dim3(256), 0, s, a);
-    return hipGetLastError();
+    const long rows = wide_rows(a.n, a.k);
+    for (long r = 0; r < a.n; r += rows) {
+        WideArgs b = a;
+        b.row0 = r;
+        b.n = a.n - r < rows ? a.n - r : rows;
+        b.X += r * a.ld;
+        b.labels += r;
+        b.keys += r;
+        hipLaunchKernelGGL(k_screen_wide, dim3((unsigned)wide_blocks(b.n, b.k)), dim3(512), 4 * kWideStage, s, b);
+        hipLaunchKernelGGL(k_screen_merge, dim3((unsigned)((b.n + 255) / 256)), dim3(256), 0, s, b);
+        const hipError_t le = hipGetLastError();
+        if (le != hipSuccess) return le;
+    }
+    return hipSuccess;
 }
 
 size_t screen_image_bytes(int k, int ld)

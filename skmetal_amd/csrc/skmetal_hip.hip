@@ -28,7 +28,6 @@
 #include <rocblas/rocblas.h>  // types only: librocblas is opened on the first skmetal_gemm
 
 #include "skmetal_hip.h"
-#include "host_rules.h"
 #include "internal.h"
 
 using namespace skm;
@@ -731,8 +730,8 @@ struct Lloyd {
             if (minima) a.emin = emin;
             if (screened() && ld > 128) {
                 if (simg == nullptr) {
-                    TRY(grab_workspace({{(void**)&spart, wide_part_floats(n, k) * sizeof(float)},
-                                        {(void**)&sxx, size_t(n) * sizeof(float)},
+                    TRY(grab_workspace({{(void**)&spart, wide_part_floats(wide_rows(n, k), k) * sizeof(float)},
+                                        {(void**)&sxx, size_t(wide_rows(n, k)) * sizeof(float)},
                                         {(void**)&slist, size_t(n) * sizeof(unsigned)},
                                         {(void**)&snlist, sizeof(int)},
                                         {(void**)&smask, size_t(n) * sizeof(unsigned long long)},

@@ -49,6 +49,8 @@ def _both(monkeypatch, X, C, steps=5):
     # rows of more than 128 floats: 256 x 256 units, ends off both, one
     # 64-feature stage more than whole ones
     (3000, 129, 200, 0.5), (777, 300, 257, 0.4), (20011, 768, 700, 0.3), (300, 1000, 300, 0.2), (256, 192, 256, 0.3),
+    # two launches of k_screen_wide (210,944 rows and the rest)
+    (212_000, 132, 20_000, 0.4),
 ])
 def test_screen_labels_match_six_products(monkeypatch, n, d, k, spread):
     _both(monkeypatch, *_blobs(n, d, k, spread, n + d))

@@ -44,6 +44,9 @@ extern "C" int workspace(int fails)
         if (p[i] != mem + i + 1) return 6;
     return 0;
 }
+extern "C" long rows(long n, int k) { return wide_rows(n, k); }
+extern "C" long blocks(long rows, int k) { return wide_blocks(rows, k); }
+extern "C" long part_bytes(long rows, int k) { return (long)wide_part_floats(rows, k) * 4; }
 """
 
 
@@ -53,9 +56,25 @@ def rules(tmp_path_factory):
     (d / "rules.cpp").write_text(SOURCE)
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}", str(d / "rules.cpp"),
                     "-o", str(d / "rules.so")], check=True)
-    return ctypes.CDLL(str(d / "rules.so"))
+    lib = ctypes.CDLL(str(d / "rules.so"))
+    for f in (lib.rows, lib.blocks, lib.part_bytes):
+        f.argtypes, f.restype = [ctypes.c_long, ctypes.c_int], ctypes.c_long
+    return lib
 
 
 @pytest.mark.parametrize("fails", range(6))
 def test_a_workspace_is_whole_or_absent(rules, fails):
     assert rules.workspace(fails) == 0
+
+
+# all rows in one launch: 4.8 and 5.1 G threads, where HIP takes less than 2^32,
+# and 38 and 41 GB of workspace
+@pytest.mark.parametrize("n,k", [(100_000_000, 6_000), (10_000_000, 65_536), (2**31 - 1, 2**20), (2**31 - 1, 129),
+                                 (300, 2**20), (2048, 257), (1, 1), (212_000, 20_000)])
+def test_the_wide_screen_in_launches_that_hip_takes(rules, n, k):
+    rows = rules.rows(n, k)
+    assert 0 < rows <= n and (rows == n or rows % 2048 == 0)
+    assert rules.blocks(rows, k) * 512 < 2**32 and (rows + 255) // 256 * 256 < 2**32
+    assert rules.part_bytes(rows, k) == rows * ((k + 255) // 256) * 16 <= 2**28
+    # (the rows of a launch: their blocks cover them, 256 a block and 256 centres)
+    assert rules.blocks(rows, k) * 256 >= rows * ((k + 255) // 256)
