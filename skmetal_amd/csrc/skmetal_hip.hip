@@ -168,7 +168,10 @@ struct Context {
             (void)hipGetLastError();  // clear the failed allocation's error
             release_cache();
             e = hipMalloc(&p, bytes);
-            if (e != hipSuccess) return hip_fail(e, "hipMalloc");
+            if (e != hipSuccess) {
+                (void)hipGetLastError();  // else the next launch reports it
+                return hip_fail(e, "hipMalloc");
+            }
         }
         sizes[p] = bytes;
         *out = p;
@@ -712,13 +715,36 @@ struct Lloyd {
     unsigned* slist = nullptr;
     int* snlist = nullptr;
     // the E-step behind k_screen.  SKMETAL_HIP_SCREEN=0 keeps every row on
-    // the six products, 1 screens every shape that the screen takes (tests)
+    // the six products, 1 screens every shape that the screen takes, 2 does so
+    // and refuses the screen its memory (tests)
+    bool screen_nomem = false;  // the device had no memory for the screen's buffers
     bool screened() const
     {
-        if (!split_on || !a3cap || n >= (1L << 31) || (ld > 128 && k <= 128)) return false;
+        if (!split_on || !a3cap || screen_nomem || n >= (1L << 31) || (ld > 128 && k <= 128)) return false;
         const char* e = getenv("SKMETAL_HIP_SCREEN");
-        if (e != nullptr && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
+        if (e != nullptr && e[0] >= '0' && e[0] <= '2') return e[0] != '0';
         return screen_pays(n, ld, k);
+    }
+
+    // The screen's buffers.  Without memory for them the handle stays on the
+    // six products, which need none of it: screened() is false from then on.
+    int screen_buffers()
+    {
+        if (simg != nullptr) return 0;
+        const char* e = getenv("SKMETAL_HIP_SCREEN");
+        const size_t more = e != nullptr && e[0] == '2' ? size_t(1) << 50 : 0;
+        const int rc = ld > 128 ? grab_workspace({{(void**)&spart, wide_part_floats(wide_rows(n, k), k) * sizeof(float)},
+                                                  {(void**)&sxx, size_t(wide_rows(n, k)) * sizeof(float)},
+                                                  {(void**)&slist, size_t(n) * sizeof(unsigned)},
+                                                  {(void**)&snlist, sizeof(int)},
+                                                  {(void**)&smask, size_t(n) * sizeof(unsigned long long)},
+                                                  {(void**)&simg, wide_image_bytes(k, ld) + more}})
+                                : grab_workspace({{(void**)&smask, size_t((n + 63) / 64) * sizeof(unsigned long long)},
+                                                  {(void**)&simg, screen_image_bytes(k, ld) + more}});
+        if (rc != SKMETAL_ENOMEM) return rc;
+        g_err.clear();
+        screen_nomem = true;
+        return 0;
     }
 
     int assign(const float* cents, LoopState* state, int* changed, bool minima = false)
@@ -728,15 +754,8 @@ struct Lloyd {
             if (a3img == nullptr) TRY(grab((void**)&a3img, assign3_image_bytes(k, ld)));
             a.img = a3img;
             if (minima) a.emin = emin;
+            if (screened()) TRY(screen_buffers());
             if (screened() && ld > 128) {
-                if (simg == nullptr) {
-                    TRY(grab_workspace({{(void**)&spart, wide_part_floats(wide_rows(n, k), k) * sizeof(float)},
-                                        {(void**)&sxx, size_t(wide_rows(n, k)) * sizeof(float)},
-                                        {(void**)&slist, size_t(n) * sizeof(unsigned)},
-                                        {(void**)&snlist, sizeof(int)},
-                                        {(void**)&smask, size_t(n) * sizeof(unsigned long long)},
-                                        {(void**)&simg, wide_image_bytes(k, ld)}}));
-                }
                 const WideArgs wa{X, n, ld, cnorm, k, labels, state, changed, simg, spart, sxx, slist, snlist, smask};
                 HIP_TRY(launch_wide_images(a, simg, snlist, s), "centre image launch");
                 HIP_TRY(launch_screen_wide(wa, s), "screen launch");
@@ -744,10 +763,6 @@ struct Lloyd {
                 return 0;
             }
             if (screened()) {
-                if (simg == nullptr) {
-                    TRY(grab_workspace({{(void**)&smask, size_t((n + 63) / 64) * sizeof(unsigned long long)},
-                                        {(void**)&simg, screen_image_bytes(k, ld)}}));
-                }
                 const ScreenArgs sa{X, n, ld, k, labels, state, changed, simg, a.emin, smask};
                 HIP_TRY(launch_centre_images(a, simg, s), "centre image launch");
                 HIP_TRY(launch_screen(sa, C->num_cu, s), "screen launch");
@@ -767,6 +782,7 @@ struct Lloyd {
     int assign_inertia(const float* cents, double* out)
     {
         const long blocks = std::min<long>(C->num_cu, (n + 255) / 256);
+        if (screened()) TRY(screen_buffers());
         if (split_on && a3cap && blocks <= rowdist_grid(n) && !screened()) {
             if (a3img == nullptr) TRY(grab((void**)&a3img, assign3_image_bytes(k, ld)));
             AssignArgs a{X, n, ld, cents, cnorm, k, labels, nullptr, nullptr, a3img};

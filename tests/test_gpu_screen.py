@@ -126,3 +126,28 @@ def test_screen_worst_rounding(monkeypatch, d, scale):
     lab = np.empty(len(X), np.int32)  # with the screen
     _bridge.kmeans_assign(X, C, lab, len(X), d, len(C))
     assert (lab == 70).all()
+
+
+# a device without memory for the screen's buffers: the six products take every
+# row, in that call and in the handle's later ones, and nothing is reported
+@pytest.mark.parametrize("n,d,k", [(5000, 64, 300), (5000, 200, 300)])
+def test_screen_without_memory(monkeypatch, n, d, k):
+    from skmetal_amd import _bridge
+
+    X, C = _blobs(n, d, k, 0.5, 9)
+    got = []
+    for mode in "02":
+        monkeypatch.setenv("SKMETAL_HIP_SCREEN", mode)
+        lab = np.empty(n, np.int32)
+        _bridge.kmeans_assign(X, C, lab, n, d, k)
+        with _bridge.LloydHandle(n, d, k) as h:
+            h.load(X)
+            for mode in {"0": "0", "2": "21"}[mode]:
+                monkeypatch.setenv("SKMETAL_HIP_SCREEN", mode)
+                h.set_centers(C)
+                run = h.run(4, 0.0, strict=False)
+                got.append((lab, h.labels(), h.centers(), np.array(run)))
+            assert _bridge.last_error() == ""
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            np.testing.assert_array_equal(a, b)
