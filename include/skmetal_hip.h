@@ -306,6 +306,13 @@ SKMETAL_API int skmetal_hip_lloyd_sample_draw(skmetal_hip_lloyd* h, const int64_
  * separate E-step kernel (generic path, final E-step, assign) uses the same
  * split; *partials = per-step partial sums the finalize reduces. */
 SKMETAL_API int skmetal_hip_lloyd_info(skmetal_hip_lloyd* h, int* fused, int* partials);
+/* The screened E-step of the generic path (one bf16 product settles most
+ * labels, the split's six products the rest): *screened = 1 when the handle's
+ * steps run it on the loaded data; of the last run or iterate, *left = rows
+ * that its last screened step left to the six products (-1: none was
+ * screened), *off = 1 when the steps after that took the six products for
+ * every row. */
+SKMETAL_API int skmetal_hip_lloyd_screen_info(skmetal_hip_lloyd* h, int* screened, int64_t* left, int* off);
 SKMETAL_API int skmetal_hip_lloyd_get_centers(skmetal_hip_lloyd* h, float* C);
 SKMETAL_API int skmetal_hip_lloyd_get_labels(skmetal_hip_lloyd* h, int32_t* labels);
 /* Inertia of the current labels against the current centres (fp64). */

@@ -60,6 +60,8 @@ _REGISTRY = [
     ("skmetal_hip_lloyd_run", ctypes.c_int, _vp, _c_size, ctypes.c_double, ctypes.c_int,
      ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_double)),
     ("skmetal_hip_lloyd_info", ctypes.c_int, _vp, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)),
+    ("skmetal_hip_lloyd_screen_info", ctypes.c_int, _vp, ctypes.POINTER(ctypes.c_int),
+     ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int)),
     ("skmetal_hip_lloyd_get_centers", ctypes.c_int, _vp, _vp),
     ("skmetal_hip_lloyd_get_labels", ctypes.c_int, _vp, _vp),
     ("skmetal_hip_lloyd_inertia", ctypes.c_int, _vp, ctypes.POINTER(ctypes.c_double)),
@@ -481,6 +483,15 @@ class LloydHandle:
                "skmetal_hip_lloyd_info")
         mode = int(fused.value)
         return dict(fused=bool(mode & 3), split=(mode & 3) == 2, asplit=bool(mode & 4), partials=int(partials.value))
+
+    def screen_info(self):
+        """The screened E-step: whether the loaded problem's steps run it, the rows that the
+        last screened step of the last run left to the six products (-1: none was screened),
+        and whether the steps after it took the six products for every row."""
+        on, off, left = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int64(0)
+        _check(_lib.skmetal_hip_lloyd_screen_info(self._h, ctypes.byref(on), ctypes.byref(left), ctypes.byref(off)),
+               "skmetal_hip_lloyd_screen_info")
+        return dict(screened=bool(on.value), left=int(left.value), off=bool(off.value))
 
     def centers(self):
         out = np.empty((self.k, self.d), np.float32)

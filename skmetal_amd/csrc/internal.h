@@ -35,12 +35,14 @@ struct LoopState {
     // fused steps (k <= 64): bit j set when a block of iteration i's fused
     // kernel labelled a row j: present[i & 1]
     unsigned long long present[2];
-    // the screened E-step: rows the last one left to the six products (added
-    // by k_assign3_list, taken and cleared by k_finalize_loop), the count
-    // above which the screen does not pay, and 1 once a step went past it
+    // the screened E-step: rows the step's left to the six products (from
+    // k_assign3_list or k_assign3_units; taken and cleared by the step's loop
+    // decision), the count above which the screen does not pay, 1 once a step
+    // went past it, and the count of the last step before that
     int unsure;
     int unsure_limit;
     int screen_off;
+    int left;
 };
 
 enum StepFlags : int {

@@ -1297,6 +1297,7 @@ __device__ __forceinline__ void loop_decision(const FinalizeArgs& a, int nch)
         st->done = done;
         // a step that left more rows than the screen is worth is the last
         // screened one of the run
+        if (st->screen_off == 0) st->left = st->unsure;
         if (st->unsure > st->unsure_limit) st->screen_off = 1;
         st->unsure = 0;
     }

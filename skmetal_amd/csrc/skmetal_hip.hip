@@ -718,6 +718,10 @@ struct Lloyd {
     // the six products, 1 screens every shape that the screen takes, 2 does so
     // and refuses the screen its memory (tests)
     bool screen_nomem = false;  // the device had no memory for the screen's buffers
+    // of the last run_loop: rows the last screened step left (-1: no step was
+    // screened), and whether the later steps took the six products alone
+    long run_left = -1;
+    bool run_off = false;
     bool screened() const
     {
         if (!split_on || !a3cap || screen_nomem || n >= (1L << 31) || (ld > 128 && k <= 128)) return false;
@@ -1032,6 +1036,8 @@ struct Lloyd {
             flags &= ~kStopStrict;
             tol = -1.0;  // no shift rule: sklearn's `shift <= tol` stops at tol = 0 on a zero shift
         }
+        run_left = -1;
+        run_off = false;
         LoopState hs{};
         hs.reloc_iter = -1;
         hs.unsure_limit = (int)std::min<long>(n / 2, 1L << 30);
@@ -1078,6 +1084,10 @@ struct Lloyd {
             }
             it += nb;
             batch = std::min<long>(batch * 2, fixed ? 1024 : 64);
+        }
+        if (screened() && fblocks == 0 && max_iter > 0) {
+            run_left = hs.left;
+            run_off = hs.screen_off != 0;
         }
         if (n_iter_out) *n_iter_out = max_iter > 0 ? hs.n_iter : 0;
         if (done_out) *done_out = final_done;
@@ -2034,6 +2044,18 @@ int skmetal_hip_lloyd_info(skmetal_hip_lloyd* h, int* fused, int* partials)
     const Lloyd& L = h->L;
     if (fused) *fused = (L.fblocks > 0 ? (L.split_on && L.f3cap ? 2 : 1) : 0) | (L.split_on && L.a3cap ? 4 : 0);
     if (partials) *partials = h->L.fblocks > 0 ? h->L.fblocks : h->L.sg.on ? (int)h->L.sg.nchunks : h->L.ug.R;
+    return 0;
+}
+
+int skmetal_hip_lloyd_screen_info(skmetal_hip_lloyd* h, int* screened, int64_t* left, int* off)
+{
+    Context& c = ctx();
+    Guard g(c);
+    if (!h) return fail(SKMETAL_EINVAL, "null pointer argument");
+    const Lloyd& L = h->L;
+    if (screened) *screened = L.fblocks == 0 && L.screened() ? 1 : 0;
+    if (left) *left = (int64_t)L.run_left;
+    if (off) *off = L.run_off ? 1 : 0;
     return 0;
 }
 

@@ -17,7 +17,7 @@ def _blobs(n, d, k, spread, seed):
     return X, np.ascontiguousarray(X[:k])
 
 
-def _both(monkeypatch, X, C, steps=5):
+def _both(monkeypatch, X, C, steps=5, center=True):
     from skmetal_amd import _bridge
 
     n, d = X.shape
@@ -28,17 +28,19 @@ def _both(monkeypatch, X, C, steps=5):
         lab = np.empty(n, np.int32)
         _bridge.kmeans_assign(X, C, lab, n, d, k)
         with _bridge.LloydHandle(n, d, k) as h:
-            h.load(X)
+            h.load(X, center=center)
             h.set_centers(C)
             run = h.run(steps, 0.0, strict=False)
             got.append((lab, run, h.centers(), h.labels()))
             assert h.info()["asplit"] and not h.info()["fused"]
+            info = h.screen_info()
+            assert info["screened"] == (mode == "1") and (info["left"] >= 0) == (mode == "1")
     (l0, r0, c0, f0), (l1, r1, c1, f1) = got
     np.testing.assert_array_equal(l0, l1)
     np.testing.assert_array_equal(f0, f1)
     np.testing.assert_array_equal(c0, c1)
     assert r0[0] == r1[0] and r0[1] == pytest.approx(r1[1], rel=1e-12)
-    return f1
+    return f1, info["left"], info["off"]
 
 
 # every K-step count, row ends off the 32-feature and 64-row grid, one stage
@@ -53,7 +55,26 @@ def _both(monkeypatch, X, C, steps=5):
     (212_000, 132, 20_000, 0.4),
 ])
 def test_screen_labels_match_six_products(monkeypatch, n, d, k, spread):
-    _both(monkeypatch, *_blobs(n, d, k, spread, n + d))
+    _, left, _ = _both(monkeypatch, *_blobs(n, d, k, spread, n + d))
+    assert left < 0.9 * n
+    assert left > 0 or n < 512  # (a few hundred rows around as many centres: all settled)
+
+
+# rows on centres far apart are settled, rows half way between two are not
+@pytest.mark.parametrize("n,d,k", [(20000, 48, 300), (5000, 128, 700), (20000, 160, 300), (3000, 600, 260)])
+@pytest.mark.parametrize("share", [0.0, 0.3, 1.0])
+def test_screen_settles_what_it_can(monkeypatch, n, d, k, share):
+    rng = np.random.default_rng(n)
+    C = rng.standard_normal((k, d)).astype(np.float32)
+    a, b = rng.integers(0, k, n), rng.integers(0, k, n)
+    X = C[a].copy()
+    mid = rng.random(n) < share
+    X[mid] = (0.5 * (C[a] + C[b]))[mid]
+    _, left, off = _both(monkeypatch, X, C, steps=1)
+    G = np.partition(X.astype(np.float64) @ C.T.astype(np.float64) - 0.5 * (C.astype(np.float64) ** 2).sum(1), -2, 1)
+    unsettled = (G[:, -1] - G[:, -2] < 1e-4).sum()  # (a third centre may be the nearest)
+    assert unsettled <= left <= unsettled + 0.1 * n
+    assert off == (left > n // 2)
 
 
 @pytest.mark.parametrize("d", [24, 150])
@@ -62,7 +83,7 @@ def test_screen_hard_data(monkeypatch, kind, d):
     X, C = _blobs(6000, d, 140, 0.5, 3)
     if kind == "duplicates":
         C[50], C[99] = C[3], C[0]  # ties: the lowest index wins
-    elif kind == "lattice":  # exact ties everywhere: the screen settles few rows and is turned off
+    elif kind == "lattice":  # exact ties all over
         rng = np.random.default_rng(4)
         X = rng.integers(0, 3, X.shape).astype(np.float32)
         C = rng.integers(0, 3, C.shape).astype(np.float32)
@@ -96,10 +117,10 @@ def test_screen_non_finite_centres(monkeypatch, d):
 def test_screen_relocation(monkeypatch, n, d, k):
     """Empty clusters: the farthest rows come from the screen's row minima and
     are those of the six products' minima."""
-    X, C = _blobs(n, d, k, 0.5, 8)
-    C[[4, 20, k - 1]] += 300.0
-    lab = _both(monkeypatch, X, C)
-    assert len(np.unique(lab)) == k
+    X, C = _blobs(n, d, k, 1.0, 8)
+    C[[4, 20, k - 1]] = C[0]  # ties: the lowest index takes the rows
+    lab, left, _ = _both(monkeypatch, X, C, steps=1)
+    assert len(np.unique(lab)) == k and 0 < left < n // 2
 
 
 # Every value rounds to bf16 by 2^-8 of itself, in the direction that moves the
@@ -120,7 +141,8 @@ def test_screen_worst_rounding(monkeypatch, d, scale):
     C[70], C[7] = c1, -c1
     C *= np.float32(2.0**scale)
     X = np.repeat(x[None], 1000, 0).astype(np.float32)
-    _both(monkeypatch, X, C, steps=1)
+    _, left, _ = _both(monkeypatch, X, C, steps=1, center=False)
+    assert left == len(X)
     from skmetal_amd import _bridge
 
     lab = np.empty(len(X), np.int32)  # with the screen
