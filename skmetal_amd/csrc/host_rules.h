@@ -48,4 +48,74 @@ inline size_t wide_part_floats(long rows, int k) { return size_t(rows) * ((size_
 // k_screen_wide's blocks for `rows` rows: whole turns of the XCDs.
 inline long wide_blocks(long rows, int k) { return ((rows + 255) / 256 + 7) / 8 * 8 * ((k + 255) / 256); }
 
+// Where the screen pays.  k_assign3 alone takes its 256-row blocks in rounds
+// of 256 (one a CU), each round proportional to the padded centres times
+// features (0.64 us per 1,000).  Rows of at most 128 floats: what is left
+// costs about one round again (nearly every block has a row) and the second
+// launch and its image 20 us, so it is the rounds after the first that are
+// saved.  Timed, a step without / with the screen: 64 floats, k = 1,024:
+// 60,000 rows 92 / 107 us, 120,000 134 / 111, 1,000,000 693 / 311; 128
+// floats, k = 256: 120,000 91 / 89, 250,000 144 / 114, 1,000,000 442 / 280.
+// Longer rows: the rest goes by units of 256 rows x 256 centres and costs
+// little, but there are two more launches.  768 floats, k = 1,500: 8,000 rows
+// 610 / 126; 300 floats: k = 600, 8,000 rows 161 / 87; k = 200, 130,000 rows
+// 158 / 142, 400,000 444 / 337; k = 512, 64,000 rows 150 / 124, 130,000 251 /
+// 175.  The slack grows with the norms: of blobs of 768 floats most rows are
+// left, and with at most two units of centres nothing is saved once
+// k_assign3's blocks fill half the CUs: k = 200, 130,000 rows 326 / 363,
+// 390,000 890 / 958; k = 400, 30,000 rows 242 / 183, 64,000 271 / 302,
+// 130,000 521 / 588.
+inline bool screen_pays(long n, int ld, int k)
+{
+    if (n >= (1L << 31) || k <= 128) return false;
+    if (ld > 512 && k <= 512 && n > 32768) return false;
+    const double round = (double)((k + 255) / 256 * 256) * ((ld + 31) / 32 * 32);
+    const double rounds = (double)((n + 65535) / 65536);
+    return ld <= 128 ? (rounds - 1) * round >= 60e3 : rounds * round >= 230e3;
+}
+
+// The E-step's time in us on 256 CUs, fitted to timings of 27 shapes (60,000 to
+// 1M rows of 32 to 128 floats, 4,000 to 400,000 of 200 to 1,000, 200 to 2,048
+// centres; within 15% but for rows of 32 floats).  plain: k_assign3, 14 us and
+// 4.3 to 4.7 for 32 features of 256 centres of a round of 256-row blocks.
+// screen: k_screen or k_screen_wide with the centres' images and the empty
+// launches behind it.  rest: the six products of the rows left; `passes` is
+// k_assign3_list's busiest block's, which k_assign3_units (long rows) has not:
+// its units of 64 centres (few rows) or 256 go round the CUs.
+inline double plain_us(long n, int ld, int k)
+{
+    const long rounds = (n + 65535) / 65536, steps = (long)((k + 255) / 256) * ((ld + 31) / 32);
+    return 14.0 + (ld <= 128 ? 4.7 : 4.3) * (double)(rounds * steps);
+}
+inline double screen_us(long n, int ld, int k)
+{
+    const double bytes = 4.0 * (double)n * ld;
+    if (ld <= 128) {
+        const double values = (double)n * ((k + 127) / 128 * 128), mac = values * ((ld + 31) / 32 * 32);
+        const double t = mac * 1.95e-9 > values * 8.8e-8 ? mac * 1.95e-9 : values * 8.8e-8;
+        return 26.0 + (t > bytes / 5.3e6 ? t : bytes / 5.3e6);
+    }
+    const double t = 2.4 * (double)((wide_blocks(n, k) + 255) / 256 * ((ld + 63) / 64));
+    return 35.0 + (t > bytes / 3.5e6 ? t : bytes / 3.5e6);
+}
+inline double rest_us(long n, int ld, int k, long left, long passes)
+{
+    const double step = 4.3 * 1.15 * ((ld + 31) / 32);
+    if (ld <= 128) return (double)passes * (plain_us(n, ld, k) - 14.0) / (double)((n + 65535) / 65536);
+    const long units = (left + 255) / 256 * ((k + 255) / 256);
+    return units * 2 <= 256 ? (units > 0 ? 0.35 * step : 0.0) : step * (double)((units + 255) / 256);
+}
+// Whether a step that left these rows took longer than without the screen.
+// Timed with the rows left spread evenly, without / with the screen, at the last
+// share before the line and the first past it: 1M x 128, k = 256 (9 passes of
+// 16) 338 / 285 and 336 / 319; 250,000 x 128, k = 256 (1 of 4) 96 / 65 and 95 /
+// 70; 1M x 64, k = 1,024 (11 of 16) 650 / 543 and 640 / 601; 400,000 x 300, k =
+// 200 (a third) 327 / 296 and 338 / 348; 64,000 x 768, k = 400 (half) 218 / 205
+// and 216 / 302; 100,000 x 768, k = 2,048 (nine tenths) 1,544 / 1,396 and 1,545
+// / 1,647.  Rows left in one stretch, a tenth of 1M x 128: 338 / 404.
+inline bool screen_lost(long n, int ld, int k, long left, long passes)
+{
+    return screen_us(n, ld, k) + rest_us(n, ld, k, left, passes) > 0.98 * plain_us(n, ld, k);
+}
+
 }  // namespace skm

@@ -35,14 +35,13 @@ struct LoopState {
     // fused steps (k <= 64): bit j set when a block of iteration i's fused
     // kernel labelled a row j: present[i & 1]
     unsigned long long present[2];
-    // the screened E-step: rows the step's left to the six products (from
-    // k_assign3_list or k_assign3_units; taken and cleared by the step's loop
-    // decision), the count above which the screen does not pay, 1 once a step
-    // went past it, and the count of the last step before that
+    // the screened E-step: rows left to the six products, and the 256-row
+    // passes that k_assign3_list's busiest block took over them; the step's
+    // loop decision clears them and keeps the last values for the host
     int unsure;
-    int unsure_limit;
-    int screen_off;
+    int passes;
     int left;
+    int left_passes;
 };
 
 enum StepFlags : int {
@@ -96,8 +95,7 @@ hipError_t launch_assign3(const AssignArgs& a, int num_cu, hipStream_t s);
 // launch_assign3_list (a.img), before both.
 hipError_t launch_centre_images(const AssignArgs& a, char* simg, hipStream_t s);
 // k_assign3 for the rows that k_screen left (screen_kernels.hip): bit r of
-// masks[i] set, row 64 i + r.  With a.state's screen_off set every row is
-// taken.  The rows taken are added to state->unsure.
+// masks[i] set, row 64 i + r.  The rows taken are added to state->unsure.
 hipError_t launch_assign3_list(const AssignArgs& a, const unsigned long long* masks, int num_cu, hipStream_t s);
 
 // The same for rows of more than 128 floats: the images of launch_screen_wide
@@ -142,32 +140,6 @@ struct WideArgs {
 };
 size_t wide_image_bytes(int k, int ld);
 hipError_t launch_screen_wide(const WideArgs& a, hipStream_t s);
-
-// Where the screen pays.  k_assign3 alone takes its 256-row blocks in rounds
-// of 256 (one a CU), each round proportional to the padded centres times
-// features (0.64 us per 1,000).  Rows of at most 128 floats: what is left
-// costs about one round again (nearly every block has a row) and the second
-// launch and its image 20 us, so it is the rounds after the first that are
-// saved.  Timed, a step without / with the screen: 64 floats, k = 1,024:
-// 60,000 rows 92 / 107 us, 120,000 134 / 111, 1,000,000 693 / 311; 128
-// floats, k = 256: 120,000 91 / 89, 250,000 144 / 114, 1,000,000 442 / 280.
-// Longer rows: the rest goes by units of 256 rows x 256 centres and costs
-// little, but there are two more launches.  768 floats, k = 1,500: 8,000 rows
-// 610 / 126; 300 floats: k = 600, 8,000 rows 161 / 87; k = 200, 130,000 rows
-// 158 / 142, 400,000 444 / 337; k = 512, 64,000 rows 150 / 124, 130,000 251 /
-// 175.  The slack grows with the norms: of blobs of 768 floats most rows are
-// left, and with at most two units of centres nothing is saved once
-// k_assign3's blocks fill half the CUs: k = 200, 130,000 rows 326 / 363,
-// 390,000 890 / 958; k = 400, 30,000 rows 242 / 183, 64,000 271 / 302,
-// 130,000 521 / 588.
-inline bool screen_pays(long n, int ld, int k)
-{
-    if (n >= (1L << 31) || k <= 128) return false;
-    if (ld > 512 && k <= 512 && n > 32768) return false;
-    const double round = (double)((k + 255) / 256 * 256) * ((ld + 31) / 32 * 32);
-    const double rounds = (double)((n + 65535) / 65536);
-    return ld <= 128 ? (rounds - 1) * round >= 60e3 : rounds * round >= 230e3;
-}
 
 // The three-part bf16 split is exact for finite values of magnitude >= 2^-103,
 // and the E-step's smallest kept part products stay normal fp32 numbers when

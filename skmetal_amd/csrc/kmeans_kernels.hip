@@ -1295,11 +1295,10 @@ __device__ __forceinline__ void loop_decision(const FinalizeArgs& a, int nch)
             done = 2;
         if (done != 0) st->halt_iter = a.iter;
         st->done = done;
-        // a step that left more rows than the screen is worth is the last
-        // screened one of the run
-        if (st->screen_off == 0) st->left = st->unsure;
-        if (st->unsure > st->unsure_limit) st->screen_off = 1;
+        st->left = st->unsure;
+        st->left_passes = st->passes;
         st->unsure = 0;
+        st->passes = 0;
     }
 }
 

@@ -109,8 +109,7 @@ __global__ __launch_bounds__(64 * screen_waves(NK), screen_waves(NK) / 4) void k
     using G = ScreenGeom<NK>;
     constexpr int NW = screen_waves(NK);
     constexpr bool PIPE = true;
-    const LoopState* st = a.state;
-    if (st != nullptr && (st->done != 0 || st->screen_off != 0)) return;
+    if (a.state != nullptr && a.state->done != 0) return;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     __shared__ int sChg;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -357,8 +356,7 @@ static hipError_t launch_screen_nk(const ScreenArgs& a, int num_cu, hipStream_t 
 // image come from its L2.  A launch takes wide_rows rows.
 __global__ __launch_bounds__(512, 2) void k_screen_wide(WideArgs a)
 {
-    const LoopState* st = a.state;
-    if (st != nullptr && (st->done != 0 || st->screen_off != 0)) return;
+    if (a.state != nullptr && a.state->done != 0) return;
     const int ncg = (a.k + 255) / 256, nks = (a.ld + 63) / 64;
     const long nrb = (a.n + 255) / 256;
     const long i = blockIdx.x >> 3;
@@ -512,15 +510,9 @@ __global__ __launch_bounds__(512, 2) void k_screen_wide(WideArgs a)
 // its place on the list.
 __global__ __launch_bounds__(256) void k_screen_merge(WideArgs a)
 {
-    const LoopState* st = a.state;
-    if (st != nullptr && st->done != 0) return;
-    const bool all = st != nullptr && st->screen_off != 0;
+    if (a.state != nullptr && a.state->done != 0) return;
     constexpr unsigned long long kNone = 0xff800000ull << 32;  // +inf in order_bits's form, centre 0
     const long row = (long)blockIdx.x * 256 + threadIdx.x;
-    if (all) {
-        if (row < a.n) a.keys[row] = kNone;
-        return;
-    }
     __shared__ unsigned sMax;
     __shared__ int sChg, sLeft, sAt;
     const int tid = threadIdx.x;

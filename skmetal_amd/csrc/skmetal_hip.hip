@@ -721,13 +721,18 @@ struct Lloyd {
     // of the last run_loop: rows the last screened step left (-1: no step was
     // screened), and whether the later steps took the six products alone
     long run_left = -1;
+    long run_passes = 0;  // LoopState::left_passes beside run_left
     bool run_off = false;
+    static int screen_switch()  // -1: by the rules
+    {
+        const char* e = getenv("SKMETAL_HIP_SCREEN");
+        return e != nullptr && e[0] >= '0' && e[0] <= '2' ? e[0] - '0' : -1;
+    }
     bool screened() const
     {
-        if (!split_on || !a3cap || screen_nomem || n >= (1L << 31) || (ld > 128 && k <= 128)) return false;
-        const char* e = getenv("SKMETAL_HIP_SCREEN");
-        if (e != nullptr && e[0] >= '0' && e[0] <= '2') return e[0] != '0';
-        return screen_pays(n, ld, k);
+        if (!split_on || !a3cap || screen_nomem || run_off || n >= (1L << 31) || (ld > 128 && k <= 128)) return false;
+        const int sw = screen_switch();
+        return sw >= 0 ? sw > 0 : screen_pays(n, ld, k);
     }
 
     // The screen's buffers.  Without memory for them the handle stays on the
@@ -735,8 +740,7 @@ struct Lloyd {
     int screen_buffers()
     {
         if (simg != nullptr) return 0;
-        const char* e = getenv("SKMETAL_HIP_SCREEN");
-        const size_t more = e != nullptr && e[0] == '2' ? size_t(1) << 50 : 0;
+        const size_t more = screen_switch() == 2 ? size_t(1) << 50 : 0;
         const int rc = ld > 128 ? grab_workspace({{(void**)&spart, wide_part_floats(wide_rows(n, k), k) * sizeof(float)},
                                                   {(void**)&sxx, size_t(wide_rows(n, k)) * sizeof(float)},
                                                   {(void**)&slist, size_t(n) * sizeof(unsigned)},
@@ -782,7 +786,8 @@ struct Lloyd {
     // The final E-step with the inertia of its labels: on the split path one
     // pass over X (k_assign3 adds each row's distance to its new centre into
     // per-block totals, k_rowdist_total adds those), else the E-step and then
-    // the row-distance pass.
+    // the row-distance pass.  (Behind the screen too: the distances cost
+    // k_assign3 as much as that pass, 170 and 145 us at 1M x 128.)
     int assign_inertia(const float* cents, double* out)
     {
         const long blocks = std::min<long>(C->num_cu, (n + 255) / 256);
@@ -1037,10 +1042,11 @@ struct Lloyd {
             tol = -1.0;  // no shift rule: sklearn's `shift <= tol` stops at tol = 0 on a zero shift
         }
         run_left = -1;
+        run_passes = 0;
         run_off = false;
         LoopState hs{};
         hs.reloc_iter = -1;
-        hs.unsure_limit = (int)std::min<long>(n / 2, 1L << 30);
+        hs.left = -1;
         // the reset is a kernel on the stream: nothing waits for the host
         HIP_TRY(launch_state_reset(st, hs, s), "state reset launch");
         HIP_TRY(hipMemsetAsync(labels, 0xff, size_t(n) * sizeof(int), s), "hipMemsetAsync(labels)");
@@ -1049,8 +1055,12 @@ struct Lloyd {
         // back after each: a halt (convergence, or more empty clusters than
         // k_reloc takes, which the host relocates) then skips at most one
         // batch of launches.  A fixed-iteration run has no convergence stop:
-        // with the relocation in-stream it is one batch.
-        long batch = fixed ? (reloc_inline ? max_iter : 8) : 4;
+        // with the relocation in-stream it is one batch.  Screened steps: two
+        // first, whose last tells whether the screen pays on this data (the
+        // first step's rows left say little: from rows of X as centres they
+        // are many more than from the means that follow).
+        bool look = fblocks == 0 && screened();
+        long batch = look ? 2 : fixed ? (reloc_inline ? max_iter : 8) : 4;
         int final_done = 0;
         while (it < max_iter) {
             const long nb = std::min(batch, max_iter - it);
@@ -1058,6 +1068,11 @@ struct Lloyd {
             for (long t = it; t < it + nb; ++t) TRY(enqueue_step((int)t, tol, flags, t > it, t + 1 == it + nb));
             if (batch_end) HIP_TRY(hipEventRecord(batch_end, s), "hipEventRecord");
             TRY(read_state(&hs));
+            if (fblocks == 0 && screened()) {
+                run_left = hs.left;
+                run_passes = hs.left_passes;
+                run_off = screen_switch() < 0 && screen_lost(n, ld, k, run_left, run_passes);
+            }
             if (hs.done == 3) {
                 const int t = hs.halt_iter;
                 const int old = (c0 + (t - (int)it)) & 1;
@@ -1083,11 +1098,8 @@ struct Lloyd {
                 break;
             }
             it += nb;
-            batch = std::min<long>(batch * 2, fixed ? 1024 : 64);
-        }
-        if (screened() && fblocks == 0 && max_iter > 0) {
-            run_left = hs.left;
-            run_off = hs.screen_off != 0;
+            batch = !look ? std::min<long>(batch * 2, fixed ? 1024 : 64) : fixed && reloc_inline ? max_iter : 4;
+            look = false;
         }
         if (n_iter_out) *n_iter_out = max_iter > 0 ? hs.n_iter : 0;
         if (done_out) *done_out = final_done;
@@ -2053,7 +2065,7 @@ int skmetal_hip_lloyd_screen_info(skmetal_hip_lloyd* h, int* screened, int64_t* 
     Guard g(c);
     if (!h) return fail(SKMETAL_EINVAL, "null pointer argument");
     const Lloyd& L = h->L;
-    if (screened) *screened = L.fblocks == 0 && L.screened() ? 1 : 0;
+    if (screened) *screened = L.fblocks == 0 && (L.screened() || L.run_off) ? 1 : 0;
     if (left) *left = (int64_t)L.run_left;
     if (off) *off = L.run_off ? 1 : 0;
     return 0;

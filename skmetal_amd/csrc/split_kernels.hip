@@ -1098,9 +1098,11 @@ __global__ __launch_bounds__(512, 1) void k_assign3(const float* __restrict__ X,
 // k_assign3 for the rows that k_screen left.  Block b takes a contiguous
 // share of the rows: it turns their mask bits into a list in LDS, 2,048 rows'
 // bits at a time until 256 rows are on it, and runs the six products for 256
-// rows of the list (32 per wave) at a time.  Once the screen is off every
-// row is taken.  The list keeps the blocks' work even while rows are left
-// all over X; a share with few rows costs a block one pass over the centres.
+// rows of the list (32 per wave) at a time.  The list keeps the blocks' work
+// even while rows are left all over X; a share with few rows costs a block one
+// pass over the centres.  Rows left all in one stretch of X are a few blocks'
+// work and take as long as k_assign3 does for all rows, so the busiest block's
+// passes go to the state beside the count.
 template <int CB>
 __global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict__ X, long n, int ld,
                                                          const char* __restrict__ img, int k,
@@ -1109,7 +1111,6 @@ __global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict
                                                          const unsigned long long* __restrict__ masks)
 {
     if (st != nullptr && st->done != 0) return;
-    const bool all = st != nullptr && st->screen_off != 0;
     using G = Assign3Geom<CB>;
     constexpr int CPC = G::CPC, SEG = G::SEG;
     constexpr int CH = 2048;  // rows whose bits are listed at a time, 256 per wave
@@ -1171,7 +1172,7 @@ __global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict
             for (int j = 0; j < 4; ++j) {
                 const long q = c + 256 * wave + 64 * j;
                 const long left = r1 - q;
-                m[j] = left <= 0 ? 0ull : all ? (left >= 64 ? ~0ull : (1ull << left) - 1ull) : masks[q >> 6];
+                m[j] = left <= 0 ? 0ull : masks[q >> 6];
                 mine += (int)__popcll(m[j]);
             }
             if (lane == 0) sCnt[wave] = mine;
@@ -1241,12 +1242,14 @@ __global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict
         __syncthreads();
         if (tid == 0 && sChg != 0) atomicAdd(changed, sChg);
     }
-    if (st != nullptr && !all && tid == 0 && taken != 0) atomicAdd(&st->unsure, taken);
+    if (st != nullptr && tid == 0 && taken != 0) {
+        atomicAdd(&st->unsure, taken);
+        atomicMax(&st->passes, (taken + 255) / 256);
+    }
 }
 
 // k_assign3 split over the centres as well, for long rows: a unit is 256 rows
-// (of the list that k_screen_merge left, or, once the screen is off, of X)
-// against one pass of 256 centres, and its row minima meet in `keys` by a
+// (of the list that k_screen_merge left) against one pass of 256 centres, and its row minima meet in `keys` by a
 // 64-bit minimum of (distance, centre) -- the first minimum over all centres,
 // in any order of the units.  With 768 floats a row 256 rows against 2,048
 // centres keep a CU busy for 0.8 ms, so a few hundred rows left all over X
@@ -1272,7 +1275,7 @@ struct UnitGeom {
 template <int CB>
 __device__ __forceinline__ void assign3_units(const float* __restrict__ X, int ld, const char* __restrict__ img,
                                               const float* __restrict__ cnorm, int k,
-                                              const unsigned* __restrict__ list, bool all, long cnt,
+                                              const unsigned* __restrict__ list, long cnt,
                                               unsigned long long* __restrict__ keys, char* smem)
 {
     using A = Assign3Geom<16>;
@@ -1313,7 +1316,7 @@ __device__ __forceinline__ void assign3_units(const float* __restrict__ X, int l
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
             const long q = min(b0 + 16 * g, cnt - 1);
-            xp[g] = X + (all ? q : (long)list[q]) * ld;
+            xp[g] = X + (long)list[q] * ld;
         }
     };
     // past the row's end its first values meet zero centre parts
@@ -1389,10 +1392,7 @@ __device__ __forceinline__ void assign3_units(const float* __restrict__ X, int l
                 key = o < key ? o : key;
             }
             const long q = row0 + 16 * g + r16;
-            if (h == g && q < cnt && (key >> 32) < order_bits(INFINITY)) {
-                const long row = all ? q : (long)list[q];
-                atomicMin(&keys[row], key);
-            }
+            if (h == g && q < cnt && (key >> 32) < order_bits(INFINITY)) atomicMin(&keys[list[q]], key);
         }
         if (!more) break;
         i = nx;
@@ -1401,7 +1401,7 @@ __device__ __forceinline__ void assign3_units(const float* __restrict__ X, int l
 
 // Units of 256 centres, or of 64 while those would leave half the CUs without
 // one: a unit's K steps are a chain of 12 us per 100 features at 256 centres.
-__global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restrict__ X, long n, int ld,
+__global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restrict__ X, int ld,
                                                           const char* __restrict__ img,
                                                           const float* __restrict__ cnorm, int k,
                                                           const unsigned* __restrict__ list, const int* nlist,
@@ -1409,28 +1409,26 @@ __global__ __launch_bounds__(512, 1) void k_assign3_units(const float* __restric
 {
     if (st != nullptr && st->done != 0) return;
     extern __shared__ __attribute__((aligned(1024))) char smem[];  // two stages
-    const bool all = st != nullptr && st->screen_off != 0;
-    const long cnt = all ? n : (long)*nlist;
-    if (st != nullptr && !all && blockIdx.x == 0 && threadIdx.x == 0) st->unsure = (int)min(cnt, 0x7fffffffL);
+    const long cnt = *nlist;
+    if (st != nullptr && blockIdx.x == 0 && threadIdx.x == 0) st->unsure = (int)cnt;
     if ((cnt + 255) / 256 * ((k + 255) / 256) * 2 <= (long)gridDim.x)
-        assign3_units<4>(X, ld, img, cnorm, k, list, all, cnt, keys, smem);
+        assign3_units<4>(X, ld, img, cnorm, k, list, cnt, keys, smem);
     else
-        assign3_units<16>(X, ld, img, cnorm, k, list, all, cnt, keys, smem);
+        assign3_units<16>(X, ld, img, cnorm, k, list, cnt, keys, smem);
 }
 
 // The labels of the units' rows from their keys.
-__global__ __launch_bounds__(256) void k_units_finish(long n, const unsigned* __restrict__ list, const int* nlist,
+__global__ __launch_bounds__(256) void k_units_finish(const unsigned* __restrict__ list, const int* nlist,
                                                       const unsigned long long* __restrict__ keys,
                                                       int* __restrict__ labels, LoopState* st, int* changed)
 {
     if (st != nullptr && st->done != 0) return;
-    const bool all = st != nullptr && st->screen_off != 0;
-    const long cnt = all ? n : (long)*nlist;
+    const long cnt = *nlist;
     __shared__ int sChg;
     if (threadIdx.x == 0) sChg = 0;
     __syncthreads();
     for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < cnt; q += (long)gridDim.x * 256) {
-        const long row = all ? q : (long)list[q];
+        const long row = list[q];
         const int lab = (int)(unsigned)keys[row];
         if (changed != nullptr && labels[row] != lab) atomicAdd(&sChg, 1);
         labels[row] = lab;
@@ -1596,10 +1594,10 @@ hipError_t launch_assign3_units(const AssignArgs& a, const unsigned* list, const
     const long units = (a.n + 255) / 256 * ((a.k + 255) / 256) * 4;
     long blocks = num_cu < units ? num_cu : units;
     blocks = (blocks + 7) / 8 * 8;
-    hipLaunchKernelGGL(k_assign3_units, dim3((unsigned)blocks), dim3(512), 2 * UnitGeom<16>::STAGE, s, a.X, a.n,
-                       a.ld, a.img, a.cnorm, a.k, list, nlist, a.state, keys);
+    hipLaunchKernelGGL(k_assign3_units, dim3((unsigned)blocks), dim3(512), 2 * UnitGeom<16>::STAGE, s, a.X, a.ld,
+                       a.img, a.cnorm, a.k, list, nlist, a.state, keys);
     const long fb = (a.n + 255) / 256;
-    hipLaunchKernelGGL(k_units_finish, dim3((unsigned)(fb < num_cu ? fb : num_cu)), dim3(256), 0, s, a.n, list, nlist,
+    hipLaunchKernelGGL(k_units_finish, dim3((unsigned)(fb < num_cu ? fb : num_cu)), dim3(256), 0, s, list, nlist,
                        keys, a.labels, a.state, a.changed);
     return hipGetLastError();
 }

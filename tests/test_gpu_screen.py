@@ -40,7 +40,8 @@ def _both(monkeypatch, X, C, steps=5, center=True):
     np.testing.assert_array_equal(f0, f1)
     np.testing.assert_array_equal(c0, c1)
     assert r0[0] == r1[0] and r0[1] == pytest.approx(r1[1], rel=1e-12)
-    return f1, info["left"], info["off"]
+    assert not info["off"]
+    return f1, info["left"]
 
 
 # every K-step count, row ends off the 32-feature and 64-row grid, one stage
@@ -55,7 +56,7 @@ def _both(monkeypatch, X, C, steps=5, center=True):
     (212_000, 132, 20_000, 0.4),
 ])
 def test_screen_labels_match_six_products(monkeypatch, n, d, k, spread):
-    _, left, _ = _both(monkeypatch, *_blobs(n, d, k, spread, n + d))
+    _, left = _both(monkeypatch, *_blobs(n, d, k, spread, n + d))
     assert left < 0.9 * n
     assert left > 0 or n < 512  # (a few hundred rows around as many centres: all settled)
 
@@ -70,11 +71,10 @@ def test_screen_settles_what_it_can(monkeypatch, n, d, k, share):
     X = C[a].copy()
     mid = rng.random(n) < share
     X[mid] = (0.5 * (C[a] + C[b]))[mid]
-    _, left, off = _both(monkeypatch, X, C, steps=1)
+    _, left = _both(monkeypatch, X, C, steps=1)
     G = np.partition(X.astype(np.float64) @ C.T.astype(np.float64) - 0.5 * (C.astype(np.float64) ** 2).sum(1), -2, 1)
     unsettled = (G[:, -1] - G[:, -2] < 1e-4).sum()  # (a third centre may be the nearest)
     assert unsettled <= left <= unsettled + 0.1 * n
-    assert off == (left > n // 2)
 
 
 @pytest.mark.parametrize("d", [24, 150])
@@ -119,7 +119,7 @@ def test_screen_relocation(monkeypatch, n, d, k):
     are those of the six products' minima."""
     X, C = _blobs(n, d, k, 1.0, 8)
     C[[4, 20, k - 1]] = C[0]  # ties: the lowest index takes the rows
-    lab, left, _ = _both(monkeypatch, X, C, steps=1)
+    lab, left = _both(monkeypatch, X, C, steps=1)
     assert len(np.unique(lab)) == k and 0 < left < n // 2
 
 
@@ -141,7 +141,7 @@ def test_screen_worst_rounding(monkeypatch, d, scale):
     C[70], C[7] = c1, -c1
     C *= np.float32(2.0**scale)
     X = np.repeat(x[None], 1000, 0).astype(np.float32)
-    _, left, _ = _both(monkeypatch, X, C, steps=1, center=False)
+    _, left = _both(monkeypatch, X, C, steps=1, center=False)
     assert left == len(X)
     from skmetal_amd import _bridge
 
@@ -173,3 +173,45 @@ def test_screen_without_memory(monkeypatch, n, d, k):
     for other in got[1:]:
         for a, b in zip(got[0], other):
             np.testing.assert_array_equal(a, b)
+
+
+# Without the switch a run keeps the screen while it pays: on rows that it
+# settles; not on rows far from the origin, whose norms make its bound useless;
+# nor where the rows it leaves lie in one stretch of X (with rows of at most 128
+# floats a few blocks' work).  Labels and centres are those of the six products
+# either way.
+@pytest.mark.parametrize("n,d,k", [(135_000, 128, 260), (70_000, 200, 520), (9_000, 400, 1100)])
+@pytest.mark.parametrize("kind", ["settled", "far", "stretch"])
+def test_screen_stays_while_it_pays(monkeypatch, n, d, k, kind):
+    from skmetal_amd import _bridge
+
+    rng = np.random.default_rng(n)
+    C = rng.standard_normal((k, d)).astype(np.float32)
+    a, b = rng.integers(0, k, n), rng.integers(0, k, n)
+    X = C[a] + 0.02 * rng.standard_normal((n, d), dtype=np.float32)
+    X[:k] = C
+    if kind == "far":
+        X, C = X + np.float32(100), C + np.float32(100)
+    elif kind == "stretch":
+        some = slice(k, k + n // 10)
+        X[some] = 0.5 * (C[a[some]] + C[b[some]])
+    got = []
+    for mode in ("0", None):
+        monkeypatch.setenv("SKMETAL_HIP_SCREEN", mode) if mode else monkeypatch.delenv("SKMETAL_HIP_SCREEN")
+        with _bridge.LloydHandle(n, d, k) as h:
+            h.load(X, center=False)
+            h.set_centers(C)
+            h.iterate(7)
+            mid = h.labels(), h.centers(), h.screen_info()["off"]
+            h.set_centers(C)
+            run = h.run(7, 0.0, strict=False)
+            got.append((mid[0], mid[1], h.labels(), h.centers(), np.array(run[:1])))
+            info = h.screen_info()
+            assert info["screened"] == (mode is None)
+    for x, y in zip(*got):
+        np.testing.assert_array_equal(x, y)
+    # (9,000 rows of 1,100 centres: the units spread the work over the CUs, which
+    # k_assign3 does not, and all of the rows take less than without the screen)
+    lost = {"settled": False, "far": n != 9_000, "stretch": d <= 128}[kind]
+    assert info["off"] == mid[2] == lost
+    assert (info["left"] == n) == (kind == "far") and (info["left"] > 0) == (kind != "settled")

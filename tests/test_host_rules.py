@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import ctypes
+import math
 import subprocess
 from pathlib import Path
 
@@ -44,6 +45,7 @@ extern "C" int workspace(int fails)
         if (p[i] != mem + i + 1) return 6;
     return 0;
 }
+extern "C" bool lost(long n, int ld, int k, long left, long passes) { return screen_lost(n, ld, k, left, passes); }
 extern "C" long rows(long n, int k) { return wide_rows(n, k); }
 extern "C" long blocks(long rows, int k) { return wide_blocks(rows, k); }
 extern "C" long part_bytes(long rows, int k) { return (long)wide_part_floats(rows, k) * 4; }
@@ -57,6 +59,8 @@ def rules(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}", str(d / "rules.cpp"),
                     "-o", str(d / "rules.so")], check=True)
     lib = ctypes.CDLL(str(d / "rules.so"))
+    lib.lost.argtypes = [ctypes.c_long, ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_long]
+    lib.lost.restype = ctypes.c_bool
     for f in (lib.rows, lib.blocks, lib.part_bytes):
         f.argtypes, f.restype = [ctypes.c_long, ctypes.c_int], ctypes.c_long
     return lib
@@ -78,3 +82,27 @@ def test_the_wide_screen_in_launches_that_hip_takes(rules, n, k):
     assert rules.part_bytes(rows, k) == rows * ((k + 255) // 256) * 16 <= 2**28
     # (the rows of a launch: their blocks cover them, 256 a block and 256 centres)
     assert rules.blocks(rows, k) * 256 >= rows * ((k + 255) // 256)
+
+
+# what steps took without and with the screen (us), the rows left evenly over X,
+# where the two differ by a tenth or more
+@pytest.mark.parametrize("n,ld,k,share,plain,screened", [
+    (1_000_000, 128, 256, 0.4, 340, 260), (1_000_000, 128, 256, 0.9, 339, 416), (250_000, 128, 256, 0.2, 95, 70),
+    (250_000, 128, 256, 0.6, 95, 106), (1_000_000, 64, 1024, 0.6, 650, 543), (1_000_000, 64, 1024, 0.9, 640, 716),
+    (120_000, 64, 1024, 0.2, 98, 86), (120_000, 64, 1024, 0.5, 98, 116), (300_000, 32, 1024, 0.3, 136, 100),
+    (200_000, 128, 2048, 0.6, 562, 489), (200_000, 128, 2048, 0.9, 563, 628), (400_000, 300, 200, 0.2, 329, 290),
+    (400_000, 300, 200, 0.5, 330, 399), (64_000, 768, 400, 0.3, 215, 194), (64_000, 768, 400, 0.6, 216, 302),
+    (130_000, 512, 512, 0.4, 297, 273), (130_000, 512, 512, 0.6, 301, 351), (100_000, 768, 2048, 0.6, 1511, 1270),
+    (8_000, 768, 1500, 0.9, 541, 176), (20_000, 400, 600, 0.9, 156, 112), (390_000, 768, 200, 0.2, 643, 510),
+    (390_000, 768, 200, 0.6, 647, 750), (50_000, 200, 1000, 0.2, 136, 118), (50_000, 200, 1000, 0.6, 137, 159),
+])
+def test_the_screen_is_kept_where_it_was_faster(rules, n, ld, k, share, plain, screened):
+    block = ((n + 255) // 256 + 63) // 64 * 64  # rows of a block's share
+    busiest = share * block + 2.8 * math.sqrt(share * (1 - share) * block)  # of 256 blocks
+    assert rules.lost(n, ld, k, int(share * n), math.ceil(busiest / 256)) == (screened > plain)
+
+
+def test_rows_left_in_one_stretch(rules):
+    # a tenth of 1M x 128: 338 without the screen, 404 with it
+    assert rules.lost(1_000_000, 128, 256, 100_000, 16)
+    assert not rules.lost(1_000_000, 128, 256, 100_000, 2)
