@@ -755,23 +755,29 @@ struct Lloyd {
         return 0;
     }
 
+    // The labels of all rows, or of rows [r0, r0 + rows).
     int assign(const float* cents, LoopState* state, int* changed, bool minima = false)
     {
-        AssignArgs a{X, n, ld, cents, cnorm, k, labels, state, changed, nullptr};
+        return assign_rows(cents, state, changed, minima, 0, n);
+    }
+    int assign_rows(const float* cents, LoopState* state, int* changed, bool minima, long r0, long rows)
+    {
+        AssignArgs a{X + r0 * ld, rows, ld, cents, cnorm, k, labels + r0, state, changed, nullptr};
         if (split_on && a3cap) {
             if (a3img == nullptr) TRY(grab((void**)&a3img, assign3_image_bytes(k, ld)));
             a.img = a3img;
             if (minima) a.emin = emin;
             if (screened()) TRY(screen_buffers());
             if (screened() && ld > 128) {
-                const WideArgs wa{X, n, ld, cnorm, k, labels, state, changed, simg, spart, sxx, slist, snlist, smask};
+                const WideArgs wa{a.X, rows, ld, cnorm, k, a.labels, state, changed, simg, spart, sxx, slist, snlist,
+                                  smask};
                 HIP_TRY(launch_wide_images(a, simg, snlist, s), "centre image launch");
                 HIP_TRY(launch_screen_wide(wa, s), "screen launch");
                 HIP_TRY(launch_assign3_units(a, slist, snlist, smask, C->num_cu, s), "assign launch");
                 return 0;
             }
             if (screened()) {
-                const ScreenArgs sa{X, n, ld, k, labels, state, changed, simg, a.emin, smask};
+                const ScreenArgs sa{a.X, rows, ld, k, a.labels, state, changed, simg, a.emin, smask};
                 HIP_TRY(launch_centre_images(a, simg, s), "centre image launch");
                 HIP_TRY(launch_screen(sa, C->num_cu, s), "screen launch");
                 HIP_TRY(launch_assign3_list(a, smask, C->num_cu, s), "assign launch");
@@ -781,6 +787,26 @@ struct Lloyd {
         } else
             HIP_TRY(launch_assign(a, C->num_cu, s), "assign launch");
         return 0;
+    }
+
+    // An E-step by itself, with no steps before it that tell whether the screen
+    // pays on this data: its first rows do, a round of k_assign3's blocks or (to
+    // 8,192 rows) of k_screen_wide's.  On rows that the screen does not settle a
+    // call from host rows takes, before / now / without the screen: 100,000 x
+    // 768, k = 2,048 8.56 / 8.36 / 8.24 ms; 1M x 64, k = 8,192 12.4 / 11.3 / 11.1;
+    // on rows that it does 6.99 / 6.98 / 8.32 and 6.90 / 6.81 / 11.5.
+    int assign_once(const float* cents)
+    {
+        const long ncg = (k + 255) / 256;
+        const long part = ld <= 128 ? 65536 : std::min(8192L, std::max(2048L, 65536 / ncg / 2048 * 2048));
+        if (!screened() || screen_switch() > 0 || n < 4 * part) return assign(cents, nullptr, nullptr);
+        LoopState hs{};
+        HIP_TRY(launch_state_reset(st, hs, s), "state reset launch");
+        TRY(assign_rows(cents, st, nullptr, false, 0, part));
+        TRY(read_state(&hs));
+        const double share = (double)hs.unsure / (double)part;
+        run_off = screen_lost(n, ld, k, (long)(share * (double)n), (long)std::ceil(share * (double)((n + 65535) / 65536)));
+        return assign_rows(cents, nullptr, nullptr, false, part, n - part);
     }
 
     // The final E-step with the inertia of its labels: on the split path one
@@ -1502,7 +1528,7 @@ int skmetal_kmeans_assign(const void* X, const void* centroids, void* assignment
     TRY(L.create(&c, (long)n, (int)d, (int)k));
     TRY(L.load_X(static_cast<const float*>(X), false));
     TRY(L.set_centers(static_cast<const float*>(centroids)));
-    TRY(L.assign(L.cen[L.cur], nullptr, nullptr));
+    TRY(L.assign_once(L.cen[L.cur]));
     TRY(L.get_labels(static_cast<int32_t*>(assignments)));
     return 0;
 }

@@ -215,3 +215,28 @@ def test_screen_stays_while_it_pays(monkeypatch, n, d, k, kind):
     lost = {"settled": False, "far": n != 9_000, "stretch": d <= 128}[kind]
     assert info["off"] == mid[2] == lost
     assert (info["left"] == n) == (kind == "far") and (info["left"] > 0) == (kind != "settled")
+
+
+# An E-step by itself looks at its first rows and takes the rest with or without
+# the screen: the six products' labels for rows that are settled, that are not,
+# and where the first rows are of the other kind than the rest.
+@pytest.mark.parametrize("n,d,k", [(262_200, 40, 300), (33_000, 300, 520)])
+@pytest.mark.parametrize("first,rest", [("near", "near"), ("far", "far"), ("near", "far"), ("far", "near")])
+def test_screen_in_an_e_step_by_itself(monkeypatch, n, d, k, first, rest):
+    from skmetal_amd import _bridge
+
+    rng = np.random.default_rng(n)
+    C = rng.standard_normal((k, d)).astype(np.float32)
+    a, b = rng.integers(0, k, n), rng.integers(0, k, n)
+    X = C[a] + 0.02 * rng.standard_normal((n, d), dtype=np.float32)
+    part = 65536 if d <= 128 else 8192  # (at up to 8 groups of 256 centres)
+    for rows, kind in ((slice(0, part), first), (slice(part, n), rest)):
+        if kind == "far":
+            X[rows] = 0.5 * (C[a[rows]] + C[b[rows]])
+    lab = [np.empty(n, np.int32) for _ in range(2)]
+    monkeypatch.setenv("SKMETAL_HIP_SCREEN", "0")
+    _bridge.kmeans_assign(X, C, lab[0], n, d, k)
+    monkeypatch.delenv("SKMETAL_HIP_SCREEN")
+    _bridge.kmeans_assign(X, C, lab[1], n, d, k)
+    np.testing.assert_array_equal(lab[0], lab[1])
+    assert len(np.unique(lab[0])) == k
