@@ -108,7 +108,6 @@ __global__ __launch_bounds__(64 * screen_waves(NK), screen_waves(NK) / 4) void k
 {
     using G = ScreenGeom<NK>;
     constexpr int NW = screen_waves(NK);
-    constexpr bool PIPE = true;
     if (a.state != nullptr && a.state->done != 0) return;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     __shared__ int sChg;
@@ -207,10 +206,8 @@ __global__ __launch_bounds__(64 * screen_waves(NK), screen_waves(NK) / 4) void k
         unsigned cmax = 0u;
         auto take = [&](int g, const v16f& acc, int cb) { two_largest(m1[g], m2[g], acc, 16 * cb); };
         v16f late;  // group 1 of the block before
-        if constexpr (PIPE) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) late[i] = -3e38f;
-        }
+        for (int i = 0; i < 16; ++i) late[i] = -3e38f;
         float was[2] = {m1[0], m1[1]};
         for (int stg = 0; stg < nst; ++stg) {
             if (!resident) copy_stage(stg + 1 < nst ? stg + 1 : 0, cur ^ 1);
@@ -231,45 +228,26 @@ __global__ __launch_bounds__(64 * screen_waves(NK), screen_waves(NK) / 4) void k
                 auto centres = [&](int s) {
                     return *reinterpret_cast<const v8bf*>(cb0 + 32 * cb * G::CSTR + 32 * (s >> 1) + 8 * (s & 1));
                 };
-                if constexpr (PIPE) {
-                    v8bf ca[2 * NK];
+                v8bf ca[2 * NK];
 #pragma unroll
-                    for (int s = 0; s < 2 * NK; ++s) ca[s] = centres(s);
-                    v16f acc = init;
+                for (int s = 0; s < 2 * NK; ++s) ca[s] = centres(s);
+                v16f acc = init;
 #pragma unroll
-                    for (int s = 0; s < 2 * NK; ++s) acc = mfma32_bf16(ca[s], xh[0][s], acc);
-                    take(1, late, cb == 0 ? NB - 1 : cb - 1);
-                    if (cb == 0) {  // the stage before is through
+                for (int s = 0; s < 2 * NK; ++s) acc = mfma32_bf16(ca[s], xh[0][s], acc);
+                take(1, late, cb == 0 ? NB - 1 : cb - 1);
+                if (cb == 0) {  // the stage before is through
 #pragma unroll
-                        for (int g = 0; g < 2; ++g) {
-                            ms[g] = m1[g] != was[g] ? stg - 1 : ms[g];
-                            was[g] = m1[g];
-                        }
+                    for (int g = 0; g < 2; ++g) {
+                        ms[g] = m1[g] != was[g] ? stg - 1 : ms[g];
+                        was[g] = m1[g];
                     }
-                    __builtin_amdgcn_sched_barrier(0);
-                    late = init;
-#pragma unroll
-                    for (int s = 0; s < 2 * NK; ++s) late = mfma32_bf16(ca[s], xh[1][s], late);
-                    take(0, acc, cb);
-                    __builtin_amdgcn_sched_barrier(0);
-                } else {
-                    v16f acc[2] = {init, init};
-#pragma unroll
-                    for (int s = 0; s < 2 * NK; ++s) {
-                        const v8bf ca = centres(s);
-#pragma unroll
-                        for (int g = 0; g < 2; ++g) acc[g] = mfma32_bf16(ca, xh[g][s], acc[g]);
-                    }
-#pragma unroll
-                    for (int g = 0; g < 2; ++g) take(g, acc[g], cb);
                 }
-            }
-            if constexpr (!PIPE) {
+                __builtin_amdgcn_sched_barrier(0);
+                late = init;
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    ms[g] = m1[g] != was[g] ? stg : ms[g];
-                    was[g] = m1[g];
-                }
+                for (int s = 0; s < 2 * NK; ++s) late = mfma32_bf16(ca[s], xh[1][s], late);
+                take(0, acc, cb);
+                __builtin_amdgcn_sched_barrier(0);
             }
             if (!resident) {
                 // the next stage is in (every wave's copies) and this one is
@@ -279,11 +257,9 @@ __global__ __launch_bounds__(64 * screen_waves(NK), screen_waves(NK) / 4) void k
                 cur ^= 1;
             }
         }
-        if constexpr (PIPE) {
-            take(1, late, kScreenSC / 32 - 1);
+        take(1, late, kScreenSC / 32 - 1);
 #pragma unroll
-            for (int g = 0; g < 2; ++g) ms[g] = m1[g] != was[g] ? nst - 1 : ms[g];
-        }
+        for (int g = 0; g < 2; ++g) ms[g] = m1[g] != was[g] ? nst - 1 : ms[g];
         // the two lanes of a row; lane l keeps row l of the wave's 64
         float b1 = 0.f, b2 = 0.f, bx = 0.f;
         int bi = 0;

@@ -730,7 +730,7 @@ struct Lloyd {
     }
     bool screened() const
     {
-        if (!split_on || !a3cap || screen_nomem || run_off || n >= (1L << 31) || (ld > 128 && k <= 128)) return false;
+        if (!split_on || !a3cap || screen_nomem || run_off || n >= (1L << 31) || k <= 128) return false;
         const int sw = screen_switch();
         return sw >= 0 ? sw > 0 : screen_pays(n, ld, k);
     }

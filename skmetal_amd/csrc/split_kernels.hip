@@ -14,6 +14,7 @@
 #include <stdlib.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "split_common.h"
 
@@ -800,14 +801,14 @@ __global__ __launch_bounds__(256) void k_centre_image(const float* __restrict__ 
 
 // The images of k_assign3_list (its nst stages) and of k_screen (the blocks
 // past them) in one launch.
-template <int CB, int NK>
+template <int NK>
 __global__ __launch_bounds__(256) void k_centre_images(const float* __restrict__ C, const float* __restrict__ cnorm,
                                                        int k, int ld, int nseg, int nst, char* __restrict__ img,
                                                        char* __restrict__ simg, const LoopState* st)
 {
     if (st != nullptr && st->done != 0) return;
     if ((int)blockIdx.x < nst)
-        centre_image<CB>(C, cnorm, k, ld, nseg, img);
+        centre_image<16>(C, cnorm, k, ld, nseg, img);
     else
         screen_image<NK>(C, cnorm, k, ld, simg, (int)blockIdx.x - nst);
 }
@@ -863,7 +864,7 @@ __device__ __forceinline__ void assign3_rows(char* smem, int ld, int npass, int 
                                              int& mylab, float& mymin)
 {
     using G = Assign3Geom<CB>;
-    constexpr int CPC = G::CPC, SEG = G::SEG, NKS = G::NKS, CSTR = G::CSTR, CPART = G::CPART;
+    constexpr int CPC = G::CPC, SEG = G::SEG, NKS = G::NKS, CSTR = G::CSTR;
     const int nst = npass * nseg;
     float bd[2] = {INFINITY, INFINITY};
     int bi[2] = {0, 0};
@@ -1103,7 +1104,6 @@ __global__ __launch_bounds__(512, 1) void k_assign3(const float* __restrict__ X,
 // pass over the centres.  Rows left all in one stretch of X are a few blocks'
 // work and take as long as k_assign3 does for all rows, so the busiest block's
 // passes go to the state beside the count.
-template <int CB>
 __global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict__ X, long n, int ld,
                                                          const char* __restrict__ img, int k,
                                                          int* __restrict__ labels, LoopState* st, int* changed,
@@ -1111,6 +1111,7 @@ __global__ __launch_bounds__(512, 1) void k_assign3_list(const float* __restrict
                                                          const unsigned long long* __restrict__ masks)
 {
     if (st != nullptr && st->done != 0) return;
+    constexpr int CB = 16;  // (more than 128 centres)
     using G = Assign3Geom<CB>;
     constexpr int CPC = G::CPC, SEG = G::SEG;
     constexpr int CH = 2048;  // rows whose bits are listed at a time, 256 per wave
@@ -1495,25 +1496,19 @@ static bool split_disabled()
     return env != nullptr && env[0] == '0';
 }
 
-typedef void (*assign3_list_fn)(const float*, long, int, const char*, int, int*, LoopState*, int*, float*,
-                                const unsigned long long*);
-static assign3_list_fn assign3_list_kernel(int k)
-{
-    const int cb = assign3_cb(k);
-    return cb == 4 ? &k_assign3_list<4> : cb == 8 ? &k_assign3_list<8> : &k_assign3_list<16>;
-}
-
 int assign3_ready(int d, int k)
 {
     if (split_disabled() || d < 17 || k < 1) return 0;
-    for (const int kk : {64, 128, 129}) {
-        for (const void* f : {reinterpret_cast<const void*>(assign3_kernel(kk)),
-                              reinterpret_cast<const void*>(assign3_list_kernel(kk))}) {
-            if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)assign3_lds(kk)) !=
-                hipSuccess) {
-                (void)hipGetLastError();
-                return 0;
-            }
+    const std::pair<const void*, int> kernels[] = {
+        {reinterpret_cast<const void*>(assign3_kernel(64)), 64},
+        {reinterpret_cast<const void*>(assign3_kernel(128)), 128},
+        {reinterpret_cast<const void*>(assign3_kernel(129)), 129},
+        {reinterpret_cast<const void*>(&k_assign3_list), 129},
+    };
+    for (const auto& [f, kk] : kernels) {
+        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)assign3_lds(kk)) != hipSuccess) {
+            (void)hipGetLastError();
+            return 0;
         }
     }
     return 1;
@@ -1537,25 +1532,23 @@ hipError_t launch_assign3(const AssignArgs& a, int num_cu, hipStream_t s)
     return hipGetLastError();
 }
 typedef void (*images_fn)(const float*, const float*, int, int, int, int, char*, char*, const LoopState*);
-template <int CB>
 static images_fn images_kernel(int ld)
 {
     switch ((ld + 31) / 32) {
-    case 1: return &k_centre_images<CB, 1>;
-    case 2: return &k_centre_images<CB, 2>;
-    case 3: return &k_centre_images<CB, 3>;
-    default: return &k_centre_images<CB, 4>;
+    case 1: return &k_centre_images<1>;
+    case 2: return &k_centre_images<2>;
+    case 3: return &k_centre_images<3>;
+    default: return &k_centre_images<4>;
     }
 }
 
 hipError_t launch_centre_images(const AssignArgs& a, char* simg, hipStream_t s)
 {
-    if (a.img == nullptr || simg == nullptr) return hipErrorInvalidValue;
+    if (a.img == nullptr || simg == nullptr || a.k <= 128 || a.ld > 128) return hipErrorInvalidValue;
     int nst = 0, nseg = 0;
     size_t stage = 0;
     assign3_stages(a.k, a.ld, &nst, &nseg, &stage);
-    const int cb = assign3_cb(a.k);
-    const images_fn f = cb == 4 ? images_kernel<4>(a.ld) : cb == 8 ? images_kernel<8>(a.ld) : images_kernel<16>(a.ld);
+    const images_fn f = images_kernel(a.ld);
     const int snst = (a.k + kScreenSC - 1) / kScreenSC;
     hipLaunchKernelGGL(f, dim3((unsigned)(nst + snst)), dim3(256), 0, s, a.C, a.cnorm, a.k, a.ld, nseg, nst, a.img, simg,
                        a.state);
@@ -1565,10 +1558,10 @@ hipError_t launch_centre_images(const AssignArgs& a, char* simg, hipStream_t s)
 hipError_t launch_assign3_list(const AssignArgs& a, const unsigned long long* masks, int num_cu, hipStream_t s)
 {
     if (a.n <= 0) return hipSuccess;
-    if (a.img == nullptr || masks == nullptr) return hipErrorInvalidValue;
+    if (a.img == nullptr || masks == nullptr || a.k <= 128 || a.ld > 128) return hipErrorInvalidValue;
     long blocks = (a.n + 255) / 256;
     if (blocks > num_cu) blocks = num_cu;
-    hipLaunchKernelGGL(assign3_list_kernel(a.k), dim3((unsigned)blocks), dim3(512), assign3_lds(a.k), s, a.X, a.n,
+    hipLaunchKernelGGL(k_assign3_list, dim3((unsigned)blocks), dim3(512), assign3_lds(a.k), s, a.X, a.n,
                        a.ld, a.img, a.k, a.labels, a.state, a.changed, a.emin, masks);
     return hipGetLastError();
 }

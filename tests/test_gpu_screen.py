@@ -47,8 +47,8 @@ def _both(monkeypatch, X, C, steps=5, center=True):
 # every K-step count, row ends off the 32-feature and 64-row grid, one stage
 # of centres, several, and more than LDS keeps (k = 2000 at 4 K steps)
 @pytest.mark.parametrize("n,d,k,spread", [
-    (300, 17, 300, 1.0), (777, 37, 101, 0.6), (4099, 66, 129, 0.5), (513, 128, 200, 0.2), (20011, 96, 128, 0.4),
-    (33333, 125, 257, 0.1), (70001, 64, 300, 0.9), (5000, 104, 2000, 0.5), (66, 32, 65, 1.0),
+    (300, 17, 300, 1.0), (777, 37, 201, 0.6), (4099, 66, 129, 0.5), (513, 128, 200, 0.2), (20011, 96, 256, 0.4),
+    (33333, 125, 257, 0.1), (70001, 64, 300, 0.9), (5000, 104, 2000, 0.5), (130, 32, 130, 1.0),
     # rows of more than 128 floats: 256 x 256 units, ends off both, one
     # 64-feature stage more than whole ones
     (3000, 129, 200, 0.5), (777, 300, 257, 0.4), (20011, 768, 700, 0.3), (300, 1000, 300, 0.2), (256, 192, 256, 0.3),
@@ -113,7 +113,7 @@ def test_screen_non_finite_centres(monkeypatch, d):
     np.testing.assert_array_equal(lab[0], lab[1])
 
 
-@pytest.mark.parametrize("n,d,k", [(9000, 50, 80), (30000, 128, 140), (5000, 200, 150)])
+@pytest.mark.parametrize("n,d,k", [(9000, 50, 180), (30000, 128, 140), (5000, 200, 150)])
 def test_screen_relocation(monkeypatch, n, d, k):
     """Empty clusters: the farthest rows come from the screen's row minima and
     are those of the six products' minima."""
