@@ -567,9 +567,13 @@ __global__ __launch_bounds__(256) void k_label_offs(SortArgs a, int nw)
 // k_label_segs, k_label_scan and k_label_offs in one block, for histograms that
 // fit in LDS (nw k <= kScanLds): the histogram in, thread (j, part) of 1,024
 // runs down its share of cluster j's ranges, the clusters' exclusive scan, and
-// the range offsets out.  Two launches fewer: 12 -> 9.4 us a step at 101
-// clusters and 256 ranges.
-constexpr int kScanLds = 32768;
+// the range offsets out.  Two launches fewer, for one block's pass over the
+// histogram.  The update with three launches / with this, us: 20,000 x 64, k =
+// 100 28.5 / 24.8; 100,000 x 64, k = 80 29.6 / 28.0, k = 128 29.5 / 28.1; 300,000
+// x 64, k = 128 38.7 / 37.2; 500,000 x 64, k = 66 47.8 / 46.6; 200,000 x 64, k =
+// 160 35.4 / 36.0.  Histograms of up to 32,768 counts here took 31.0, 30.0, 39.4
+// and 38.0 at k = 80 and 128 (twice) and 160: more than the three launches.
+constexpr int kScanLds = 20480;
 __global__ __launch_bounds__(1024) void k_label_scan1(SortArgs a, int nw, int B)
 {
     const int done = a.state->done;
@@ -876,7 +880,7 @@ SortGeom sort_geometry(long n, int d, int ld, int k)
     long wr = (n + 1023) / 1024;
     wr = ((wr + 63) / 64) * 64;
     if (wr < 256) wr = 256;
-    // up to 512K rows and 340 clusters: fewer ranges (at least 96), whose
+    // up to 512K rows and 213 clusters: fewer ranges (at least 96), whose
     // histogram one block scans (k_label_scan1)
     if (n <= (512L << 10) && (long)((n + wr - 1) / wr) * k > kScanLds) {
         const long nw = min(256L, (long)kScanLds / k);
