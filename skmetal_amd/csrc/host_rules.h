@@ -74,18 +74,21 @@ inline bool screen_pays(long n, int ld, int k)
     return ld <= 128 ? (rounds - 1) * round >= 60e3 : rounds * round >= 230e3;
 }
 
-// The E-step's time in us on 256 CUs, fitted to timings of 27 shapes (60,000 to
-// 1M rows of 32 to 128 floats, 4,000 to 400,000 of 200 to 1,000, 200 to 2,048
-// centres; within 15% but for rows of 32 floats).  plain: k_assign3, 14 us and
-// 4.3 to 4.7 for 32 features of 256 centres of a round of 256-row blocks.
-// screen: k_screen or k_screen_wide with the centres' images and the empty
+// The E-step's time in us on 256 CUs, fitted to timings of 35 shapes (60,000 to
+// 4M rows of 32 to 128 floats, 4,000 to 1M of 200 to 1,000, 200 to 4,096
+// centres; within 15%, but for rows of 32 floats, and for fewer row blocks than
+// CUs, where plain is up to 20% less).  plain: k_assign3, 14 us and 4.45 to 4.7
+// for 32 features of 256 centres of a round of 256-row blocks.  screen: k_screen
+// or k_screen_wide (4 us a block and 2.25 for 64 features, or X's bytes, of which
+// rows off the cache lines cost more) with the centres' images and the empty
 // launches behind it.  rest: the six products of the rows left; `passes` is
 // k_assign3_list's busiest block's, which k_assign3_units (long rows) has not:
-// its units of 64 centres (few rows) or 256 go round the CUs.
+// its units of 256 centres, or of 64 where those would leave half the CUs idle,
+// go round the CUs.
 inline double plain_us(long n, int ld, int k)
 {
     const long rounds = (n + 65535) / 65536, steps = (long)((k + 255) / 256) * ((ld + 31) / 32);
-    return 14.0 + (ld <= 128 ? 4.7 : 4.3) * (double)(rounds * steps);
+    return 14.0 + (ld <= 128 ? 4.7 : 4.45) * (double)(rounds * steps);
 }
 inline double screen_us(long n, int ld, int k)
 {
@@ -95,24 +98,26 @@ inline double screen_us(long n, int ld, int k)
         const double t = mac * 1.95e-9 > values * 8.8e-8 ? mac * 1.95e-9 : values * 8.8e-8;
         return 26.0 + (t > bytes / 5.3e6 ? t : bytes / 5.3e6);
     }
-    const double t = 2.4 * (double)((wide_blocks(n, k) + 255) / 256 * ((ld + 63) / 64));
-    return 35.0 + (t > bytes / 3.5e6 ? t : bytes / 3.5e6);
+    const double t = (4.0 + 2.25 * ((ld + 63) / 64)) * (double)((wide_blocks(n, k) + 255) / 256);
+    const double m = bytes * (ld % 32 != 0 ? 1.4 : 1.0) / 5e6;
+    return 35.0 + (t > m ? t : m);
 }
 inline double rest_us(long n, int ld, int k, long left, long passes)
 {
-    const double step = 4.3 * 1.15 * ((ld + 31) / 32);
     if (ld <= 128) return (double)passes * (plain_us(n, ld, k) - 14.0) / (double)((n + 65535) / 65536);
     const long units = (left + 255) / 256 * ((k + 255) / 256);
-    return units * 2 <= 256 ? (units > 0 ? 0.35 * step : 0.0) : step * (double)((units + 255) / 256);
+    const double unit = 4.95 * ((ld + 31) / 32);
+    return units * 2 <= 256 ? 0.33 * unit * (double)((units * 4 + 255) / 256) : unit * (double)((units + 255) / 256);
 }
 // Whether a step that left these rows took longer than without the screen.
-// Timed with the rows left spread evenly, without / with the screen, at the last
-// share before the line and the first past it: 1M x 128, k = 256 (9 passes of
-// 16) 338 / 285 and 336 / 319; 250,000 x 128, k = 256 (1 of 4) 96 / 65 and 95 /
-// 70; 1M x 64, k = 1,024 (11 of 16) 650 / 543 and 640 / 601; 400,000 x 300, k =
-// 200 (a third) 327 / 296 and 338 / 348; 64,000 x 768, k = 400 (half) 218 / 205
-// and 216 / 302; 100,000 x 768, k = 2,048 (nine tenths) 1,544 / 1,396 and 1,545
-// / 1,647.  Rows left in one stretch, a tenth of 1M x 128: 338 / 404.
+// Timed with the rows left spread evenly, without / with the screen, at shares
+// before the line and past it: 1M x 128, k = 256 (9 passes of 16) 338 / 285 and
+// 336 / 319; 250,000 x 128, k = 256 (1 of 4) 96 / 65 and 95 / 70; 1M x 64, k =
+// 1,024 (11 of 16) 650 / 543 and 640 / 601; 400,000 x 300, k = 200 (a half) 327 /
+// 296 and 330 / 399; 64,000 x 768, k = 400 (a half) 218 / 205 and 216 / 302;
+// 100,000 x 768, k = 2,048 (four fifths) 1,544 / 1,396 and 1,545 / 1,647; 500,000
+// x 768, k = 4,096 (two thirds) 13,760 / 12,227 and 13,773 / 15,280.  Rows left
+// in one stretch, a tenth of 1M x 128: 338 / 404.
 inline bool screen_lost(long n, int ld, int k, long left, long passes)
 {
     return screen_us(n, ld, k) + rest_us(n, ld, k, left, passes) > 0.98 * plain_us(n, ld, k);
