@@ -227,6 +227,7 @@ def main():
         h.set_centers(C0)
         _, (ms_assign, ms_update, ms_final) = h.iterate(args.steps, kernel_times=True)
         mode = h.info()
+        screen = h.screen_info()
     finally:
         h.close()
     if args.calib_copy:
@@ -280,14 +281,17 @@ def main():
         }
     elif asplit:
         # MFMA roofline of the split E-step over the padded centres (multiples
-        # of 16 per pass) and features (32): one bf16 product per x.c term, which
-        # every row takes (the certified screen; the rows it leaves, and shapes
-        # without it, take six)
+        # of 16 per pass) and features (32): six bf16 products per x.c term; behind
+        # the certified screen one for every row, and six for the rows it left
+        # (the last step's count)
+        screened = screen["screened"] and not screen["off"]
+        products = 1.0 + 6.0 * screen["left"] / n if screened else 6.0
         kp = -(-k // (16 * (4 if k <= 64 else 8 if k <= 128 else 16))) * (16 * (4 if k <= 64 else 8 if k <= 128 else 16))
         dp = -(-d // 32) * 32
-        mflops = 2.0 * n * kp * dp
+        mflops = products * 2.0 * n * kp * dp
         roofline = {
-            "kernel": "k_screen / k_assign3: ||c||^2 - 2 x.c on bf16 MFMAs over the exact three-part split + argmin",
+            "kernel": (("k_screen and the six products of the rows it left" if screened else "k_assign3")
+                       + ": ||c||^2 - 2 x.c on bf16 MFMAs over the exact three-part split + argmin"),
             "bound": "mfma",
             "achieved": round(mflops / assign_s / 1e12, 1),
             "peak": PEAK_BF16_MFMA_TFLOPS,
@@ -295,6 +299,7 @@ def main():
             "frac": round(mflops / assign_s / 1e12 / PEAK_BF16_MFMA_TFLOPS, 4),
             "traffic": traffic,
             "fp32_equiv_tflops": round(flops / assign_s / 1e12, 2),
+            "products_per_term": round(products, 3),
         }
     else:
         achieved = flops / assign_s / 1e12

@@ -48,7 +48,8 @@ inline size_t wide_part_floats(long rows, int k) { return size_t(rows) * ((size_
 // k_screen_wide's blocks for `rows` rows: whole turns of the XCDs.
 inline long wide_blocks(long rows, int k) { return ((rows + 255) / 256 + 7) / 8 * 8 * ((k + 255) / 256); }
 
-// Where the screen pays.  k_assign3 alone takes its 256-row blocks in rounds
+// Where a run's steps begin behind the screen (screen_lost then tells whether
+// they stay there).  k_assign3 alone takes its 256-row blocks in rounds
 // of 256 (one a CU), each round proportional to the padded centres times
 // features (0.64 us per 1,000).  Rows of at most 128 floats: what is left
 // costs about one round again (nearly every block has a row) and the second
@@ -60,11 +61,17 @@ inline long wide_blocks(long rows, int k) { return ((rows + 255) / 256 + 7) / 8 
 // little, but there are two more launches.  768 floats, k = 1,500: 8,000 rows
 // 610 / 126; 300 floats: k = 600, 8,000 rows 161 / 87; k = 200, 130,000 rows
 // 158 / 142, 400,000 444 / 337; k = 512, 64,000 rows 150 / 124, 130,000 251 /
-// 175.  The slack grows with the norms: of blobs of 768 floats most rows are
-// left, and with at most two units of centres nothing is saved once
-// k_assign3's blocks fill half the CUs: k = 200, 130,000 rows 326 / 363,
-// 390,000 890 / 958; k = 400, 30,000 rows 242 / 183, 64,000 271 / 302,
-// 130,000 521 / 588.
+// 175.  What is left depends on the data, not on the shape.  64,000 rows of 400 to
+// 768 floats, k = 400, at the second step: 2 to 3% of overlapping blobs from
+// their means as centres, 95% of the same from rows of X, half of blobs a
+// little further apart, from rows too.  With at most two groups of 256 centres
+// and more row blocks than one round of their units (32,768 rows) the two steps
+// looked at cost most: 64,000 x 768, k = 400, three steps of the 95% kind 1,165 us
+// without the screen and 1,527 with, ten steps from the means 1,435 and 1,003;
+// 130,000 x 640 1,934 and 2,586, 2,926 and 1,709; 33,000 x 640, k = 300 (one
+// round) 926 and 908, 1,628 and 1,103.  Rows of more than 512 floats, where those
+// two steps are longest, begin without the screen there; of 64,000 x 512 the same
+// runs take 861 and 1,133, 1,545 and 1,055, and begin with it.
 inline bool screen_pays(long n, int ld, int k)
 {
     if (n >= (1L << 31) || k <= 128) return false;

@@ -296,10 +296,11 @@ struct RelocArgs {
 hipError_t launch_relocate(const RelocArgs& a, int E, hipStream_t s);
 
 // In-stream relocation (k_reloc, launched after every step's
-// k_finalize_cols): when step `iter` left 1..kMaxReloc clusters empty, the
+// k_finalize_recs or k_finalize_cols): when step `iter` left 1..kMaxReloc clusters empty, the
 // rows farthest from their centres move to them and the centres and chunk
 // partials of the clusters involved are redone, before the step's loop
-// decision; with no empty cluster the kernel returns at once.
+// decision (on the generic path made by the same launch); with no empty
+// cluster there is nothing but that decision.
 struct InRelocArgs {
     const float* X; long n; int ld; int d; int k;
     const int* labels;     // step iter's labels

@@ -1936,9 +1936,10 @@ hipError_t launch_relocate(const RelocArgs& a, int E, hipStream_t s)
 // in-stream relocation: k_reloc
 // ---------------------------------------------------------------------------
 //
-// Launched after every step's k_finalize_cols, which counts the clusters it
-// finds empty in state->empty_cnt[iter & 1]; with none the kernel returns at
-// its first load.  Otherwise, as the device path above but in one kernel:
+// Launched after every step's k_finalize_recs or k_finalize_cols, which counts
+// the clusters it finds empty in state->empty_cnt[iter & 1]; with none, block 0
+// makes the step's loop decision on the generic path and the others return at
+// their first load.  Otherwise, as the device path above but in one kernel:
 // (A) each block takes the distances of its contiguous share of the rows and
 // its E farthest, in order, and counts itself done; (B) the last block to
 // finish merges the blocks' lists, moves the rows in the fp64 sums and

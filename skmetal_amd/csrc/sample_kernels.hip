@@ -444,7 +444,7 @@ __device__ __forceinline__ bool grid_q(double v, int e, long long& q)
 // a value ends in .5 of the grid (or the sum is 0).  k_ws_chain uses them
 // where that binade is the running sum's: the chunks then cost it a few
 // cycles, and only those that cross a binade or hold a tie are walked (807 ->
-// 144 us at 500,000 rows, against every chunk's values loaded by the one block).
+// 149 us at 500,000 rows, against every chunk's values loaded by the one block).
 __global__ __launch_bounds__(kWSThreads) void k_ws_grid(WSArgs a)
 {
     constexpr int PT = kWSChunk / kWSThreads;

@@ -876,7 +876,8 @@ struct Lloyd {
     // One Lloyd step, old centres cen[cur] -> new centres cen[cur ^ 1].  On
     // the fused path the stopping rules of a step are evaluated by the next
     // step's kernel (decide) or, for the last step of a batch (last), by
-    // k_finalize_loop; on the generic path by k_finalize_loop every step.
+    // k_finalize_loop; on the generic path every step, by k_reloc or, without the
+    // in-stream relocation, by k_finalize_loop.
     int enqueue_step(int iter, double tol, int flags, bool decide, bool last)
     {
         hipEvent_t* ev = nullptr;
