@@ -123,7 +123,8 @@ __device__ __forceinline__ void step_norms_apply(const FusedArgs& a, int lane, c
             LoopState* st = a.state;
             if (j < k) {
                 a.shift_sq[j] = (float)tsq;
-                if (count > 0) a.cnorm_out[j] = (float)tnr;
+                // (a cluster still empty after its relocation has a new centre too)
+                if (count > 0 || in.reloc_iter == a.iter - 1) a.cnorm_out[j] = (float)tnr;
             }
             if (lane == 0) {
                 st->n_empty = n_empty;

@@ -1256,6 +1256,8 @@ __device__ __forceinline__ void loop_decision(const FinalizeArgs& a, int nch)
 {
     LoopState* st = a.state;
     const int tid = threadIdx.x;
+    // every empty cluster's centre and partials are the relocation's
+    const bool relocated = a.after_reloc || st->reloc_iter == a.iter;
     __shared__ double shd[4];
     __shared__ int shi[4];
     __shared__ float shm[4];
@@ -1273,7 +1275,7 @@ __device__ __forceinline__ void loop_decision(const FinalizeArgs& a, int nch)
             }
             shift = (float)tsq;
             a.shift_sq[j] = shift;
-            if (count > 0 || a.after_reloc) a.cnorm[j] = (float)tnr;
+            if (count > 0 || relocated) a.cnorm[j] = (float)tnr;
         } else {
             shift = a.shift_sq[j];
         }
@@ -2376,7 +2378,7 @@ __device__ __forceinline__ bool reloc_body(const InRelocArgs& a, int E)
                 tnr += a.part[((long)j * a.nch + c) * 2 + 1];
             }
             a.fold_shift[j] = (float)tsq;
-            if (a.counts[j] > 0) a.fold_cnorm[j] = (float)tnr;
+            a.fold_cnorm[j] = (float)tnr;  // (a cluster still empty has the heaviest one's centre now)
         }
     }
     if (tid == 0) st->reloc_iter = a.iter;
