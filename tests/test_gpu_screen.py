@@ -61,7 +61,9 @@ def test_screen_labels_match_six_products(monkeypatch, n, d, k, spread):
     assert left > 0 or n < 512  # (a few hundred rows around as many centres: all settled)
 
 
-# rows on centres far apart are settled, rows half way between two are not
+# Rows on centres far apart are settled, rows half way between two are not.  (Of
+# 20,000 x 160 with 300 centres, units of 64 centres take the third that is left,
+# up to 128 units of 256, and units of 256 centres all of them.)
 @pytest.mark.parametrize("n,d,k", [(20000, 48, 300), (5000, 128, 700), (20000, 160, 300), (3000, 600, 260)])
 @pytest.mark.parametrize("share", [0.0, 0.3, 1.0])
 def test_screen_settles_what_it_can(monkeypatch, n, d, k, share):
